@@ -365,13 +365,15 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     }
     RPFastConst fk{0, 0, 0, 0, 0, 0, 0, 0};
     // The E longest bubbles (the queue's first entries) run one per workgroup
-    // in lane 0 of its first wavefront, alone: a wavefront issues the same
-    // instructions whether one lane or 64 are active, so a lone lane skips
-    // the paths the other lanes would need (the thermal impedance is a
-    // closed form instead of a table lookup for s > 20), and it never waits
-    // for the other lanes' refills.  The wavefront runs at raised issue priority
-    // until that bubble is done, then joins the shared queue, which starts
-    // after the E dedicated entries.
+    // in its first wavefront, alone: a wavefront issues the same instructions
+    // whether one lane or 64 are active, so a lone bubble never pays for the
+    // paths the other lanes would need, nor waits for their refills, and a
+    // pair of lanes evaluates two sub-steps' Omega and Lp in one pass
+    // (rp_integrate_pair; the launch is bound by this chain: RP launch 2.69 ->
+    // 2.23 ms at 2048^2 with 2^20 bubbles, 2.48 -> 1.79 ms with 30 011, 2.85 ->
+    // 2.65 ms at 4096^2 with 2^22, against one lane).  Lane 0 writes back.
+    // The wavefront runs at raised issue priority until that bubble is done,
+    // then joins the shared queue, which starts after the E dedicated entries.
     int E, nb;
     {
         const BubbleArrays &b = rpl(kp)->b;
@@ -381,7 +383,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     int idx = -1;                  // bubble of this lane, -1 when idle
     bool reuse = false;            // idx keeps its previous iteration's results
     bool pre = false;
-    if (threadIdx.x == 0 && (int)blockIdx.x < E) {
+    if (threadIdx.x < (FAST ? 2 : 1) && (int)blockIdx.x < E) {
         idx = rpl(kp)->b.order[blockIdx.x];
         pre = true;
     }
@@ -477,15 +479,14 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         bool fin, capped;
         double remain;
         if (FAST && solo) {
-            // a dedicated wavefront: lane 0 runs its bubble to the sync time
-            // without the batch bookkeeping of the shared loop below
-            // (lane 0 alone: its conditions are wave-uniform)
-            if (active)
-                while (cond<true>(LF.remain > 0.0 && LF.counter < max_substeps))
-                    rp_substep_g<double, false, true, true>(LF, fk, fsh);
+            // a dedicated wavefront: lanes 0 and 1 run its bubble to the sync
+            // time without the batch bookkeeping of the shared loop below
+            // (both hold one bubble: its conditions are wave-uniform)
+            if (active) rp_integrate_pair(LF, fk, fsh, lane & 1, max_substeps);
+            if (lane == 1) idx = -1;  // lane 0 writes back
             capped = active && LF.counter >= max_substeps;
             remain = active ? LF.remain : 0.0;
-            fin = active;
+            fin = idx >= 0;
         } else
         while (true) {
             capped = false;
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
                 break;
         }
         // ---- write back the bubbles that reached the sync time
-        if (active) {
+        if (idx >= 0) {
             crpl *P = rpl(kp);
             const GridParams &g = P->g;
             const BubbleParams &bp = P->bp;

@@ -361,15 +361,17 @@ __device__ inline void omega_lp_g(T Rn, T iRn, const RPFastConst &k, const RPFas
     *iom_out = iom;
 }
 
-// One pass of the sub-step loop body (bubble_CUDA_kernel.cuh:508-538).
-// FORCED: the step size is forced_dtp instead of the step-size control's
-// (the replay of a recorded schedule; the rest of the sub-step is unchanged).
-// HEAT: accumulate the heat and viscous dissipation of Q_B (T = double).
-// UNI: one lane runs the sub-step alone (branches on the scalar unit, cond).
-template <typename T, bool FORCED = false, bool HEAT = true, bool UNI = false>
-__device__ inline void rp_substep_g(RPLaneF<T> &L, const RPFastConst &k, const RPFastShared &s,
-                                    double forced_dtp = 0.0) {
-    // solveRayleighPlesset (bubble_CUDA_kernel.cuh:227-260)
+// solveRayleighPlesset (bubble_CUDA_kernel.cuh:227-260) and the clock of the
+// sub-step loop: the lane advances one sub-step in R and dR/dt.  Returns what
+// the gas pressure needs: the radius the sub-step starts from, its reciprocal
+// and the pressure before it.
+template <typename T>
+struct RPMove {
+    T Rn, iRn, PGn;
+};
+template <typename T, bool FORCED = false, bool UNI = false>
+__device__ inline RPMove<T> rp_advance_g(RPLaneF<T> &L, const RPFastShared &s,
+                                         double forced_dtp = 0.0) {
     const T PGn = L.PG;
     const double t = L.time;
     const T PL = fma_(L.PC2, T(t * t), fma_(L.PC1, T(t), L.PC0));
@@ -404,10 +406,17 @@ __device__ inline void rp_substep_g(RPLaneF<T> &L, const RPFastConst &k, const R
     L.Rp = Rp;
     L.Rn = Rn;
     L.d1R = d1R;
-    cx<T> Ln;  // Lp / |Lp|^2
-    T iom;
-    omega_lp_g<T, UNI>(Rn, iRn, k, s, &Ln, &iom);
-    // solvePG (bubble_CUDA_kernel.cuh:322-340)
+    return RPMove<T>{Rn, iRn, PGn};
+}
+
+// solvePG (bubble_CUDA_kernel.cuh:322-340) after rp_advance_g, with Ln =
+// Lp / |Lp|^2 and iom = 1 / omega_N at the radius the sub-step started from,
+// and the sub-step's share of Q_B.
+template <typename T, bool HEAT = true>
+__device__ inline void rp_gas_g(RPLaneF<T> &L, const RPMove<T> &mv, cx<T> Ln, T iom,
+                                const RPFastConst &k, const RPFastShared &s) {
+    const T Rn = mv.Rn, PGn = mv.PGn, Rp = L.Rp, d1R = L.d1R;
+    const double dtL = L.dtL;
     const T Rbar = 0.5 * (Rp + Rn);
     const T iRbar = rcp_(Rbar);
     const T Rx_ = Rbar * k.iR0, Rpx = Rp * k.iR0, Rnx = Rn * k.iR0;
@@ -431,6 +440,58 @@ __device__ inline void rp_substep_g(RPLaneF<T> &L, const RPFastConst &k, const R
         L.SumVis = fma(s.sixteen_pi_mu * Rp * dtL, d1R * d1R, L.SumVis);
     }
     L.counter++;
+}
+
+// One pass of the sub-step loop body (bubble_CUDA_kernel.cuh:508-538).
+// FORCED: the step size is forced_dtp instead of the step-size control's
+// (the replay of a recorded schedule; the rest of the sub-step is unchanged).
+// HEAT: accumulate the heat and viscous dissipation of Q_B (T = double).
+// UNI: one lane runs the sub-step alone (branches on the scalar unit, cond).
+template <typename T, bool FORCED = false, bool HEAT = true, bool UNI = false>
+__device__ inline void rp_substep_g(RPLaneF<T> &L, const RPFastConst &k, const RPFastShared &s,
+                                    double forced_dtp = 0.0) {
+    const RPMove<T> mv = rp_advance_g<T, FORCED, UNI>(L, s, forced_dtp);
+    cx<T> Ln;  // Lp / |Lp|^2
+    T iom;
+    omega_lp_g<T, UNI>(mv.Rn, mv.iRn, k, s, &Ln, &iom);
+    rp_gas_g<T, HEAT>(L, mv, Ln, iom, k, s);
+}
+
+// A value of the even (or odd) lane of each lane pair, in both lanes.
+template <int CTRL>
+__device__ inline double quad_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ inline double from_even(double v) { return quad_move<0xA0>(v); }  // quad_perm 0,0,2,2
+__device__ inline double from_odd(double v) { return quad_move<0xF5>(v); }   // quad_perm 1,1,3,3
+
+// A bubble's whole integration on a pair of lanes (both hold its state).
+// The Omega iteration and Lp, more than half of a sub-step's instructions,
+// depend on the radius a sub-step starts from alone; the next sub-step starts
+// from the radius this one reaches, which needs only the gas pressure of the
+// sub-step before.  So once a sub-step has moved, the radii that it and its
+// successor start from are both known, and the two lanes evaluate Omega and
+// Lp for both at once, in the one instruction stream that the wavefront
+// issues anyway.  The operations of each sub-step and their order are
+// rp_substep_g's, so the results are its results bit for bit.  All lanes of
+// the wavefront that run this hold one bubble (UNI conditions).
+__device__ inline void rp_integrate_pair(RPLaneF<double> &L, const RPFastConst &k,
+                                         const RPFastShared &s, bool odd, int max_substeps) {
+    while (cond<true>(L.remain > 0.0 && L.counter < max_substeps)) {
+        const RPMove<double> m0 = rp_advance_g<double, false, true>(L, s);
+        const double R = odd ? L.Rp : m0.Rn;
+        cx<double> Ln;
+        double iom;
+        omega_lp_g<double>(R, drcp(R), k, s, &Ln, &iom);
+        rp_gas_g<double>(L, m0, cx<double>{from_even(Ln.re), from_even(Ln.im)}, from_even(iom), k,
+                         s);
+        if (!cond<true>(L.remain > 0.0 && L.counter < max_substeps)) break;
+        const RPMove<double> m1 = rp_advance_g<double, false, true>(L, s);
+        rp_gas_g<double>(L, m1, cx<double>{from_odd(Ln.re), from_odd(Ln.im)}, from_odd(iom), k, s);
+    }
 }
 
 // ---- reverse mode: adjoints of the RP map of one Picard iteration ----------
