@@ -440,6 +440,8 @@ int alloc_bubbles(brp_handle *h, int n) {
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.part, sizeof(int) * 2 * (size_t)((n + 255) / 256 + 1))))
         return rc;
+    if ((rc = dalloc(h, (void **)&h->b.totals, sizeof(RPTotals) * 4 * (size_t)(h->cus * h->per_cu))))
+        return rc;
     if ((rc = dalloc(h, (void **)&h->b.bbox_blk, sizeof(int) * 4 * (size_t)((n + 255) / 256 + 1))))
         return rc;
     return BRP_OK;
@@ -899,7 +901,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                  (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0, h->fgb[old_cur],
                                  h->fgb[old_n], h->fgb[old_m], h->W, ax, bx, ay, by, h->xu_d,
                                  h->rxp_d, h->sc_d);
-        launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t);
+        launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, nullptr, 0,
+                                  h->sc_d);
         HIPCHK(h, hipEventRecord(h->ev[3], s));
         HIPCHK(h, hipMemcpyAsync(h->sc_h, h->sc_d, hdr + sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         HIPCHK(h, hipStreamSynchronize(s));
@@ -938,7 +941,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 HIPCHK(h, hipEventRecord(h->ev[7], s));
                 const StepRecord *tin = ctl ? ctl->tape_in : nullptr;
                 const bool replay = h->sched_mode == 2;
-                if (!tin && !replay) {
+                if (!tin && !replay && !bubble_step_unordered(*h->rpl_h, h->cus)) {
                     // the pressure gather, then the queue: the first iteration's
                     // from the start state (the previous step's counts do not
                     // find this step's longest chains), the later ones from the
@@ -950,6 +953,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                            h->bp.extreme_threshold);
                 }
                 HIPCHK(h, hipEventRecord(h->ev[4], s));
+                int rp_waves = 0;  // wavefront records the launch leaves
                 if (tin) {  // replay: the void fraction from the taped radii, no RP
                     launch_scatter_radii(s, h->g, h->bp, h->b, tin->Rt_it[loop], h->fgb[target], h->sc_d);
                 } else if (replay) {  // the recorded step sizes of this RP call
@@ -963,8 +967,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     const bool lean = bubble_step_lean(h->last_sub_max, h->last_sub_per_launch,
                                                        h->bp.extreme_threshold, h->cus);
                     st.rp_lean_launches += lean ? 1 : 0;
-                    launch_bubble_step<F>(s, *h->rpl_h, h->rpl_d, h->rp_cur, h->pl_m, h->pl_n,
-                                          h->pl_p, h->fgb[target], h->sc_d, loop, lean, h->cus,
+                    rp_waves = launch_bubble_step<F>(s, *h->rpl_h, h->rpl_d, h->rp_cur, h->pl_m, h->pl_n,
+                                          h->pl_p, p0, h->fgb[target], h->sc_d, loop, lean, h->cus,
                                           h->per_cu);
                     if (h->sched_mode == 1) {
                         int rc = schedule_record_call(h);
@@ -986,7 +990,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                           (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0,
                                           h->fgb[target], h->fgb[old_cur], h->fgb[prev], h->W, ax,
                                           bx, ay, by, h->xu_d, h->rxp_d, h->sc_d, loop);
-                launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t);
+                launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, h->b.totals,
+                                          rp_waves, h->sc_d);
                 if (rec && rec->want_grid) {
                     int rc = copy_rect(h, rec->p0_it[loop], p0, sizeof(F), rec->rect);
                     if (rc) return rc;

@@ -64,6 +64,14 @@ struct Window {
     int i0, i1, j0, j1;  // inclusive, within [0, N+1]
 };
 
+// What one wavefront of an RP launch did; k_pressure_ghosts, the iteration's
+// last kernel, adds the wavefronts' records to the step's scalars.
+struct RPTotals {
+    unsigned long long sub_sum;  // sub-steps integrated
+    unsigned int done, kept;     // bubbles written back; of them, kept
+    int sub_max, flags;          // StepScalars::flags bits
+};
+
 // Device-side per-step scalars written by the kernels and read by the host.
 struct StepScalars {
     int bbox[4];                         // min i, max i, min j, max j of bubble stencils
@@ -96,6 +104,7 @@ struct BubbleArrays {
     int *sort_hist;       // partition scratch: 2048 bin counts / offsets of that sort
     int *part;            // partition scratch: per-block extreme and heavy offsets + totals
     int *bbox_blk;        // per-block stencil bounding boxes of k_motion (4 ints each)
+    RPTotals *totals;     // per wavefront of the RP launch
 };
 
 // Bubble physics constants shared by every bubble.
@@ -178,16 +187,22 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
                             const double *xu, const double *rxp, StepScalars *sc, int slot);
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
-                            const double *el_phase, double t);
+                            const double *el_phase, double t, const RPTotals *tot, int n_tot,
+                            StepScalars *sc);
 template <typename F>
 void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                    const BubbleArrays &b, const F *vx, const F *vy, StepScalars *sc);
 // The RP launch of Picard iteration `slot` over the queue order, with the
 // gathered pressures of launch_queue_keys in PL[plp].
+// Returns the number of wavefronts launched (their records in b.totals).
 template <typename F>
-void launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
-                        int plm, int pln, int plp, int64_t *fg_target, StepScalars *sc, int slot,
-                        bool lean, int cus, int per_cu);
+int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
+                        int plm, int pln, int plp, const F *p0, int64_t *fg_target, StepScalars *sc,
+                        int slot, bool lean, int cus, int per_cu);
+// Whether the launch runs every bubble on a lane pair, and whether it then
+// needs no queue (it gathers the pressures itself).
+bool bubble_step_pairs(const RPLaunch &host, int cus);
+bool bubble_step_unordered(const RPLaunch &host, int cus);
 // The device's compute units and the persistent RP kernel's workgroups per
 // compute unit (its occupancy limit), queried once per handle.
 void rp_grid_query(int device, int *cus, int *per_cu);

@@ -291,6 +291,22 @@ __device__ inline unsigned long long lanemask_lt(int lane) {
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
+// A wavefront's record of an RP launch (RPTotals), one plain store.
+__device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
+                                        unsigned long long sub_sum, unsigned int done,
+                                        unsigned int kept, bool bad, bool capped) {
+    for (int off = 32; off > 0; off >>= 1) {
+        sub_max = max(sub_max, __shfl_xor(sub_max, off, 64));
+        sub_sum += __shfl_xor(sub_sum, off, 64);
+        done += __shfl_xor(done, off, 64);
+        kept += __shfl_xor(kept, off, 64);
+    }
+    const int flags = (__ballot(bad) ? 2 : 0) | (__ballot(capped) ? 4 : 0);
+    if (lane == 0)
+        tot[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)] =
+            RPTotals{sub_sum, done, kept, sub_max, flags};
+}
+
 // One Picard iteration for every bubble, fused (after k_queue_keys gathered
 // PL_p, BubbleInterpolationScalarKernel, kernel.cuh:361-395):
 //   BubbleRadiusKernel              (RP from the step's start state, 471-554)
@@ -339,7 +355,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     const int lane = threadIdx.x & 63;
     const int nxt = cur ^ 1;
     __shared__ WaveAgg agg_all[4];  // 25 KB: one table per wavefront
-    __shared__ double vtab[FAST ? kRpVSize : 1];  // 50 KB: the V and Y tables
+    __shared__ __align__(16) double vtab[FAST ? kRpVSize : 1];  // 50 KB: the V and Y tables
     WaveAgg &agg = agg_all[threadIdx.x >> 6];
     agg_clear(agg, lane);
     // The shared RP constants go through LDS into vector registers, held for
@@ -550,21 +566,179 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         if (__builtin_amdgcn_readfirstlane(agg.count) > kAggSlots / 2) agg_flush(agg, lane, fg_target);
     }
     agg_flush(agg, lane, fg_target);
-    for (int off = 32; off > 0; off >>= 1) {
-        sub_max = max(sub_max, __shfl_xor(sub_max, off, 64));
-        sub_sum += __shfl_xor(sub_sum, off, 64);
-        done += __shfl_xor(done, off, 64);
-        kept += __shfl_xor(kept, off, 64);
+    rp_launch_totals(rpl(kp)->b.totals, lane, sub_max, sub_sum, done, kept, bad, capped_any);
+}
+
+// The same launch for a population that the chip can hold at once on lane
+// pairs (bubble_step_pairs): every bubble runs on a pair of lanes
+// (rp_pair_pass), at most `quota` to a wavefront, so that each sub-step takes
+// the pair's time, and the population spreads over all the wavefronts instead
+// of filling the lanes of a few.  ORDERED: the queue of launch_order_partition;
+// its first bubbles go to wavefronts of their own (at most solo_cap, one per
+// workgroup first), the others are taken in order as pairs come free.  Not
+// ORDERED: at most one bubble per wavefront, so no queue and no keys are
+// needed, and the pressure is gathered here.
+template <typename F, bool ORDERED>
+__global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int max_substeps,
+                                                      const double *rp_shared, int cur, int plm,
+                                                      int pln, int plp, const F *__restrict__ p0,
+                                                      int64_t *__restrict__ fg_target,
+                                                      StepScalars *sc, int slot, int quota,
+                                                      int solo_cap) {
+    const int lane = threadIdx.x & 63;
+    const bool odd = lane & 1;
+    const int nxt = cur ^ 1;
+    __shared__ WaveAgg agg_all[4];
+    __shared__ __align__(16) double vtab[kRpVSize];
+    __shared__ double shc[16];
+    WaveAgg &agg = agg_all[threadIdx.x >> 6];
+    agg_clear(agg, lane);
+    rp_vtab_stage(rp_shared, vtab);
+    if (threadIdx.x < 15) shc[threadIdx.x] = rp_shared[threadIdx.x];
+    __syncthreads();
+    const ldouble *t = (const ldouble *)shc;
+    const RPFastShared fsh{t[0], t[1], t[2],  t[3],  t[4],  t[5],  t[6], t[7],
+                           t[8], t[9], t[10], t[11], t[12], t[13], t[14], vtab};
+    // wavefront slots: the first wavefronts of all workgroups, then the second ...
+    const int wslot = (int)(threadIdx.x >> 6) * (int)gridDim.x + (int)blockIdx.x;
+    int nb, E;
+    {
+        const BubbleArrays &b = rpl(kp)->b;
+        nb = b.n;
+        E = ORDERED ? min(b.part[(b.n + 255) / 256], solo_cap) : nb;
     }
-    if (lane == 0) {
-        if (done) atomicAdd(&sc->done, done);
-        if (kept) atomicAdd(&sc->reused, kept);
-        if (sub_sum) atomicAdd(&sc->sub_sum, sub_sum);
-        if (sub_max > __hip_atomic_load(&sc->sub_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax(&sc->sub_max, sub_max);
+    int idx = -1;
+    bool solo = wslot < E;  // wave-uniform
+    bool fresh = false;
+    if (solo && lane < 2) {
+        idx = ORDERED ? rpl(kp)->b.order[wslot] : wslot;
+        fresh = true;
     }
-    if (bad) atomicOr(&sc->flags, 2);
-    if (capped_any) atomicOr(&sc->flags, 4);
+    if (solo) __builtin_amdgcn_s_setprio(3);
+    int batch_next = 0, batch_end = 0;  // wave-uniform
+    bool exhausted = !ORDERED;          // wave-uniform
+    bool reuse = false;
+    RPLaneF<double> L{};
+    RPFastConst fk{0, 0, 0, 0, 0, 0, 0, 0};
+    double x = 0.0, y = 0.0;
+    int ibnx = 0, ibny = 0;
+    int sub_max = 0;
+    unsigned long long sub_sum = 0;
+    unsigned int done = 0, kept = 0;
+    bool bad = false, capped_any = false;
+    while (true) {
+        if (solo && __ballot(idx >= 0) == 0ull) {
+            solo = false;
+            __builtin_amdgcn_s_setprio(0);
+        }
+        {  // ---- refill idle pairs (the even lane takes, its partner copies)
+            crpl *P = rpl(kp);
+            const GridParams &g = P->g;
+            const BubbleParams &bp = P->bp;
+            const BubbleArrays &b = P->b;
+            bool need = ORDERED && idx < 0 && !solo && !odd && (lane >> 1) < quota;
+            unsigned long long m = __ballot(need);
+            while (m != 0ull && !exhausted) {
+                if (batch_next >= batch_end) {
+                    const int leader = __ffsll((long long)m) - 1;
+                    unsigned int base = 0;
+                    if (lane == leader) base = atomicAdd(&sc->work[slot], (unsigned)quota);
+                    base = __shfl(base, leader, 64);
+                    if ((int)base >= nb - E) {
+                        exhausted = true;
+                        break;
+                    }
+                    batch_next = (int)base + E;
+                    batch_end = min((int)base + E + quota, nb);
+                }
+                const int avail = batch_end - batch_next;
+                const int rank = __popcll(m & lanemask_lt(lane));
+                if (need && rank < avail) {
+                    idx = b.order[batch_next + rank];
+                    need = false;
+                    fresh = true;
+                }
+                batch_next += min(avail, __popcll(m));
+                m = __ballot(need);
+            }
+            if (ORDERED && !solo) {
+                idx = __shfl(idx, lane & ~1, 64);
+                fresh = __shfl((int)fresh, lane & ~1, 64) != 0;
+            }
+            if (fresh) {
+                x = b.x[idx];
+                y = b.y[idx];
+                ibnx = bin_index(x, g.rdx, 0.5);
+                ibny = bin_index(y, g.rdy, 0.5);
+                double PL;
+                if (ORDERED) {
+                    PL = b.PL[plp][idx];  // gathered by k_queue_keys
+                    reuse = b.key[idx] < 0;
+                } else {  // k_queue_keys' gather and test
+                    PL = gather_p0(g, bp, p0, x, y, ibnx, ibny);
+                    reuse = slot > 1 && PL == b.PL[plp][idx];
+                    if (!odd) b.PL[plp][idx] = PL;
+                }
+                fk = rp_fast_const(b.R0[idx], b.PG0[idx], b.calpha[idx], bp.T0, fsh);
+                rp_begin_g(L, b.R[cur][idx], b.Rn[cur][idx], b.d1R[cur][idx], b.PG[cur][idx],
+                           b.bdt[cur][idx], b.re[cur][idx], b.PL[plm][idx], b.PL[pln][idx], PL,
+                           g.dt, bp.PL0);
+                if (reuse) L.remain = 0.0;
+                fresh = false;
+            }
+        }
+        const bool active = idx >= 0;
+        if (__ballot(active) == 0ull) break;
+        // ---- sub-steps: a bubble of its own to the end; else until half of
+        // the wavefront's pairs have finished, or none is running
+        if (solo) {
+            if (active) rp_integrate_pair(L, fk, fsh, odd, max_substeps);
+        } else {
+            while (true) {
+                const bool run = active && L.remain > 0.0 && L.counter < max_substeps;
+                const unsigned long long rm = __ballot(run);
+                if (rm == 0ull || (!exhausted && __popcll(rm) <= quota)) break;
+                if (run) rp_pair_pass<false>(L, fk, fsh, odd, max_substeps);
+            }
+        }
+        const bool capped = L.counter >= max_substeps;
+        const bool fin = active && (!(L.remain > 0.0) || capped);
+        if (fin && !odd) {  // ---- write back
+            crpl *P = rpl(kp);
+            const GridParams &g = P->g;
+            const BubbleParams &bp = P->bp;
+            const BubbleArrays &b = P->b;
+            double R_t;
+            if (reuse) {
+                R_t = b.R_t[idx];
+                kept++;
+            } else {
+                RPState out;
+                double Q_B;
+                rp_end_g(L, g.dt, &out, &R_t, &Q_B);
+                b.R[nxt][idx] = out.Rp;
+                b.Rn[nxt][idx] = out.Rn;
+                b.d1R[nxt][idx] = out.d1R;
+                b.PG[nxt][idx] = out.PG;
+                b.bdt[nxt][idx] = out.dt;
+                b.re[nxt][idx] = out.re;
+                b.R_t[idx] = R_t;
+                b.Q_B[idx] = Q_B;
+                b.sub[idx] = L.counter;
+                sub_max = max(sub_max, L.counter);
+                sub_sum += (unsigned long long)L.counter;
+                capped_any |= capped && L.remain > 0.0;
+            }
+            done++;
+            bad |= !isfinite(R_t);
+            scatter_bubble_agg(g, bp, x, y, ibnx, ibny, fg_temp_of(g, bp, b.n_B[idx], R_t, x), agg,
+                               fg_target, &bad);
+        }
+        if (fin) idx = -1;
+        if (__builtin_amdgcn_readfirstlane(agg.count) > kAggSlots / 2) agg_flush(agg, lane, fg_target);
+    }
+    agg_flush(agg, lane, fg_target);
+    rp_launch_totals(rpl(kp)->b.totals, lane, sub_max, sub_sum, done, kept, bad, capped_any);
 }
 
 // ---- frozen schedule (finite differences of the frozen-schedule map) ------
@@ -579,7 +753,7 @@ __global__ __launch_bounds__(256) void k_rp_record(const RPLaunch *kp, int cur, 
                                                     int plp, const int64_t *off, double *dts,
                                                     unsigned int *mismatch) {
     const RPLaunch &P = *kp;
-    __shared__ double vtab[kRpVSize];
+    __shared__ __align__(16) double vtab[kRpVSize];
     rp_vtab_stage(P.bp.rp_shared, vtab);
     __syncthreads();
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -624,7 +798,7 @@ __global__ __launch_bounds__(256) void k_rp_replay(const RPLaunch *kp, int cur, 
     const BubbleArrays &b = P.b;
     const int lane = threadIdx.x & 63;
     __shared__ WaveAgg agg_all[4];
-    __shared__ double vtab[kRpVSize];
+    __shared__ __align__(16) double vtab[kRpVSize];
     WaveAgg &agg = agg_all[threadIdx.x >> 6];
     agg_clear(agg, lane);
     rp_vtab_stage(bp.rp_shared, vtab);
@@ -842,13 +1016,41 @@ int bubble_step_blocks(int n_bubbles, bool lean, int cus, int per_cu) {
     return std::max(1, std::min(cus * (lean ? 1 : per_cu), (n_bubbles + 255) / 256));
 }
 
+// Every bubble on a lane pair while that gives a wavefront at most eight of
+// them (one wavefront per SIMD): a pair halves the Omega and Lp work of a
+// sub-step but takes two lanes.  RP launch of collapsing bubbles, the queue
+// of k_bubble_persistent against pairs: 1024 bubbles 1.62 against 1.11 ms,
+// 2500 1.90 against 1.55, 8000 1.43 against 1.40, 30 011 1.76 against 1.79,
+// 65 536 1.37 against 1.40.  The cap of one dedicated wavefront per workgroup
+// holds here too: two or three of them cost 30 011 bubbles 5 and 7 %, 65 536
+// 14 %, and 2500 nothing either way.
+bool bubble_step_pairs(const RPLaunch &host, int cus) {
+    return !host.bp.rp_exact && host.b.n <= 8 * 4 * cus;
+}
+bool bubble_step_unordered(const RPLaunch &host, int cus) {
+    return bubble_step_pairs(host, cus) && host.b.n <= 4 * cus;
+}
+
 template <typename F>
-void launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
-                        int plm, int pln, int plp, int64_t *fg_target,
+int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
+                        int plm, int pln, int plp, const F *p0, int64_t *fg_target,
                         StepScalars *sc, int slot, bool lean, int cus, int per_cu) {
-    if (host.b.n <= 0) return;
-    const dim3 grid(bubble_step_blocks(host.b.n, lean, cus, per_cu));
+    if (host.b.n <= 0) return 0;
     const int cap = host.bp.max_substeps;
+    if (bubble_step_pairs(host, cus)) {
+        const int n = host.b.n, waves = 4 * cus;
+        const int blocks = std::min(cus, n);
+        if (n <= waves)
+            hipLaunchKernelGGL((k_bubble_pairs<F, false>), dim3(blocks), dim3(256), 0, s,
+                               dev, cap, host.bp.rp_shared, cur, plm, pln, plp, p0, fg_target, sc,
+                               slot, 1, 0);
+        else
+            hipLaunchKernelGGL((k_bubble_pairs<F, true>), dim3(blocks), dim3(256), 0, s, dev, cap,
+                               host.bp.rp_shared, cur, plm, pln, plp, p0, fg_target, sc, slot,
+                               (n + waves - 1) / waves, cus);
+        return 4 * blocks;
+    }
+    const dim3 grid(bubble_step_blocks(host.b.n, lean, cus, per_cu));
     // Dedicated wavefronts: up to one per workgroup on the lean grid, where
     // the longest chains bound the launch; CUs / 8 on the full grid, which
     // is chosen when the total work bounds it: a wavefront with one active
@@ -866,6 +1068,7 @@ void launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev
         hipLaunchKernelGGL((k_bubble_persistent<F, true>), grid, dim3(256), 0, s, dev, cap,
                            host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, slot,
                            solo_cap);
+    return 4 * (int)grid.x;
 }
 
 // Work-queue order (longest-first scheduling: long sequential sub-step
@@ -1178,11 +1381,11 @@ template void launch_motion<double>(hipStream_t, const GridParams &, const Bubbl
 template void launch_motion<float>(hipStream_t, const GridParams &, const BubbleParams &,
                                    const BubbleArrays &, const float *, const float *,
                                    StepScalars *);
-template void launch_bubble_step<double>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
-                                         int, int, int64_t *, StepScalars *, int, bool, int,
+template int launch_bubble_step<double>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
+                                         int, int, const double *, int64_t *, StepScalars *, int, bool, int,
                                          int);
-template void launch_bubble_step<float>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
-                                         int, int, int64_t *, StepScalars *, int, bool, int,
+template int launch_bubble_step<float>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
+                                         int, int, const float *, int64_t *, StepScalars *, int, bool, int,
                                          int);
 
 }  // namespace brp

@@ -424,15 +424,48 @@ __global__ __launch_bounds__(256) void k_pressure_picard(
     block_max_to(rmax, &sc->resid[slot]);
 }
 
+__device__ inline void totals_add(RPTotals &a, const RPTotals &b) {
+    a.sub_sum += b.sub_sum;
+    a.done += b.done;
+    a.kept += b.kept;
+    a.sub_max = max(a.sub_max, b.sub_max);
+    a.flags |= b.flags;
+}
+
 // MixtureBoundaryPressureKernel (bubble_CUDA_kernel.cuh:870-952) for order 2,
 // parts in program order in one workgroup.  Extension E1 (g.src_row) writes
-// the source row even when pml.y0 = 1.
+// the source row even when pml.y0 = 1.  After a Picard iteration's RP launch
+// the workgroup also adds the n_tot wavefront records to the step's scalars:
+// two or three atomics of every wavefront on one address each cost the launch
+// about 14 ns apiece (256^2, 1024 bubbles, one per wavefront: 73 us a launch
+// with them, 25 us with the records).
 template <typename F>
 __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           const double *el_amp,
-                                                          const double *el_phase, double t) {
+                                                          const double *el_phase, double t,
+                                                          const RPTotals *tot, int n_tot,
+                                                          StepScalars *sc) {
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
+    if (n_tot > 0) {  // workgroup-uniform
+        __shared__ RPTotals red[16];
+        RPTotals a{0ull, 0u, 0u, 0, 0};
+        for (int k = tid; k < n_tot; k += nt) totals_add(a, tot[k]);
+        for (int off = 32; off > 0; off >>= 1)
+            totals_add(a, RPTotals{__shfl_xor(a.sub_sum, off, 64), __shfl_xor(a.done, off, 64),
+                                   __shfl_xor(a.kept, off, 64), __shfl_xor(a.sub_max, off, 64),
+                                   __shfl_xor(a.flags, off, 64)});
+        if ((tid & 63) == 0) red[tid >> 6] = a;
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < nt / 64; w++) totals_add(a, red[w]);
+            sc->sub_sum += a.sub_sum;
+            sc->done += a.done;
+            sc->reused += a.kept;
+            sc->sub_max = max(sc->sub_max, a.sub_max);
+            sc->flags |= a.flags;
+        }
+    }
     const double pamp = g.rho_inf * g.cs_inf * g.amp;
     for (int i = 1 + tid; i <= N; i += nt) {
         if (!g.pml_y0) p0[frame_off(i, 0, P)] = p0[frame_off(i, 1, P)];
@@ -527,9 +560,10 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
 
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
-                            const double *el_phase, double t) {
+                            const double *el_phase, double t, const RPTotals *tot, int n_tot,
+                            StepScalars *sc) {
     hipLaunchKernelGGL(k_pressure_ghosts<F>, dim3(1), dim3(1024), 0, s, g, p0, el_amp,
-                       el_phase, t);
+                       el_phase, t, tot, n_tot, sc);
 }
 
 void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
@@ -551,7 +585,8 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
         F *, F *, const int64_t *, const int64_t *, int64_t *, Window, const F *, const F *, \
         const F *, const F *, const double *, const double *, StepScalars *, int);           \
     template void launch_pressure_ghosts<F>(hipStream_t, const GridParams &, F *,           \
-                                            const double *, const double *, double);
+                                            const double *, const double *, double,          \
+                                            const RPTotals *, int, StepScalars *);
 
 BRP_INST(double)
 BRP_INST(float)

@@ -124,7 +124,12 @@ typedef const double ldouble;  // the host pass only parses device code
 // Copies the V and Y tables (kRpVSize doubles from the device table) into the
 // workgroup's LDS array; the caller synchronises the workgroup afterwards.
 __device__ inline void rp_vtab_stage(const double *tab, double *lds) {
-    for (int k = threadIdx.x; k < kRpVSize; k += blockDim.x) lds[k] = tab[kRpVOffset + k];
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 *src = (const d2 *)(tab + kRpVOffset);
+    d2 *dst = (d2 *)lds;
+    static_assert(kRpVSize % 2 == 0 && kRpVOffset % 2 == 0, "16-byte pieces");
+#pragma unroll 13
+    for (int k = threadIdx.x; k < kRpVSize / 2; k += 256) dst[k] = src[k];
 }
 
 struct cx_d {
@@ -468,7 +473,7 @@ __device__ inline double quad_move(double v) {
 __device__ inline double from_even(double v) { return quad_move<0xA0>(v); }  // quad_perm 0,0,2,2
 __device__ inline double from_odd(double v) { return quad_move<0xF5>(v); }   // quad_perm 1,1,3,3
 
-// A bubble's whole integration on a pair of lanes (both hold its state).
+// Up to two sub-steps of a bubble on a pair of lanes (both hold its state).
 // The Omega iteration and Lp, more than half of a sub-step's instructions,
 // depend on the radius a sub-step starts from alone; the next sub-step starts
 // from the radius this one reaches, which needs only the gas pressure of the
@@ -476,22 +481,28 @@ __device__ inline double from_odd(double v) { return quad_move<0xF5>(v); }   // 
 // successor start from are both known, and the two lanes evaluate Omega and
 // Lp for both at once, in the one instruction stream that the wavefront
 // issues anyway.  The operations of each sub-step and their order are
-// rp_substep_g's, so the results are its results bit for bit.  All lanes of
-// the wavefront that run this hold one bubble (UNI conditions).
-__device__ inline void rp_integrate_pair(RPLaneF<double> &L, const RPFastConst &k,
-                                         const RPFastShared &s, bool odd, int max_substeps) {
-    while (cond<true>(L.remain > 0.0 && L.counter < max_substeps)) {
-        const RPMove<double> m0 = rp_advance_g<double, false, true>(L, s);
-        const double R = odd ? L.Rp : m0.Rn;
-        cx<double> Ln;
-        double iom;
-        omega_lp_g<double>(R, drcp(R), k, s, &Ln, &iom);
-        rp_gas_g<double>(L, m0, cx<double>{from_even(Ln.re), from_even(Ln.im)}, from_even(iom), k,
-                         s);
-        if (!cond<true>(L.remain > 0.0 && L.counter < max_substeps)) break;
-        const RPMove<double> m1 = rp_advance_g<double, false, true>(L, s);
+// rp_substep_g's, so the results are its results bit for bit.  UNI: all lanes
+// of the wavefront that run this hold one bubble.
+template <bool UNI>
+__device__ inline void rp_pair_pass(RPLaneF<double> &L, const RPFastConst &k,
+                                    const RPFastShared &s, bool odd, int max_substeps) {
+    const RPMove<double> m0 = rp_advance_g<double, false, UNI>(L, s);
+    const double R = odd ? L.Rp : m0.Rn;
+    cx<double> Ln;
+    double iom;
+    omega_lp_g<double>(R, drcp(R), k, s, &Ln, &iom);
+    rp_gas_g<double>(L, m0, cx<double>{from_even(Ln.re), from_even(Ln.im)}, from_even(iom), k, s);
+    if (cond<UNI>(L.remain > 0.0 && L.counter < max_substeps)) {
+        const RPMove<double> m1 = rp_advance_g<double, false, UNI>(L, s);
         rp_gas_g<double>(L, m1, cx<double>{from_odd(Ln.re), from_odd(Ln.im)}, from_odd(iom), k, s);
     }
+}
+
+// The whole integration of the one bubble that a wavefront's lane pair holds.
+__device__ inline void rp_integrate_pair(RPLaneF<double> &L, const RPFastConst &k,
+                                         const RPFastShared &s, bool odd, int max_substeps) {
+    while (cond<true>(L.remain > 0.0 && L.counter < max_substeps))
+        rp_pair_pass<true>(L, k, s, odd, max_substeps);
 }
 
 // ---- reverse mode: adjoints of the RP map of one Picard iteration ----------

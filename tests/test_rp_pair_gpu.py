@@ -10,9 +10,10 @@ import cases
 pytestmark = pytest.mark.gpu
 
 
-# one bubble; fewer than a workgroup; one lane more than a wavefront and a
-# workgroup; more than the lanes of the first workgroups
-@pytest.mark.parametrize("nb", [1, 3, 65, 257, 1500])
+# one bubble; fewer than a workgroup; one more than a wavefront and a workgroup;
+# the last and first population that takes each of the three launches (one bubble
+# a wavefront, a queue of lane pairs, a queue of lanes)
+@pytest.mark.parametrize("nb", [1, 3, 65, 257, 1024, 1025, 1500, 8192, 8193])
 @pytest.mark.parametrize("mixed", [0, 1])
 def test_launch_equals_one_lane_integration(brp, nb, mixed):
     prec = brp.abi.PREC_MIXED if mixed else brp.abi.PREC_FP64
