@@ -440,6 +440,8 @@ int alloc_bubbles(brp_handle *h, int n) {
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.part, sizeof(int) * 2 * (size_t)((n + 255) / 256 + 1))))
         return rc;
+    if ((rc = dalloc(h, (void **)&h->b.heads, sizeof(unsigned int) * kQueueHeads * kHeadStride)))
+        return rc;
     if ((rc = dalloc(h, (void **)&h->b.totals, sizeof(RPTotals) * 4 * (size_t)(h->cus * h->per_cu))))
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.bbox_blk, sizeof(int) * 4 * (size_t)((n + 255) / 256 + 1))))

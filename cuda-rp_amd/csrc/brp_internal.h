@@ -72,6 +72,10 @@ struct RPTotals {
     int sub_max, flags;          // StepScalars::flags bits
 };
 
+// The RP launch's work queue has kQueueHeads heads, each on a line of its own:
+// head q hands out the batches q, q + kQueueHeads, ... of the queue order.
+constexpr int kQueueHeads = 16, kHeadStride = 32;
+
 // Device-side per-step scalars written by the kernels and read by the host.
 struct StepScalars {
     int bbox[4];                         // min i, max i, min j, max j of bubble stencils
@@ -83,7 +87,6 @@ struct StepScalars {
     unsigned int reused;                 // of them, kept from the previous iteration
     double focal[2];                     // (x, y) of the largest temperature increment
     unsigned long long resid[kMaxEval];  // max |dp0| bit patterns (>= 0 doubles)
-    unsigned int work[kMaxEval];         // bubble work-queue heads, one per Picard iteration
     double focal_v[256];                 // per-block maxima of the focal-point search
     int focal_i[256];
 };
@@ -105,6 +108,7 @@ struct BubbleArrays {
     int *part;            // partition scratch: per-block extreme and heavy offsets + totals
     int *bbox_blk;        // per-block stencil bounding boxes of k_motion (4 ints each)
     RPTotals *totals;     // per wavefront of the RP launch
+    unsigned int *heads;  // kQueueHeads work-queue heads, kHeadStride apart
 };
 
 // Bubble physics constants shared by every bubble.

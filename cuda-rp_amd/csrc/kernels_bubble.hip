@@ -307,6 +307,40 @@ __device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
             RPTotals{sub_sum, done, kept, sub_max, flags};
 }
 
+// The next batch of `size` entries of a wavefront from the queue of n (whole
+// wavefront).  `head` (wave-uniform) is the head it draws from; when that has
+// run out, one read of all heads finds another that has not, or that the
+// queue is empty (returns false).  One head for all wavefronts hands out a
+// batch every 14 ns, which bounds a launch of short chains: 2^20 bubbles with
+// 11 sub-steps each, in batches of 64, 260 us a launch with one head, 211 us
+// with sixteen.
+__device__ inline bool queue_batch(unsigned int *heads, int lane, int n, int size, int &head,
+                                   int &next, int &end) {
+    while (head >= 0) {
+        unsigned int k = 0;
+        if (lane == 0) k = atomicAdd(&heads[head * kHeadStride], 1u);
+        k = __builtin_amdgcn_readfirstlane(k);
+        const long long base = ((long long)k * kQueueHeads + head) * size;
+        if (base < n) {
+            next = (int)base;
+            end = min((int)base + size, n);
+            return true;
+        }
+        bool alive = false;
+        if (lane < kQueueHeads) {
+            const unsigned int h = __hip_atomic_load(&heads[lane * kHeadStride], __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+            alive = ((long long)h * kQueueHeads + lane) * size < n;
+        }
+        const unsigned long long m = __ballot(alive);
+        // the first live head after this one, in a circle (a head that has
+        // run out stays so: this ends)
+        const unsigned long long up = m & ~((2ull << head) - 1);
+        head = m ? __ffsll((long long)(up ? up : m)) - 1 : -1;
+    }
+    return false;
+}
+
 // One Picard iteration for every bubble, fused (after k_queue_keys gathered
 // PL_p, BubbleInterpolationScalarKernel, kernel.cuh:361-395):
 //   BubbleRadiusKernel              (RP from the step's start state, 471-554)
@@ -319,9 +353,9 @@ __device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
 // through an inertial collapse), so one bubble per lane would run each
 // wavefront at the pace of its slowest lane.  Here every lane integrates one
 // sub-step per loop pass; lanes whose bubbles reached the sync time are
-// written back and refilled with the next bubbles once kRefillBatch of them
-// have finished.  Bubbles are handed to wavefronts in
-// batches of 64 consecutive (cell-sorted) indices through one atomic counter
+// written back and refilled with the next bubbles once half of them have
+// finished.  Bubbles are handed to wavefronts in
+// batches of 64 consecutive (cell-sorted) indices through sixteen atomic counters
 // per Picard iteration, so a wavefront costs the sum, not the max, of its
 // lanes' sub-steps.  Per bubble the arithmetic is exactly that of the
 // reference kernel, so results do not depend on the schedule.
@@ -339,19 +373,18 @@ __device__ inline crpl *rpl(const RPLaunch *p) {
     return q;
 }
 
-// Finished lanes a wavefront collects before it leaves the sub-step loop to
-// write them back and refill them (4096^2 clustered on the lean grid, ms per
-// step: 16 24.5, 24 23.3, 32 23.0, 40 23.2, 48 24.2; 2048^2 equal within 1 %
-// from 24 to 48).
-constexpr int kRefillBatch = 32;
-
+// A shared wavefront holds at most `quota` bubbles (64 but for a population
+// too small to give every wavefront 64), takes as many from the queue at a
+// time, and leaves the sub-step loop to write back and refill when half of
+// them have finished (4096^2 clustered on the lean grid, quota 64, ms per step
+// for 16 / 24 / 32 / 40 / 48 finished lanes: 24.5 / 23.3 / 23.0 / 23.2 / 24.2;
+// 2048^2 equal within 1 % from 24 to 48).
 template <typename F, bool FAST>
 __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, int max_substeps,
                                                             const double *rp_shared, int cur,
                                                             int plm, int pln, int plp,
                                                             int64_t *__restrict__ fg_target,
-                                                            StepScalars *sc, int slot,
-                                                            int solo_cap) {
+                                                            int quota, int solo_cap) {
     const int lane = threadIdx.x & 63;
     const int nxt = cur ^ 1;
     __shared__ WaveAgg agg_all[4];  // 25 KB: one table per wavefront
@@ -406,6 +439,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     bool solo = threadIdx.x < 64 && (int)blockIdx.x < E;  // wave-uniform
     if (solo) __builtin_amdgcn_s_setprio(3);
     int batch_next = 0, batch_end = 0;  // wave-uniform
+    int head = (int)blockIdx.x & (kQueueHeads - 1);  // wave-uniform
     bool exhausted = false;             // wave-uniform
     RPLane L;              // operation-by-operation path
     RPLaneF<double> LF;    // shortened-chain path
@@ -423,7 +457,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
             __builtin_amdgcn_s_setprio(0);
         }
         // ---- refill idle lanes from the wave's batch / the global queue
-        bool need = idx < 0 && !solo;
+        bool need = idx < 0 && !solo && lane < quota;
         {
         crpl *P = rpl(kp);
         const GridParams &g = P->g;
@@ -433,22 +467,15 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         bool fresh = pre;
         pre = false;
         while (m != 0ull && !exhausted) {
-            if (batch_next >= batch_end) {
-                const int leader = __ffsll((long long)m) - 1;
-                unsigned int base = 0;
-                if (lane == leader) base = atomicAdd(&sc->work[slot], 64u);
-                base = __shfl(base, leader, 64);
-                if ((int)base >= nb - E) {
-                    exhausted = true;
-                    break;
-                }
-                batch_next = (int)base + E;
-                batch_end = min((int)base + E + 64, nb);
+            if (batch_next >= batch_end &&
+                !queue_batch(b.heads, lane, nb - E, quota, head, batch_next, batch_end)) {
+                exhausted = true;
+                break;
             }
             const int avail = batch_end - batch_next;
             const int rank = __popcll(m & lanemask_lt(lane));
             if (need && rank < avail) {
-                idx = b.order[batch_next + rank];
+                idx = b.order[E + batch_next + rank];
                 need = false;
                 fresh = true;
             }
@@ -483,7 +510,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         }
         const bool active = idx >= 0;
         if (__ballot(active) == 0ull) break;
-        // ---- sub-steps until kRefillBatch lanes' bubbles have reached the
+        // ---- sub-steps until half of the quota's bubbles have reached the
         // sync time (or the sub-step cap), or no active lane is left
         // running; finished lanes idle meanwhile.  The refill and write-back
         // code stays outside this loop, and with it the values only that
@@ -520,7 +547,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
             }
             fin = active && (!(remain > 0.0) || capped);
             const unsigned long long fm = __ballot(fin);
-            if (fm != 0ull && (__popcll(fm) >= kRefillBatch || __ballot(active && !fin) == 0ull))
+            if (fm != 0ull && (2 * __popcll(fm) >= quota || __ballot(active && !fin) == 0ull))
                 break;
         }
         // ---- write back the bubbles that reached the sync time
@@ -616,6 +643,7 @@ __global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int ma
     }
     if (solo) __builtin_amdgcn_s_setprio(3);
     int batch_next = 0, batch_end = 0;  // wave-uniform
+    int head = (int)blockIdx.x & (kQueueHeads - 1);  // wave-uniform
     bool exhausted = !ORDERED;          // wave-uniform
     bool reuse = false;
     RPLaneF<double> L{};
@@ -639,22 +667,15 @@ __global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int ma
             bool need = ORDERED && idx < 0 && !solo && !odd && (lane >> 1) < quota;
             unsigned long long m = __ballot(need);
             while (m != 0ull && !exhausted) {
-                if (batch_next >= batch_end) {
-                    const int leader = __ffsll((long long)m) - 1;
-                    unsigned int base = 0;
-                    if (lane == leader) base = atomicAdd(&sc->work[slot], (unsigned)quota);
-                    base = __shfl(base, leader, 64);
-                    if ((int)base >= nb - E) {
-                        exhausted = true;
-                        break;
-                    }
-                    batch_next = (int)base + E;
-                    batch_end = min((int)base + E + quota, nb);
+                if (batch_next >= batch_end &&
+                    !queue_batch(b.heads, lane, nb - E, quota, head, batch_next, batch_end)) {
+                    exhausted = true;
+                    break;
                 }
                 const int avail = batch_end - batch_next;
                 const int rank = __popcll(m & lanemask_lt(lane));
                 if (need && rank < avail) {
-                    idx = b.order[batch_next + rank];
+                    idx = b.order[E + batch_next + rank];
                     need = false;
                     fresh = true;
                 }
@@ -1012,8 +1033,14 @@ bool bubble_step_lean(int sub_max, double sub_per_launch, int extreme_threshold,
     return sub_max >= 2 * extreme_threshold && sub_per_launch < 0.6 * lanes * sub_max;
 }
 
+// A lean launch spreads a small population over all its compute units (30 011
+// bubbles: 1.84 ms on 118 workgroups of 256 lanes, 1.75 on 256 with 30 bubbles
+// to a wavefront); a full one, whose chains are short, fills its wavefronts,
+// since each has the tables to stage and its sums to flush (45 000 bubbles
+// with 10 sub-steps: 32 us on 176 workgroups, 42 on 512).
 int bubble_step_blocks(int n_bubbles, bool lean, int cus, int per_cu) {
-    return std::max(1, std::min(cus * (lean ? 1 : per_cu), (n_bubbles + 255) / 256));
+    return std::max(1, lean ? std::min(cus, (n_bubbles + 31) / 32)
+                            : std::min(cus * per_cu, (n_bubbles + 255) / 256));
 }
 
 // Every bubble on a lane pair while that gives a wavefront at most eight of
@@ -1051,23 +1078,22 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
         return 4 * blocks;
     }
     const dim3 grid(bubble_step_blocks(host.b.n, lean, cus, per_cu));
+    const int quota = std::max(8, std::min(64, (host.b.n + 4 * (int)grid.x - 1) / (4 * (int)grid.x)));
     // Dedicated wavefronts: up to one per workgroup on the lean grid, where
     // the longest chains bound the launch; CUs / 8 on the full grid, which
     // is chosen when the total work bounds it: a wavefront with one active
     // lane still takes its SIMD's issue slots, so every dedicated wavefront
     // costs a SIMD of throughput there.  4096^2, 2^22 clustered bubbles
     // (full grid): 512 dedicated 49.8, 128 46.8, 32 46.4, 0 46.2 ms/step;
-    // with refills batched by kRefillBatch: 128 29.6, 64 29.2, 32 29.3,
+    // with refills batched: 128 29.6, 64 29.2, 32 29.3,
     // 0 30.8; 2048^2 (lean grid): 256 17.2, 32 17.4, 0 19.1 ms/step.
     const int solo_cap = lean ? (int)grid.x : std::max(1, cus / 8);
     if (host.bp.rp_exact)
         hipLaunchKernelGGL((k_bubble_persistent<F, false>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, slot,
-                           solo_cap);
+                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, quota, solo_cap);
     else
         hipLaunchKernelGGL((k_bubble_persistent<F, true>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, slot,
-                           solo_cap);
+                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, quota, solo_cap);
     return 4 * (int)grid.x;
 }
 
@@ -1081,10 +1107,13 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
 constexpr int kSortBins = 2048;  // bins of the extreme-class sort
 
 __global__ __launch_bounds__(256) void k_part_count(const int *sub, int n, int ext, int thr,
-                                                    int *cntE, int *cntH, int *sort_hist) {
+                                                    int *cntE, int *cntH, int *sort_hist,
+                                                    unsigned int *heads) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0) {
         for (int k = threadIdx.x; k < kSortBins; k += 256) sort_hist[k] = 0;
+        if (threadIdx.x < kQueueHeads) heads[threadIdx.x * kHeadStride] = 0u;
+    }
     const int v = idx < n ? sub[idx] : 0;
     const int ce = __syncthreads_count(idx < n && v >= ext);
     const int ch = __syncthreads_count(idx < n && v >= thr && v < ext);
@@ -1300,7 +1329,7 @@ void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key
     const int nblk = (b.n + 255) / 256;
     int *cntE = b.part, *cntH = b.part + (nblk + 1);
     hipLaunchKernelGGL(k_part_count, dim3(nblk), dim3(256), 0, s, key, b.n, ext, threshold,
-                       cntE, cntH, b.sort_hist);
+                       cntE, cntH, b.sort_hist, b.heads);
     hipLaunchKernelGGL(k_part_scan, dim3(2), dim3(1024), 0, s, cntE, nblk);
     hipLaunchKernelGGL(k_part_scatter, dim3(nblk), dim3(256), 0, s, key, b.n, ext, threshold,
                        cntE, cntH, nblk, b.order, b.order_tmp);
