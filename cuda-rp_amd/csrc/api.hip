@@ -222,6 +222,8 @@ struct brp_handle {
     double *xu_d = nullptr, *rxp_d = nullptr;
     double *el_amp_d = nullptr, *el_phase_d = nullptr;
     int *perm_d = nullptr;           // perm on the device (sorted -> caller index)
+    int *iperm_d = nullptr;          // its inverse (caller index -> sorted)
+    HostRing ring;                   // pinned slots of read-backs
     double *scratch_d = nullptr;     // this device's `scratch` (nullptr: lookup failed)
     std::string scratch_err;
     double *T_d = nullptr, *dT_d = nullptr, *heat_d = nullptr;  // temperature solve
@@ -492,8 +494,13 @@ int place_bubbles(brp_handle *h, const std::vector<double> &x, const std::vector
         return BRP_OK;
     };
     if ((rc = dalloc(h, (void **)&h->perm_d, sizeof(int) * (size_t)std::max(n, 1)))) return rc;
-    if (n > 0)
+    if ((rc = dalloc(h, (void **)&h->iperm_d, sizeof(int) * (size_t)std::max(n, 1)))) return rc;
+    if (n > 0) {
+        std::vector<int> iperm(n);
+        for (int k = 0; k < n; k++) iperm[h->perm[k]] = k;
         HIPCHK(h, hipMemcpy(h->perm_d, h->perm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+        HIPCHK(h, hipMemcpy(h->iperm_d, iperm.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    }
     if ((rc = up(h->b.x, hx)) || (rc = up(h->b.y, hy)) || (rc = up(h->b.R0, R0)) ||
         (rc = up(h->b.PG0, PG0)) || (rc = up(h->b.calpha, ca)) || (rc = up(h->b.n_B, nB)) ||
         (rc = up(h->b.R_t, R0)) || (rc = up(h->b.Q_B, zero)) || (rc = up(h->b.vx, zero)) ||
@@ -1428,15 +1435,8 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
 
     // gradients
     if (grad_fg0) {
-        std::vector<double> c(fr), nn(fr), m(fr);
-        HIPCHK(h, hipMemcpy(c.data(), a.LfC, sizeof(double) * fr, hipMemcpyDeviceToHost));
-        HIPCHK(h, hipMemcpy(nn.data(), a.LfN, sizeof(double) * fr, hipMemcpyDeviceToHost));
-        HIPCHK(h, hipMemcpy(m.data(), a.LfM, sizeof(double) * fr, hipMemcpyDeviceToHost));
-        for (int j = 0; j <= h->M + 1; j++)
-            for (int i = 0; i <= h->N + 1; i++) {
-                const int64_t o = frame_off(i, j, h->pitch);
-                grad_fg0[(int64_t)j * ld + i] = c[o] + nn[o] + m[o];
-            }
+        const PackSrc p{PackSrc::kSum3, h->N + 2, a.LfC, a.LfN, a.LfM, nullptr, 0, 0, h->pitch, 0.0};
+        HIPCHK(h, read_back(s, h->device, h->ring, p, h->M + 2, grad_fg0, ld));
     }
     if ((grad_amp || grad_phase) && h->n_elem > 0) {
         std::vector<double> gA(h->N + 2), gP(h->N + 2);
@@ -1646,9 +1646,14 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
             return fail(set_err(h, BRP_ERR_DEVICE, "hipMemcpy failed"));
         bp.rp_shared = tab;
     }
-    if (hipHostMalloc((void **)&h->sc_h, sizeof(StepScalars), hipHostMallocDefault) != hipSuccess ||
+    // the host's copy of the step scalars and, behind it, the small read-back slot
+    const size_t sc_bytes = (sizeof(StepScalars) + 255) & ~size_t(255);
+    h->ring.small_doubles = std::min<int64_t>(HostRing::kMaxSmall, (int64_t)(h->N + 3) * (h->M + 3));
+    if (hipHostMalloc((void **)&h->sc_h, sc_bytes + sizeof(double) * h->ring.small_doubles,
+                      hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&h->rpl_h, sizeof(RPLaunch), hipHostMallocDefault) != hipSuccess)
         return fail(set_err(h, BRP_ERR_DEVICE, "hipHostMalloc failed"));
+    h->ring.small = (double *)((char *)h->sc_h + sc_bytes);
     if ((rc = dalloc(h, (void **)&h->rpl_d, sizeof(RPLaunch)))) return fail(rc);
     // init_bub_array (bubble_CUDA.cu:797-897): one bubble per cell centre in the box
     if (c.bub_enable) {
@@ -1678,6 +1683,7 @@ void brp_destroy(brp_handle *h) {
     for (auto &sn : h->snaps)
         for (void *p : sn.bufs) (void)hipFree(p);
     for (void *p : h->allocs) (void)hipFree(p);
+    h->ring.release();
     if (h->sc_h) (void)hipHostFree(h->sc_h);
     if (h->rpl_h) (void)hipHostFree(h->rpl_h);
     for (auto &e : h->ev)
@@ -1809,39 +1815,31 @@ int brp_get_field(brp_handle *h, int32_t field, double *dst, int64_t ld) {
     if (ld < nx) return set_err(h, BRP_ERR_INVALID, "ld %lld < %d", (long long)ld, nx);
     int rc = brp_prepare(h);
     if (rc) return rc;
-    std::vector<double> fr;
-    const bool dbl = h->prec == BRP_PREC_FP64;
-    auto rd = [&](const void *src) { return dbl ? read_frame<double>(h, src, fr) : read_frame<float>(h, src, fr); };
+    PackSrc p{h->prec == BRP_PREC_FP64 ? PackSrc::kDouble : PackSrc::kFloat, nx, nullptr, nullptr,
+              nullptr, nullptr, i0, j0, h->pitch, h->rho_inf};
+    double fill = 0.0;  // the value of a field without an array
     switch (field) {
-        case BRP_FIELD_P0: rc = rd(h->p0); break;
-        case BRP_FIELD_PX: rc = rd(h->pb[h->pc][0]); break;
-        case BRP_FIELD_PY: rc = rd(h->pb[h->pc][1]); break;
-        case BRP_FIELD_VX: rc = rd(h->vx); break;
-        case BRP_FIELD_VY: rc = rd(h->vy); break;
-        case BRP_FIELD_FG: rc = read_frame_fg(h, h->fgb[h->fcur], fr); break;
-        case BRP_FIELD_FGN: rc = read_frame_fg(h, h->fgb[h->fn], fr); break;
-        case BRP_FIELD_FGM: rc = read_frame_fg(h, h->fgb[h->fm], fr); break;
+        case BRP_FIELD_P0: p.src = h->p0; break;
+        case BRP_FIELD_PX: p.src = h->pb[h->pc][0]; break;
+        case BRP_FIELD_PY: p.src = h->pb[h->pc][1]; break;
+        case BRP_FIELD_VX: p.src = h->vx; break;
+        case BRP_FIELD_VY: p.src = h->vy; break;
+        case BRP_FIELD_FG: p.kind = PackSrc::kFixed; p.src = h->fgb[h->fcur]; break;
+        case BRP_FIELD_FGN: p.kind = PackSrc::kFixed; p.src = h->fgb[h->fn]; break;
+        case BRP_FIELD_FGM: p.kind = PackSrc::kFixed; p.src = h->fgb[h->fm]; break;
         case BRP_FIELD_RHO_M:
-            if (h->first_step) {
-                fr.assign(h->frame, h->rho_inf);
-            } else {
-                rc = read_frame_fg(h, h->fgb[h->fcur], fr);
-                for (double &v : fr) v = (1.0 - v) * h->rho_inf;
-            }
+            p.kind = PackSrc::kDensity;
+            p.src = h->first_step ? nullptr : h->fgb[h->fcur];
+            fill = h->rho_inf;
             break;
-        case BRP_FIELD_T:
-            if (h->T_d) {
-                fr.resize(h->frame);
-                HIPCHK(h, hipMemcpy(fr.data(), h->T_d, sizeof(double) * h->frame, hipMemcpyDeviceToHost));
-            } else {
-                fr.assign(h->frame, 0.0);
-            }
-            break;
+        case BRP_FIELD_T: p.kind = PackSrc::kDouble; p.src = h->T_d; break;
         default: return BRP_ERR_INVALID;
     }
-    if (rc) return rc;
-    for (int j = 0; j < ny; j++)
-        for (int i = 0; i < nx; i++) dst[(size_t)j * ld + i] = fr[frame_off(i + i0, j + j0, h->pitch)];
+    if (!p.src) {
+        for (int j = 0; j < ny; j++) std::fill_n(dst + (size_t)j * ld, nx, fill);
+        return BRP_OK;
+    }
+    HIPCHK(h, read_back(h->stream, h->device, h->ring, p, ny, dst, ld));
     return BRP_OK;
 }
 
@@ -1910,8 +1908,9 @@ int brp_get_bubbles(brp_handle *h, int32_t which, double *dst) {
     if (rc) return rc;
     const int n = h->nb;
     if (n == 0) return BRP_OK;
-    const double *src = nullptr;
+    const void *src = nullptr;
     double *tmpd = nullptr;
+    PackSrc::Kind kind = PackSrc::kPerm;
     const int c = h->rp_cur;
     switch (which) {
         case BRP_BUB_X: src = h->b.x; break;
@@ -1931,24 +1930,17 @@ int brp_get_bubbles(brp_handle *h, int32_t which, double *dst) {
         case BRP_BUB_VX: src = h->b.vx; break;
         case BRP_BUB_VY: src = h->b.vy; break;
         case BRP_BUB_R0: src = h->b.R0; break;
-        case BRP_BUB_SUB: {
-            std::vector<int> iv(n);
-            HIPCHK(h, hipMemcpy(iv.data(), h->b.sub, sizeof(int) * n, hipMemcpyDeviceToHost));
-            for (int k = 0; k < n; k++) dst[h->perm[k]] = (double)iv[k];
-            return BRP_OK;
-        }
+        case BRP_BUB_SUB: src = h->b.sub; kind = PackSrc::kPermInt; break;
         default: {
             HIPCHK(h, hipMalloc((void **)&tmpd, sizeof(double) * n));
             launch_bubble_index(h->stream, h->g, h->b, tmpd, which - BRP_BUB_IBM_X);
             src = tmpd;
         }
     }
-    std::vector<double> v(n);
-    hipError_t e = hipMemcpyAsync(v.data(), src, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    const PackSrc p{kind, n, src, nullptr, nullptr, h->iperm_d, 0, 0, 0, 0.0};
+    const hipError_t e = read_back(h->stream, h->device, h->ring, p, 1, dst, n);
     if (tmpd) (void)hipFree(tmpd);
     if (e != hipSuccess) return set_err(h, BRP_ERR_DEVICE, "get_bubbles: %s", hipGetErrorString(e));
-    for (int k = 0; k < n; k++) dst[h->perm[k]] = v[k];
     return BRP_OK;
 }
 

@@ -245,6 +245,34 @@ void launch_bubble_index(hipStream_t s, const GridParams &g, const BubbleArrays 
                          double *out, int which);
 void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots);
 
+// ---- read-back (readback.hip) ----
+// A device array as doubles, row-major with nx columns: a rectangle of a frame
+// from logical column i0 and row j0, or (kPerm, kPermInt) a bubble array in
+// the caller's order.
+struct PackSrc {
+    enum Kind { kFloat, kDouble, kFixed, kDensity, kSum3, kPerm, kPermInt } kind;
+    int64_t nx;
+    const void *src, *src2, *src3;  // src2, src3: kSum3
+    const int *iperm;               // caller index -> sorted bubble
+    int i0, j0, pitch;
+    double scale;                   // kDensity: the liquid's density
+};
+// Pinned memory of a handle's read-backs: `small` (the handle's, small_doubles
+// long) for arrays that it holds, else a ring of slots.
+struct HostRing {
+    static constexpr int64_t kMaxSmall = 1 << 17;
+    double *small = nullptr;
+    int64_t small_doubles = 0;
+    double *host = nullptr;
+    hipEvent_t ev[8] = {};
+    hipError_t reserve();
+    void release();
+};
+// rows x src.nx values into dst (leading dimension ld); returns when they are
+// there.
+hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &src, int64_t rows,
+                     double *dst, int64_t ld);
+
 // ---- temperature (kernels_thermal.hip) ----
 template <typename F>
 void launch_temperature(hipStream_t s, const GridParams &g, const BubbleParams &bp,
