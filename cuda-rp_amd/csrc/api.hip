@@ -872,7 +872,6 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             h->pl_n = p;
             h->pl_p = m;
         }
-        launch_zero_scalars(s, h->sc_d, max_pic + 1);
         StepRecord *rec = ctl ? ctl->rec : nullptr;
         int forced = (ctl && ctl->force_npic) ? ctl->force_npic[step] : -1;
         if (h->sched_mode == 2) {
@@ -902,7 +901,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         HIPCHK(h, hipEventRecord(h->ev[0], s));
         launch_velocity<F>(s, h->g, vx, vy, p0, h->fgb[old_cur], h->W, h->first_step, cxa, cxb,
                            cya, cyb);
-        launch_velocity_ghosts<F>(s, h->g, vx, vy, h->t);
+        launch_velocity_ghosts<F>(s, h->g, vx, vy, h->t, h->sc_d, max_pic + 1);
         HIPCHK(h, hipEventRecord(h->ev[1], s));
         if (bub) launch_motion<F>(s, h->g, h->bp, h->b, vx, vy, h->sc_d);
         HIPCHK(h, hipEventRecord(h->ev[2], s));

@@ -176,7 +176,9 @@ void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *
                      const int64_t *fgn, Window w, int first_step, const F *cvx_a,
                      const F *cvx_b, const F *cvy_a, const F *cvy_b);
 template <typename F>
-void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t);
+// Also clears the step's scalars (resid[0, nslots)).
+void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t,
+                            StepScalars *sc, int nslots);
 template <typename F>
 void launch_pressure_first(hipStream_t s, const GridParams &g, const F *vx, const F *vy,
                            const F *pnx, const F *pny, F *px, F *py, F *p0,

@@ -10,6 +10,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 namespace brp {
 namespace {
 
@@ -154,6 +156,50 @@ __global__ __launch_bounds__(256) void k_velocity(GridParams g, F *__restrict__ 
     }
 }
 
+// The same update for a grid that k_velocity would cover with too few
+// wavefronts (velocity_small): one cell per thread, so that no thread walks rows
+// one after another (256^2 FP64 beside a cloud: 16.3 -> 4.1 us).
+template <typename F>
+__global__ __launch_bounds__(256) void k_velocity_small(GridParams g, F *__restrict__ vx,
+                                                        F *__restrict__ vy,
+                                                        const F *__restrict__ p0,
+                                                        const int64_t *__restrict__ fgn, Window w,
+                                                        int first, const F *__restrict__ cxa,
+                                                        const F *__restrict__ cxb,
+                                                        const F *__restrict__ cya,
+                                                        const F *__restrict__ cyb) {
+    const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
+    if (i > g.N || j > g.M) return;
+    const int64_t o = frame_off(i, j, g.pitch);
+    const F dt = (F)g.dt, rdx = (F)g.rdx, half = (F)0.5;
+    const F dt_rho = dt / (((F)g.rho_inf + (F)g.rho_inf) * half);
+    const bool in_w = !first && j + 1 >= w.j0 && j <= w.j1 && i + 1 >= w.i0 && i <= w.i1;
+    const F pc = p0[o], pe = p0[o + 1], pn = p0[o + g.pitch];
+    const F rc = in_w ? rho_m_at<F>(g, fgn, w, first, i, j) : (F)g.rho_inf;
+    if (j >= 1) {
+        const F s2 = (-pc + pe) * rdx;
+        const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i + 1, j)) * half) : dt_rho;
+        vx[o] = (vx[o] * cxa[i + 1] - q * s2) / cxb[i + 1];
+    }
+    if (i >= 1) {
+        const F s2 = (-pc + pn) * rdx;  // rdx, as the reference (kernel.cuh:671)
+        const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i, j + 1)) * half) : dt_rho;
+        vy[o] = (vy[o] * cya[j + 1] - q * s2) / cyb[j + 1];
+    }
+}
+
+__device__ inline void clear_scalars(StepScalars *sc) {
+    sc->bbox[0] = 0x7fffffff;
+    sc->bbox[1] = -0x7fffffff;
+    sc->bbox[2] = 0x7fffffff;
+    sc->bbox[3] = -0x7fffffff;
+    sc->flags = 0;
+    sc->sub_max = 0;
+    sc->sub_sum = 0ull;
+    sc->done = 0u;
+    sc->reused = 0u;
+}
+
 // Focused source value of row-0 cell i at time t (MixtureBoundaryPressureKernel
 // Focused_P branch, bubble_CUDA_kernel.cuh:905-925, and VelocityBoundaryKernel
 // Focused_V, 763-787).  Extension E4 splits the aperture into n_elem
@@ -180,16 +226,35 @@ __device__ inline double focused_value(const GridParams &g, int i, double t, dou
 }
 
 // VelocityBoundaryKernel (bubble_CUDA_kernel.cuh:680-813) for order 2.  The
-// reference runs its four parts in one racing grid; here one workgroup runs
-// them in program order with a barrier between parts, which is the order
-// warp-mates of the reference observe.
+// reference runs its four parts in one racing grid; the values here are those
+// of the parts run in program order, the order warp-mates of the reference
+// observe, each written as what it comes to in terms of values that no part
+// writes, so that the cells need no order (one workgroup with a barrier
+// between parts took 18 us at 4096^2, this 4.2 us).  Thread k: column
+// i = k - 1 of the ghost rows, and row j = k - 1 of the ghost columns.  Also
+// clears the step's scalars, which the kernels after it use.
 template <typename F>
-__global__ __launch_bounds__(1024) void k_velocity_ghosts(GridParams g, F *vx, F *vy,
-                                                          double t) {
+__global__ __launch_bounds__(256) void k_velocity_ghosts(GridParams g, F *vx, F *vy, double t,
+                                                         StepScalars *sc, int nslots) {
     const int N = g.N, M = g.M, P = g.pitch;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    // VX part a: rows j in [1, M]
-    for (int j = 1 + tid; j <= M; j += nt) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    for (int q = k; q < nslots; q += gridDim.x * 256) sc->resid[q] = 0ull;
+    if (k == 0) clear_scalars(sc);
+    // VX: the mirrors of x0 and x1 (rows 1..M), then rows 0 and M + 1 copy
+    // rows 1 and M as the mirrors left them
+    const auto vx_at = [&](int i, int j) -> F {
+        if (!g.pml_x0 && i == 0) return (F)0;
+        if (!g.pml_x0 && i == -1) return vx[frame_off(1, j, P)];
+        if (!g.pml_x1 && i == N) return (F)0;
+        if (!g.pml_x1 && i == N + 1) return -vx[frame_off(N - 1, j, P)];
+        return vx[frame_off(i, j, P)];
+    };
+    const int i = k - 1, j = k - 1;
+    if (i <= N + 1) {
+        vx[frame_off(i, 0, P)] = vx_at(i, 1);
+        vx[frame_off(i, M + 1, P)] = vx_at(i, M);
+    }
+    if (j >= 1 && j <= M) {
         if (!g.pml_x0) {
             vx[frame_off(-1, j, P)] = vx[frame_off(1, j, P)];
             vx[frame_off(0, j, P)] = (F)0;
@@ -199,18 +264,19 @@ __global__ __launch_bounds__(1024) void k_velocity_ghosts(GridParams g, F *vx, F
             vx[frame_off(N, j, P)] = (F)0;
         }
     }
-    __syncthreads();
-    // VX part b: columns i in [-1, N+1]
-    for (int i = -1 + tid; i <= N + 1; i += nt) {
-        vx[frame_off(i, 0, P)] = vx[frame_off(i, 1, P)];
-        vx[frame_off(i, M + 1, P)] = vx[frame_off(i, M, P)];
-    }
-    __syncthreads();
-    // VY part a: columns i in [1, N]
-    for (int i = 1 + tid; i <= N; i += nt) {
+    // VY: the walls and sources of columns 1..N, then columns 0 and N + 1.
+    // Column 0 copies column 1; its thread writes both, since it has the
+    // values of the rows that the walls write.
+    if (i >= 1 && i <= N) {
+        const auto put = [&](int jj, F v) {
+            vy[frame_off(i, jj, P)] = v;
+            if (i == 1) vy[frame_off(0, jj, P)] = v;
+        };
+        F v0 = vy[frame_off(i, 0, P)], vm1 = vy[frame_off(i, -1, P)];
+        F vM = vy[frame_off(i, M, P)], vM1 = vy[frame_off(i, M + 1, P)];
         if (!g.pml_y0) {
-            if (!g.plane_p && !g.focused_p) vy[frame_off(i, 0, P)] = (F)0;
-            vy[frame_off(i, -1, P)] = vy[frame_off(i, 0, P)];
+            if (!g.plane_p && !g.focused_p) v0 = (F)0;
+            vm1 = v0;
         }
         if (g.src_row) {
             if (g.plane_v) {
@@ -218,26 +284,31 @@ __global__ __launch_bounds__(1024) void k_velocity_ghosts(GridParams g, F *vx, F
                 if (fmod(t, ((double)g.on_wave + (double)g.off_wave) / g.freq) <=
                     ((double)g.on_wave) / g.freq)
                     v = g.amp * sin(g.omega * t);
-                vy[frame_off(i, 0, P)] = (F)v;
+                v0 = (F)v;
             }
-            if (g.focused_v)
-                vy[frame_off(i, 0, P)] = (F)focused_value(g, i, t, g.amp, 0.0, nullptr, nullptr);
+            if (g.focused_v) v0 = (F)focused_value(g, i, t, g.amp, 0.0, nullptr, nullptr);
         }
         if (!g.pml_y1) {
-            vy[frame_off(i, M, P)] = (F)0;
-            vy[frame_off(i, M + 1, P)] = vy[frame_off(i, M - 1, P)];
+            vM = (F)0;
+            vM1 = vy[frame_off(i, M - 1, P)];
         }
+        put(-1, vm1);
+        put(0, v0);
+        put(M, vM);
+        put(M + 1, vM1);
     }
-    __syncthreads();
-    // VY part b: rows j in [-1, M+1].  The right ghost column copies
-    // vy(N, jsta2n + N + 1) = vy(N, N) in every row: the reference reads row
-    // vy_width*i with the loop variable i (bubble_CUDA_kernel.cuh:808).
-    const int qj = N;  // logical row jsta2n + (N + 1)
-    const bool q_in = qj <= M + 1;
-    F q = q_in ? vy[frame_off(N, qj, P)] : (F)0;
-    __syncthreads();
-    for (int j = -1 + tid; j <= M + 1; j += nt) {
-        vy[frame_off(0, j, P)] = vy[frame_off(1, j, P)];
+    if (j <= M + 1) {
+        if (j >= 1 && j <= M - 1) vy[frame_off(0, j, P)] = vy[frame_off(1, j, P)];
+        // The right ghost column copies vy(N, jsta2n + N + 1) = vy(N, N) in
+        // every row: the reference reads row vy_width*i with the loop variable
+        // i (bubble_CUDA_kernel.cuh:808).
+        F q = (F)0;
+        if (N == M && !g.pml_y1)
+            q = (F)0;
+        else if (N == M + 1 && !g.pml_y1)
+            q = vy[frame_off(N, M - 1, P)];
+        else if (N <= M + 1)
+            q = vy[frame_off(N, N, P)];
         vy[frame_off(N + 1, j, P)] = q;
     }
 }
@@ -355,6 +426,54 @@ __global__ __launch_bounds__(256) void k_pressure_first(
                 }
             }
             vyl = vyc;
+        }
+    }
+    if (bad) atomicOr(&sc->flags, 1);
+    block_max_to(rmax, &sc->resid[0]);
+}
+
+// The same evaluation for a small grid (pressure_small), one cell per
+// thread (256^2 FP64 beside a cloud 16.4 -> 8.1 us).
+template <typename F>
+__global__ __launch_bounds__(256) void k_pressure_first_small(
+    GridParams g, const F *__restrict__ vx, const F *__restrict__ vy, const F *__restrict__ pnx,
+    const F *__restrict__ pny, F *__restrict__ px, F *__restrict__ py, F *__restrict__ p0,
+    const int64_t *__restrict__ fg_cur, const int64_t *__restrict__ fg_n,
+    int64_t *__restrict__ fg_mp, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
+    const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
+    const double *__restrict__ rxp, StepScalars *sc) {
+    const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
+    double rmax = 0.0;
+    bool bad = false;
+    if (i <= g.N + 1 && j <= g.M + 1) {
+        const int64_t o = frame_off(i, j, g.pitch);
+        int64_t fpred = 0, fold = 0;
+        if (i >= w.i0 && i <= w.i1 && j >= w.j0 && j <= w.j1) {
+            fold = fg_cur[o];
+            fpred = 3 * fold - 3 * fg_n[o] + fg_mp[o];
+            fg_mp[o] = fpred;
+        }
+        if (i >= 1 && i <= g.N && j >= 1 && j <= g.M) {
+            const F s3 = (F)g.s3, rdx = (F)g.rdx, rdy = (F)g.rdy;
+            F s5h = (F)(-0.0);
+            if (fpred != 0 || fold != 0) {
+                const double s5d = -fg_to_d(fpred - fold) / g.dt / (1.0 - 0.5 * fg_to_d(fpred + fold));
+                s5h = (F)(0.5 * s5d);
+            }
+            F s1x;
+            if (g.cylindrical)
+                s1x = (F)((-xu[i] * (double)vx[o - 1] + xu[i + 1] * (double)vx[o]) * g.rdx * rxp[i + 1]);
+            else
+                s1x = (-vx[o - 1] + vx[o]) * rdx;
+            const F s1y = (-vy[o - g.pitch] + vy[o]) * rdy;
+            const F npx = pnx[o] * ax[i + 1] - s3 * (s1x + s5h) / bx[i + 1];
+            const F npy = pny[o] * ay[j + 1] - s3 * (s1y + s5h) / by[j + 1];
+            const F np0 = npx + npy;
+            px[o] = npx;
+            py[o] = npy;
+            rmax = fabs((double)p0[o] - (double)np0);
+            bad = !isfinite((double)np0) || fabs(fg_to_d(fpred)) >= 1.0;
+            p0[o] = np0;
         }
     }
     if (bad) atomicOr(&sc->flags, 1);
@@ -500,25 +619,31 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
 __global__ void k_zero_scalars(StepScalars *sc, int nslots) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < nslots) sc->resid[t] = 0ull;
-    if (t == 0) {
-        sc->bbox[0] = 0x7fffffff;
-        sc->bbox[1] = -0x7fffffff;
-        sc->bbox[2] = 0x7fffffff;
-        sc->bbox[3] = -0x7fffffff;
-        sc->flags = 0;
-        sc->sub_max = 0;
-        sc->sub_sum = 0ull;
-        sc->done = 0u;
-        sc->reused = 0u;
-    }
+    if (t == 0) clear_scalars(sc);
 }
 
 }  // namespace
+
+// Where one cell per thread is the better split: the four-cell, four-row
+// threads are fewer than a wavefront per SIMD (1024 on 256 compute units)
+// below a million cells, but they load each pressure row and velocity once.
+// With the ghost launch after it, us, four-row against one-cell threads:
+// velocity 256^2 15.4 / 12.9, 777^2 16.8 / 16.6 (FP32 15.3 / 13.2), 1400^2
+// 22.4 / 22.3, 2048^2 FP32 22.8 / 25.8; pressure 256^2 17.0 / 11.5, 400^2 16.4
+// / 14.1, 600^2 17.7 / 19.1, 1000^2 20.2 / 22.7.
+static bool velocity_small(const GridParams &g) { return (int64_t)g.N * g.M < (1 << 20); }
+static bool pressure_small(const GridParams &g) { return (int64_t)g.N * g.M < 300000; }
 
 template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
                      const int64_t *fgn, Window w, int first_step, const F *cxa, const F *cxb,
                      const F *cya, const F *cyb) {
+    if (velocity_small(g)) {
+        hipLaunchKernelGGL(k_velocity_small<F>, dim3((g.N + kBX) / kBX, (g.M + kBY) / kBY),
+                           dim3(kBX, kBY), 0, s, g, vx, vy, p0, fgn, w, first_step, cxa, cxb, cya,
+                           cyb);
+        return;
+    }
     dim3 blk(kBX, kBY);  // columns 0..N, rows 0..M
     dim3 grd((g.N + 1 + kBX * kGW - 1) / (kBX * kGW), (g.M + 1 + kGBlockRows - 1) / kGBlockRows);
     hipLaunchKernelGGL(k_velocity<F>, grd, blk, 0, s, g, vx, vy, p0, fgn, w, first_step, cxa,
@@ -526,8 +651,11 @@ void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *
 }
 
 template <typename F>
-void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t) {
-    hipLaunchKernelGGL(k_velocity_ghosts<F>, dim3(1), dim3(1024), 0, s, g, vx, vy, t);
+void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t,
+                            StepScalars *sc, int nslots) {
+    const int n = std::max(g.N, g.M) + 3;  // columns and rows -1 .. N + 1, M + 1
+    hipLaunchKernelGGL(k_velocity_ghosts<F>, dim3((n + 255) / 256), dim3(256), 0, s, g, vx, vy, t,
+                       sc, nslots);
 }
 
 template <typename F>
@@ -536,6 +664,13 @@ void launch_pressure_first(hipStream_t s, const GridParams &g, const F *vx, cons
                            const int64_t *fg_cur, const int64_t *fg_n, int64_t *fg_mp, Window w,
                            const F *ax, const F *bx, const F *ay, const F *by, const double *xu,
                            const double *rxp, StepScalars *sc) {
+    if (pressure_small(g)) {
+        hipLaunchKernelGGL(k_pressure_first_small<F>,
+                           dim3((g.N + 1 + kBX) / kBX, (g.M + 1 + kBY) / kBY), dim3(kBX, kBY), 0, s,
+                           g, vx, vy, pnx, pny, px, py, p0, fg_cur, fg_n, fg_mp, w, ax, bx, ay, by,
+                           xu, rxp, sc);
+        return;
+    }
     dim3 blk(kBX, kBY);  // columns 0..N+1, rows 0..M+1
     dim3 grd((g.N + 2 + kBX * kGW - 1) / (kBX * kGW), (g.M + 2 + kGBlockRows - 1) / kGBlockRows);
     hipLaunchKernelGGL(k_pressure_first<F>, grd, blk, 0, s, g, vx, vy, pnx, pny, px, py, p0,
@@ -572,7 +707,7 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
                                      const int64_t *, Window, int, const F *, const F *,     \
                                      const F *, const F *);                                  \
     template void launch_velocity_ghosts<F>(hipStream_t, const GridParams &, F *, F *,      \
-                                            double);                                         \
+                                            double, StepScalars *, int);                     \
     template void launch_pressure_first<F>(                                                  \
         hipStream_t, const GridParams &, const F *, const F *, const F *, const F *, F *,   \
         F *, F *, const int64_t *, const int64_t *, int64_t *, Window, const F *, const F *, \
