@@ -237,7 +237,9 @@ struct brp_handle {
     std::vector<double> pending_x, pending_y, pending_R0, pending_nB;  // host-side set-up
 
     StepScalars *sc_d = nullptr;
-    StepScalars *sc_h = nullptr;
+    StepReport *rep = nullptr;         // pinned: what a step's kernels tell the host
+    unsigned long long rep_seq = 0;    // reports asked for so far
+    double ms_per_tick = 1e-5;         // of the device's constant-rate clock
     RPLaunch *rpl_h = nullptr, *rpl_d = nullptr;  // the RP kernel's fixed parameters
     Window W{1, 0, 1, 0};
     int first_step = 1;
@@ -246,7 +248,6 @@ struct brp_handle {
     bool prepared = false;
 
     hipStream_t stream = nullptr;
-    std::vector<hipEvent_t> ev;
     double phase_ms[5] = {0, 0, 0, 0, 0};
 
     std::vector<void *> allocs;
@@ -811,6 +812,23 @@ void rec_free(StepRecord &r) {
 }
 
 // ---- the coupled step ----------------------------------------------------
+// Waits for the last report asked for.  The kernel that writes it is the last
+// one queued, so the spin ends when the stream does; a stream that ends
+// without it has failed.
+int wait_report(brp_handle *h) {
+    for (int spin = 0;; spin++) {
+        if (__atomic_load_n(&h->rep->seq, __ATOMIC_ACQUIRE) == h->rep_seq) return BRP_OK;
+        if (spin < 256) continue;
+        spin = 0;
+        const hipError_t e = hipStreamQuery(h->stream);
+        if (e == hipErrorNotReady) continue;
+        HIPCHK(h, e);
+        if (__atomic_load_n(&h->rep->seq, __ATOMIC_ACQUIRE) == h->rep_seq) return BRP_OK;
+        HIPCHK(h, hipGetLastError());
+        return set_err(h, BRP_ERR_DEVICE, "a step's report did not arrive");
+    }
+}
+
 int rec_grow(brp_handle *h, StepRecord *r, int k);
 
 // Frozen-schedule recording of the RP launch just queued: its per-bubble
@@ -845,7 +863,6 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
     const int max_pic = std::min(h->cfg.max_picard > 0 ? h->cfg.max_picard : 1000, kMaxEval - 1);
     const bool bub = h->cfg.bub_enable && h->nb > 0;
     hipStream_t s = h->stream;
-    const size_t hdr = offsetof(StepScalars, resid);
     if (bub) {  // the RP kernel's parameters as of this call (no step is in flight)
         *h->rpl_h = RPLaunch{h->g, h->bp, h->b};
         HIPCHK(h, hipMemcpyAsync(h->rpl_d, h->rpl_h, sizeof(RPLaunch), hipMemcpyHostToDevice, s));
@@ -898,28 +915,22 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             rec->first = h->first_step;
             rec->t = h->t;
         }
-        HIPCHK(h, hipEventRecord(h->ev[0], s));
         launch_velocity<F>(s, h->g, vx, vy, p0, h->fgb[old_cur], h->W, h->first_step, cxa, cxb,
-                           cya, cyb);
+                           cya, cyb, h->sc_d);
         launch_velocity_ghosts<F>(s, h->g, vx, vy, h->t, h->sc_d, max_pic + 1);
-        HIPCHK(h, hipEventRecord(h->ev[1], s));
         if (bub) launch_motion<F>(s, h->g, h->bp, h->b, vx, vy, h->sc_d);
-        HIPCHK(h, hipEventRecord(h->ev[2], s));
         launch_pressure_first<F>(s, h->g, vx, vy, (F *)h->pb[pn_i][0], (F *)h->pb[pn_i][1],
                                  (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0, h->fgb[old_cur],
                                  h->fgb[old_n], h->fgb[old_m], h->W, ax, bx, ay, by, h->xu_d,
                                  h->rxp_d, h->sc_d);
-        launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, nullptr, 0,
-                                  h->sc_d);
-        HIPCHK(h, hipEventRecord(h->ev[3], s));
-        HIPCHK(h, hipMemcpyAsync(h->sc_h, h->sc_d, hdr + sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipStreamSynchronize(s));
-        double r0;
-        std::memcpy(&r0, &h->sc_h->resid[0], 8);
-        double resimax = r0 / h->P_inf;
+        launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, 0, nullptr, 0,
+                                  h->b.bbox_blk, bub ? (h->nb + 255) / 256 : 0, h->sc_d, h->rep,
+                                  ++h->rep_seq);
+        if (int rc = wait_report(h)) return rc;
+        double resimax = h->rep->resid / h->P_inf;
         st.resimax0 = resimax;
         if (bub) {
-            window_union(h->W, h->sc_h->bbox[0], h->sc_h->bbox[1], h->sc_h->bbox[2], h->sc_h->bbox[3]);
+            window_union(h->W, h->rep->bbox[0], h->rep->bbox[1], h->rep->bbox[2], h->rep->bbox[3]);
             if (h->cfg.tr_cylindrical && h->W.i0 <= 1 && h->W.i0 <= h->W.i1) h->W.i0 = 0;  // axis fold target
         }
         if (rec && rec->want_grid) {  // the window is final for this step
@@ -934,7 +945,6 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         long long lost = 0;  // bubbles the RP kernel did not write back
         int loop = 0;
         int target = h->fz, prev = old_m;
-        double bub_ms = 0.0, pic_p_ms = 0.0, other_ms = 0.0;
         if (bub) {
             while (forced >= 0 ? loop < forced : resimax > thr) {
                 if (loop >= max_pic) {
@@ -946,7 +956,6 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     int rc = rec_grow(h, rec, loop + 1);
                     if (rc) return rc;
                 }
-                HIPCHK(h, hipEventRecord(h->ev[7], s));
                 const StepRecord *tin = ctl ? ctl->tape_in : nullptr;
                 const bool replay = h->sched_mode == 2;
                 if (!tin && !replay && !bubble_step_unordered(*h->rpl_h, h->cus)) {
@@ -956,11 +965,10 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     // previous iteration's counts, bubbles whose gathered
                     // pressure did not change last
                     launch_queue_keys<F>(s, h->g, h->bp, h->b, p0, h->rp_cur, h->pl_p, loop,
-                                         h->bp.extreme_threshold);
+                                         h->bp.extreme_threshold, h->sc_d);
                     launch_order_partition(s, h->b, h->b.key, h->bp.heavy_threshold,
                                            h->bp.extreme_threshold);
                 }
-                HIPCHK(h, hipEventRecord(h->ev[4], s));
                 int rp_waves = 0;  // wavefront records the launch leaves
                 if (tin) {  // replay: the void fraction from the taped radii, no RP
                     launch_scatter_radii(s, h->g, h->bp, h->b, tin->Rt_it[loop], h->fgb[target], h->sc_d);
@@ -993,42 +1001,29 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     HIPCHK(h, hipMemcpyAsync(rec->Rt_it[loop], h->b.R_t, sizeof(double) * h->nb, hipMemcpyDeviceToDevice, s));
                     HIPCHK(h, hipMemcpyAsync(rec->sub_it[loop], h->b.sub, sizeof(int) * h->nb, hipMemcpyDeviceToDevice, s));
                 }
-                HIPCHK(h, hipEventRecord(h->ev[5], s));
                 launch_pressure_picard<F>(s, h->g, vx, vy, (F *)h->pb[pn_i][0], (F *)h->pb[pn_i][1],
                                           (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0,
                                           h->fgb[target], h->fgb[old_cur], h->fgb[prev], h->W, ax,
                                           bx, ay, by, h->xu_d, h->rxp_d, h->sc_d, loop);
-                launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, h->b.totals,
-                                          rp_waves, h->sc_d);
+                launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
+                                          h->b.totals, rp_waves, nullptr, 0, h->sc_d, h->rep,
+                                          ++h->rep_seq);
                 if (rec && rec->want_grid) {
                     int rc = copy_rect(h, rec->p0_it[loop], p0, sizeof(F), rec->rect);
                     if (rc) return rc;
                 }
-                HIPCHK(h, hipEventRecord(h->ev[6], s));
-                HIPCHK(h, hipMemcpyAsync(h->sc_h, h->sc_d, hdr, hipMemcpyDeviceToHost, s));
-                HIPCHK(h, hipMemcpyAsync(&h->sc_h->resid[loop], &h->sc_d->resid[loop], 8,
-                                         hipMemcpyDeviceToHost, s));
-                HIPCHK(h, hipStreamSynchronize(s));
-                double r;
-                std::memcpy(&r, &h->sc_h->resid[loop], 8);
-                resimax = r / h->P_inf;
-                h->last_sub_max = h->sc_h->sub_max;
-                h->last_sub_per_launch = (double)h->sc_h->sub_sum / loop;
+                if (int rc = wait_report(h)) return rc;
+                resimax = h->rep->resid / h->P_inf;
+                h->last_sub_max = h->rep->sub_max;
+                h->last_sub_per_launch = (double)h->rep->sub_sum / loop;
                 // every bubble is written back exactly once per RP launch
-                if (!tin && h->sc_h->done != (unsigned)h->nb * (unsigned)loop) {
+                if (!tin && h->rep->done != (unsigned)h->nb * (unsigned)loop) {
                     status = BRP_ERR_STATE;
-                    lost = (long long)h->nb * loop - (long long)h->sc_h->done;
+                    lost = (long long)h->nb * loop - (long long)h->rep->done;
                     break;
                 }
                 std::swap(target, prev);
-                float a = 0.f, c = 0.f, o = 0.f;
-                (void)hipEventElapsedTime(&o, h->ev[7], h->ev[4]);
-                (void)hipEventElapsedTime(&a, h->ev[4], h->ev[5]);
-                (void)hipEventElapsedTime(&c, h->ev[5], h->ev[6]);
-                other_ms += o;
-                bub_ms += a;
-                pic_p_ms += c;
-                if (h->sc_h->flags & 4) {
+                if (h->rep->flags & 4) {
                     status = BRP_ERR_SUBSTEP_CAP;
                     break;
                 }
@@ -1037,15 +1032,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         // calculate_temperature (bubble_CUDA.cu:279-282): the final f_g and p,
         // the previous step's properties
         if (h->cfg.thermal) {
-            HIPCHK(h, hipEventRecord(h->ev[7], s));
             launch_temperature<F>(s, h->g, h->bp, h->b, bub, h->W, h->T_inf, h->T_d, h->dT_d,
                                   h->heat_d, h->fgb[prev], h->fgb[old_cur], h->first_step,
                                   (const F *)h->pb[p_i][0], (const F *)h->pb[p_i][1],
-                                  (const F *)h->pb[pn_i][0], (const F *)h->pb[pn_i][1]);
-            launch_focal_point(s, h->g, h->dT_d, h->heat_d, h->sc_d);
-            HIPCHK(h, hipMemcpyAsync(h->sc_h->focal, h->sc_d->focal, sizeof(double) * 2,
-                                     hipMemcpyDeviceToHost, s));
-            HIPCHK(h, hipEventRecord(h->ev[4], s));
+                                  (const F *)h->pb[pn_i][0], (const F *)h->pb[pn_i][1], h->sc_d);
+            launch_focal_point(s, h->g, h->dT_d, h->heat_d, h->sc_d, h->rep, ++h->rep_seq);
         }
         // rotate the void-fraction buffers: final iterate in `prev`, zero buffer in `target`
         h->fcur = prev;
@@ -1056,25 +1047,10 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         if (bub && loop == 0) launch_copy_d(s, h->b.PL[h->pl_p], h->b.PL[h->pl_n], h->nb);
         h->pc = p_i;
         h->first_step = 0;
-        if (!bub) HIPCHK(h, hipMemcpyAsync(h->sc_h, h->sc_d, hdr, hipMemcpyDeviceToHost, s));
-        HIPCHK(h, hipStreamSynchronize(s));
-        {
-            float a = 0.f, b2 = 0.f, c = 0.f;
-            (void)hipEventElapsedTime(&a, h->ev[0], h->ev[1]);
-            (void)hipEventElapsedTime(&b2, h->ev[1], h->ev[2]);
-            (void)hipEventElapsedTime(&c, h->ev[2], h->ev[3]);
-            h->phase_ms[0] += a;
-            h->phase_ms[1] += b2;
-            h->phase_ms[2] += c + pic_p_ms;
-            h->phase_ms[3] += bub_ms;
-            if (h->cfg.thermal) {
-                float th = 0.f;
-                (void)hipEventElapsedTime(&th, h->ev[7], h->ev[4]);
-                other_ms += th;
-            }
-            h->phase_ms[4] += other_ms;
-        }
-        const int flags = h->sc_h->flags;
+        if (h->cfg.thermal)
+            if (int rc = wait_report(h)) return rc;
+        for (int q = 0; q < 5; q++) h->phase_ms[q] += (double)h->rep->phase[q] * h->ms_per_tick;
+        const int flags = h->rep->flags;
         if (status == BRP_OK && (flags & 3)) status = BRP_ERR_NONFINITE;
         if (status == BRP_OK && (flags & 4)) status = BRP_ERR_SUBSTEP_CAP;
         st.nstep = h->nstep;
@@ -1082,8 +1058,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         st.resimax = resimax;
         st.n_pic = loop;
         if (h->cfg.thermal) {
-            st.focal_x = h->sc_h->focal[0];
-            st.focal_y = h->sc_h->focal[1];
+            st.focal_x = h->rep->focal[0];
+            st.focal_y = h->rep->focal[1];
         }
         if (rec) {
             rec->n_pic = loop;
@@ -1105,10 +1081,10 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             HIPCHK(h, hipMemcpy(&mm, h->sched->mismatch, sizeof mm, hipMemcpyDeviceToHost));
             if (mm) status = BRP_ERR_STATE;
         }
-        st.rp_max_substeps = h->sc_h->sub_max;
-        st.rp_reused = h->sc_h->reused;
+        st.rp_max_substeps = h->rep->sub_max;
+        st.rp_reused = h->rep->reused;
         st.rp_mean_substeps = (loop > 0 && h->nb > 0)
-                                  ? (double)h->sc_h->sub_sum / ((double)h->nb * loop)
+                                  ? (double)h->rep->sub_sum / ((double)h->nb * loop)
                                   : 0.0;
         st.status = status;
         if (stats) stats[step] = st;
@@ -1542,9 +1518,9 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
     }
     if (hipStreamCreate(&h->stream) != hipSuccess)
         return fail(set_err(h, BRP_ERR_DEVICE, "hipStreamCreate failed"));
-    h->ev.resize(8);
-    for (auto &e : h->ev)
-        if (hipEventCreate(&e) != hipSuccess) return fail(set_err(h, BRP_ERR_DEVICE, "hipEventCreate failed"));
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device) == hipSuccess && khz > 0)
+        h->ms_per_tick = 1.0 / khz;
 
     // init_grid_size (bubble_CUDA.cu:524-540)
     GridParams &g = h->g;
@@ -1645,14 +1621,15 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
             return fail(set_err(h, BRP_ERR_DEVICE, "hipMemcpy failed"));
         bp.rp_shared = tab;
     }
-    // the host's copy of the step scalars and, behind it, the small read-back slot
-    const size_t sc_bytes = (sizeof(StepScalars) + 255) & ~size_t(255);
+    // the step reports and, behind them, the small read-back slot
+    const size_t rep_bytes = (sizeof(StepReport) + 255) & ~size_t(255);
     h->ring.small_doubles = std::min<int64_t>(HostRing::kMaxSmall, (int64_t)(h->N + 3) * (h->M + 3));
-    if (hipHostMalloc((void **)&h->sc_h, sc_bytes + sizeof(double) * h->ring.small_doubles,
+    if (hipHostMalloc((void **)&h->rep, rep_bytes + sizeof(double) * h->ring.small_doubles,
                       hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&h->rpl_h, sizeof(RPLaunch), hipHostMallocDefault) != hipSuccess)
         return fail(set_err(h, BRP_ERR_DEVICE, "hipHostMalloc failed"));
-    h->ring.small = (double *)((char *)h->sc_h + sc_bytes);
+    std::memset(h->rep, 0, sizeof(StepReport));
+    h->ring.small = (double *)((char *)h->rep + rep_bytes);
     if ((rc = dalloc(h, (void **)&h->rpl_d, sizeof(RPLaunch)))) return fail(rc);
     // init_bub_array (bubble_CUDA.cu:797-897): one bubble per cell centre in the box
     if (c.bub_enable) {
@@ -1683,10 +1660,8 @@ void brp_destroy(brp_handle *h) {
         for (void *p : sn.bufs) (void)hipFree(p);
     for (void *p : h->allocs) (void)hipFree(p);
     h->ring.release();
-    if (h->sc_h) (void)hipHostFree(h->sc_h);
+    if (h->rep) (void)hipHostFree(h->rep);
     if (h->rpl_h) (void)hipHostFree(h->rpl_h);
-    for (auto &e : h->ev)
-        if (e) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
@@ -1775,9 +1750,10 @@ int brp_prepare(brp_handle *h) {
         if (h->cfg.tr_cylindrical) launch_cyl_fold(h->stream, h->g, h->fgb[0]);
         HIPCHK(h, hipMemcpyAsync(h->fgb[1], h->fgb[0], sizeof(int64_t) * h->frame, hipMemcpyDeviceToDevice, h->stream));
         HIPCHK(h, hipMemcpyAsync(h->fgb[2], h->fgb[0], sizeof(int64_t) * h->frame, hipMemcpyDeviceToDevice, h->stream));
-        HIPCHK(h, hipMemcpyAsync(h->sc_h, h->sc_d, offsetof(StepScalars, resid), hipMemcpyDeviceToHost, h->stream));
+        int flags = 0;
+        HIPCHK(h, hipMemcpyAsync(&flags, &h->sc_d->flags, sizeof flags, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
-        if (h->sc_h->flags) return set_err(h, BRP_ERR_NONFINITE, "initial void fraction out of range");
+        if (flags) return set_err(h, BRP_ERR_NONFINITE, "initial void fraction out of range");
     }
     h->fcur = 0;
     h->fn = 1;
@@ -1792,7 +1768,11 @@ int brp_step(brp_handle *h, int32_t k, brp_step_stats *stats) {
     int rc = brp_prepare(h);
     if (rc) return rc;
     for (double &v : h->phase_ms) v = 0.0;
-    return h->prec == BRP_PREC_FP64 ? run_steps<double>(h, k, stats) : run_steps<float>(h, k, stats);
+    rc = h->prec == BRP_PREC_FP64 ? run_steps<double>(h, k, stats) : run_steps<float>(h, k, stats);
+    // run_steps waits for reports, which the last kernels write before they end
+    const hipError_t e = hipStreamSynchronize(h->stream);
+    if (rc == BRP_OK) HIPCHK(h, e);
+    return rc;
 }
 
 int brp_field_shape(const brp_handle *h, int32_t field, int32_t *nx, int32_t *ny, int32_t *i0,

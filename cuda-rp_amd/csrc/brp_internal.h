@@ -76,7 +76,26 @@ struct RPTotals {
 // head q hands out the batches q, q + kQueueHeads, ... of the queue order.
 constexpr int kQueueHeads = 16, kHeadStride = 32;
 
-// Device-side per-step scalars written by the kernels and read by the host.
+// Where the phases of a step begin: the velocity update, the bubble motion,
+// the first pressure evaluation; in a Picard iteration the queue, the RP
+// launch and the pressure evaluation; the temperature solve.
+enum Mark { kMarkVelocity, kMarkMotion, kMarkPressure, kMarkQueue, kMarkRP, kMarkPicard,
+            kMarkThermal, kMarks };
+
+// What the host reads after an evaluation: k_pressure_ghosts, the
+// evaluation's last kernel, writes it into pinned host memory, seq last.
+struct StepReport {
+    double resid;                // of this evaluation (Pa)
+    int bbox[4];
+    int flags, sub_max;
+    unsigned long long sub_sum;
+    unsigned int done, reused;
+    unsigned long long phase[5];
+    double focal[2];
+    unsigned long long seq;
+};
+
+// Device-side per-step scalars written by the kernels.
 struct StepScalars {
     int bbox[4];                         // min i, max i, min j, max j of bubble stencils
     int flags;                           // bit 0 nonfinite p / f_g >= 1, bit 1 scatter
@@ -86,10 +105,28 @@ struct StepScalars {
     unsigned int done;                   // bubbles written back by the RP kernel this step
     unsigned int reused;                 // of them, kept from the previous iteration
     double focal[2];                     // (x, y) of the largest temperature increment
+    // The step's phases in ticks of the device's constant-rate clock: marks
+    // that kernels set, and the phases' sums (brp_get_phase_times' order).
+    unsigned long long mark[kMarks], phase[5];
     unsigned long long resid[kMaxEval];  // max |dp0| bit patterns (>= 0 doubles)
     double focal_v[256];                 // per-block maxima of the focal-point search
     int focal_i[256];
 };
+
+#if defined(__HIPCC__)
+// Sets a phase's mark (the kernel's first workgroup, one thread).  The store
+// is written out so that the compiler does not take it for one that may
+// change what the kernel reads through its other pointers: after it, uniform
+// reads would no longer be scalar loads.
+__device__ inline void set_mark(StepScalars *sc, Mark m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
+        const unsigned long long now = wall_clock64();
+        asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(&sc->mark[m]), "v"(now));
+    }
+#endif
+}
+#endif
 
 // Bubble arrays (device pointers; n padded to a multiple of 256).
 struct BubbleArrays {
@@ -174,7 +211,7 @@ namespace brp {
 template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
                      const int64_t *fgn, Window w, int first_step, const F *cvx_a,
-                     const F *cvx_b, const F *cvy_a, const F *cvy_b);
+                     const F *cvx_b, const F *cvy_a, const F *cvy_b, StepScalars *sc);
 template <typename F>
 // Also clears the step's scalars (resid[0, nslots)).
 void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t,
@@ -193,8 +230,9 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
                             const double *xu, const double *rxp, StepScalars *sc, int slot);
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
-                            const double *el_phase, double t, const RPTotals *tot, int n_tot,
-                            StepScalars *sc);
+                            const double *el_phase, double t, int eval, const RPTotals *tot,
+                            int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
+                            StepReport *rep, unsigned long long seq);
 template <typename F>
 void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                    const BubbleArrays &b, const F *vx, const F *vy, StepScalars *sc);
@@ -222,7 +260,8 @@ bool bubble_step_lean(int sub_max, double sub_per_launch, int extreme_threshold,
 // results stand).
 template <typename F>
 void launch_queue_keys(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                       const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext);
+                       const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext,
+                       StepScalars *sc);
 void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key, int threshold,
                             int ext);
 void launch_scatter_initial(hipStream_t s, const GridParams &g, const BubbleParams &bp,
@@ -280,10 +319,11 @@ template <typename F>
 void launch_temperature(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                         const BubbleArrays &b, bool bubbles, Window w, double T_inf, double *T,
                         double *dT, double *heat, const int64_t *fg, const int64_t *fgn,
-                        int first, const F *px, const F *py, const F *pnx, const F *pny);
+                        int first, const F *px, const F *py, const F *pnx, const F *pny,
+                        StepScalars *sc);
 
 void launch_focal_point(hipStream_t s, const GridParams &g, const double *dT, const double *heat,
-                        StepScalars *sc);
+                        StepScalars *sc, StepReport *rep, unsigned long long seq);
 
 // ---- adjoint (kernels_adjoint.hip) ----
 // Adjoint fields, FP64, same frame as the forward fields.

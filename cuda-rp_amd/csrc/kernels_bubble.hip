@@ -34,7 +34,7 @@ __device__ inline int64_t to_fixed(double v, bool *bad) {
 }
 
 // Block-wide reduction of (min, max) pairs into this block's slot of out
-// (4 ints); k_bbox_reduce folds the slots into sc->bbox.  One plain store per
+// (4 ints); k_pressure_ghosts folds the slots into sc->bbox.  One plain store per
 // block instead of device-scope atomics on four shared addresses, which
 // serialise across the whole grid.
 __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *out) {
@@ -68,37 +68,6 @@ __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *o
     }
 }
 
-__global__ __launch_bounds__(256) void k_bbox_reduce(const int *blk, int nblk, StepScalars *sc) {
-    int imin = 0x7fffffff, imax = -0x7fffffff, jmin = 0x7fffffff, jmax = -0x7fffffff;
-    for (int k = threadIdx.x; k < nblk; k += blockDim.x) {
-        imin = min(imin, blk[4 * k + 0]);
-        imax = max(imax, blk[4 * k + 1]);
-        jmin = min(jmin, blk[4 * k + 2]);
-        jmax = max(jmax, blk[4 * k + 3]);
-    }
-    __shared__ int red[4][256];
-    red[0][threadIdx.x] = imin;
-    red[1][threadIdx.x] = imax;
-    red[2][threadIdx.x] = jmin;
-    red[3][threadIdx.x] = jmax;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            red[0][threadIdx.x] = min(red[0][threadIdx.x], red[0][threadIdx.x + s]);
-            red[1][threadIdx.x] = max(red[1][threadIdx.x], red[1][threadIdx.x + s]);
-            red[2][threadIdx.x] = min(red[2][threadIdx.x], red[2][threadIdx.x + s]);
-            red[3][threadIdx.x] = max(red[3][threadIdx.x], red[3][threadIdx.x + s]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && red[0][0] <= red[1][0]) {
-        sc->bbox[0] = red[0][0];
-        sc->bbox[1] = red[1][0];
-        sc->bbox[2] = red[2][0];
-        sc->bbox[3] = red[3][0];
-    }
-}
-
 // BubbleInterpolationVelocityKernel + v_B <- v_L + BubbleMotionKernel
 // (bubble_CUDA_kernel.cuh:398-468, 1282-1297), fused per bubble; also the
 // bounding box of the new scatter stencils for the Picard window.
@@ -106,6 +75,7 @@ template <typename F>
 __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, BubbleArrays b,
                                                  const F *__restrict__ vx,
                                                  const F *__restrict__ vy, StepScalars *sc) {
+    set_mark(sc, kMarkMotion);
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     int imin = 0x7fffffff, imax = -0x7fffffff, jmin = 0x7fffffff, jmax = -0x7fffffff;
     if (idx < b.n) {
@@ -384,7 +354,9 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
                                                             const double *rp_shared, int cur,
                                                             int plm, int pln, int plp,
                                                             int64_t *__restrict__ fg_target,
-                                                            int quota, int solo_cap) {
+                                                            StepScalars *sc, int quota,
+                                                            int solo_cap) {
+    set_mark(sc, kMarkRP);
     const int lane = threadIdx.x & 63;
     const int nxt = cur ^ 1;
     __shared__ WaveAgg agg_all[4];  // 25 KB: one table per wavefront
@@ -612,6 +584,7 @@ __global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int ma
                                                       int64_t *__restrict__ fg_target,
                                                       StepScalars *sc, int slot, int quota,
                                                       int solo_cap) {
+    set_mark(sc, kMarkRP);
     const int lane = threadIdx.x & 63;
     const bool odd = lane & 1;
     const int nxt = cur ^ 1;
@@ -813,6 +786,7 @@ __global__ __launch_bounds__(256) void k_rp_replay(const RPLaunch *kp, int cur, 
                                                     int64_t *__restrict__ fg_target,
                                                     StepScalars *sc, const int64_t *off,
                                                     const double *dts) {
+    const unsigned long long began = wall_clock64();
     const RPLaunch &P = *kp;
     const GridParams &g = P.g;
     const BubbleParams &bp = P.bp;
@@ -876,6 +850,7 @@ __global__ __launch_bounds__(256) void k_rp_replay(const RPLaunch *kp, int cur, 
     }
     if (bad) atomicOr(&sc->flags, 2);
     if (capped) atomicOr(&sc->flags, 4);
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc->mark[kMarkRP] = began;
 }
 
 // The initial void fraction (calculate_void_fraction at set-up,
@@ -904,6 +879,7 @@ __global__ __launch_bounds__(256) void k_scatter_initial(GridParams g, BubblePar
 __global__ __launch_bounds__(256) void k_scatter_radii(GridParams g, BubbleParams bp,
                                                         BubbleArrays b, const double *Rt,
                                                         int64_t *fg, StepScalars *sc) {
+    set_mark(sc, kMarkRP);
     __shared__ WaveAgg agg_all[4];
     WaveAgg &agg = agg_all[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
@@ -1007,7 +983,6 @@ void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
     if (b.n <= 0) return;
     const int nblk = (b.n + 255) / 256;
     hipLaunchKernelGGL(k_motion<F>, dim3(nblk), dim3(256), 0, s, g, bp, b, vx, vy, sc);
-    hipLaunchKernelGGL(k_bbox_reduce, dim3(1), dim3(256), 0, s, b.bbox_blk, nblk, sc);
 }
 
 // Workgroups of the persistent RP kernel: as many as fit (two per CU) when
@@ -1090,10 +1065,12 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
     const int solo_cap = lean ? (int)grid.x : std::max(1, cus / 8);
     if (host.bp.rp_exact)
         hipLaunchKernelGGL((k_bubble_persistent<F, false>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, quota, solo_cap);
+                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, quota,
+                           solo_cap);
     else
         hipLaunchKernelGGL((k_bubble_persistent<F, true>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, quota, solo_cap);
+                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, quota,
+                           solo_cap);
     return 4 * (int)grid.x;
 }
 
@@ -1290,7 +1267,8 @@ constexpr double kKeyRadius = 3.0e-6;    // m
 template <typename F>
 __global__ __launch_bounds__(256) void k_queue_keys(GridParams g, BubbleParams bp, BubbleArrays b,
                                                     const F *__restrict__ p0, int cur, int plp,
-                                                    int slot, int ext) {
+                                                    int slot, int ext, StepScalars *sc) {
+    set_mark(sc, kMarkQueue);
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= b.n) return;
     const double x = b.x[idx], y = b.y[idx];
@@ -1313,15 +1291,18 @@ __global__ __launch_bounds__(256) void k_queue_keys(GridParams g, BubbleParams b
 
 template <typename F>
 void launch_queue_keys(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                       const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext) {
+                       const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext,
+                       StepScalars *sc) {
     if (b.n <= 0) return;
     hipLaunchKernelGGL(k_queue_keys<F>, dim3((b.n + 255) / 256), dim3(256), 0, s, g, bp, b, p0,
-                       cur, plp, slot, ext);
+                       cur, plp, slot, ext, sc);
 }
 template void launch_queue_keys<double>(hipStream_t, const GridParams &, const BubbleParams &,
-                                        const BubbleArrays &, const double *, int, int, int, int);
+                                        const BubbleArrays &, const double *, int, int, int, int,
+                                        StepScalars *);
 template void launch_queue_keys<float>(hipStream_t, const GridParams &, const BubbleParams &,
-                                       const BubbleArrays &, const float *, int, int, int, int);
+                                       const BubbleArrays &, const float *, int, int, int, int,
+                                       StepScalars *);
 
 void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key, int threshold,
                             int ext) {

@@ -86,7 +86,8 @@ __global__ __launch_bounds__(256) void k_velocity(GridParams g, F *__restrict__ 
                                                    int first, const F *__restrict__ cxa,
                                                    const F *__restrict__ cxb,
                                                    const F *__restrict__ cya,
-                                                   const F *__restrict__ cyb) {
+                                                   const F *__restrict__ cyb, StepScalars *sc) {
+    set_mark(sc, kMarkVelocity);
     typedef typename Vec4<F>::type V;
     const int lane = threadIdx.x;
     const int i0 = (blockIdx.x * kBX + lane) * kGW;
@@ -167,7 +168,9 @@ __global__ __launch_bounds__(256) void k_velocity_small(GridParams g, F *__restr
                                                         int first, const F *__restrict__ cxa,
                                                         const F *__restrict__ cxb,
                                                         const F *__restrict__ cya,
-                                                        const F *__restrict__ cyb) {
+                                                        const F *__restrict__ cyb,
+                                                        StepScalars *sc) {
+    set_mark(sc, kMarkVelocity);
     const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
     if (i > g.N || j > g.M) return;
     const int64_t o = frame_off(i, j, g.pitch);
@@ -198,6 +201,8 @@ __device__ inline void clear_scalars(StepScalars *sc) {
     sc->sub_sum = 0ull;
     sc->done = 0u;
     sc->reused = 0u;
+    for (int k = 0; k < 5; k++) sc->phase[k] = 0ull;
+    sc->mark[kMarkMotion] = 0ull;
 }
 
 // Focused source value of row-0 cell i at time t (MixtureBoundaryPressureKernel
@@ -330,6 +335,7 @@ __global__ __launch_bounds__(256) void k_pressure_first(
     int64_t *__restrict__ fg_mp, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
     const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
     const double *__restrict__ rxp, StepScalars *sc) {
+    set_mark(sc, kMarkPressure);
     typedef typename Vec4<F>::type V;
     const int lane = threadIdx.x;
     const int i0 = (blockIdx.x * kBX + lane) * kGW;  // cells i0 .. i0 + 3 of [0, N+1]
@@ -442,6 +448,7 @@ __global__ __launch_bounds__(256) void k_pressure_first_small(
     int64_t *__restrict__ fg_mp, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
     const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
     const double *__restrict__ rxp, StepScalars *sc) {
+    set_mark(sc, kMarkPressure);
     const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
     double rmax = 0.0;
     bool bad = false;
@@ -496,6 +503,7 @@ __global__ __launch_bounds__(256) void k_pressure_picard(
     int64_t *__restrict__ fg_prev, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
     const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
     const double *__restrict__ rxp, StepScalars *sc, int slot) {
+    set_mark(sc, kMarkPicard);
     const int i = w.i0 + (int)(blockIdx.x * kBX + threadIdx.x);
     double rmax = 0.0;
     bool bad = false;
@@ -558,14 +566,21 @@ __device__ inline void totals_add(RPTotals &a, const RPTotals &b) {
 // two or three atomics of every wavefront on one address each cost the launch
 // about 14 ns apiece (256^2, 1024 bubbles, one per wavefront: 73 us a launch
 // with them, 25 us with the records).
+// Its last duty is the evaluation's report to the host, straight into pinned
+// memory: a copy command per report, and the host's wait for it, cost 10 us a
+// step more.  eval: 0 the step's first evaluation (which also folds k_motion's
+// bounding boxes), k Picard iteration k, whose source row is the first's.
 template <typename F>
 __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           const double *el_amp,
                                                           const double *el_phase, double t,
-                                                          const RPTotals *tot, int n_tot,
-                                                          StepScalars *sc) {
+                                                          int eval, const RPTotals *tot, int n_tot,
+                                                          const int *bbox_blk, int n_bbox,
+                                                          StepScalars *sc, StepReport *rep,
+                                                          unsigned long long seq) {
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
+    const unsigned long long began = wall_clock64();
     if (n_tot > 0) {  // workgroup-uniform
         __shared__ RPTotals red[16];
         RPTotals a{0ull, 0u, 0u, 0, 0};
@@ -585,34 +600,90 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             sc->flags |= a.flags;
         }
     }
-    const double pamp = g.rho_inf * g.cs_inf * g.amp;
-    for (int i = 1 + tid; i <= N; i += nt) {
-        if (!g.pml_y0) p0[frame_off(i, 0, P)] = p0[frame_off(i, 1, P)];
-        if (g.src_row) {
-            if (g.plane_p) {
-                double v = 0.0;
-                if (fmod(t, ((double)g.on_wave + (double)g.off_wave) / g.freq) <=
-                    ((double)g.on_wave) / g.freq)
-                    v = pamp * sin(g.omega * t);
-                p0[frame_off(i, 0, P)] = (F)v;
-            }
-            if (g.focused_p)
-                p0[frame_off(i, 0, P)] =
-                    (F)focused_value(g, i, t, pamp, -0.5 * g.dy, el_amp, el_phase);
+    if (n_bbox > 0) {  // workgroup-uniform
+        __shared__ int box[16][4];
+        int v[4] = {0x7fffffff, -0x7fffffff, 0x7fffffff, -0x7fffffff};
+        for (int k = tid; k < n_bbox; k += nt) {
+            const int4 q = ((const int4 *)bbox_blk)[k];
+            v[0] = min(v[0], q.x);
+            v[1] = max(v[1], q.y);
+            v[2] = min(v[2], q.z);
+            v[3] = max(v[3], q.w);
         }
-        if (!g.pml_y1) {
-            // As the reference (kernel.cuh:929-932): rows X..X+1 copy row 2Y+1-j (rows outside [0, M+1] skipped).
-            for (int j = N; j <= N + 1; j++) {
-                int src = 2 * M + 1 - j;
-                if (j >= 0 && j <= M + 1 && src >= 0 && src <= M + 1)
-                    p0[frame_off(i, j, P)] = p0[frame_off(i, src, P)];
+        for (int off = 32; off > 0; off >>= 1)
+            for (int c = 0; c < 4; c++) {
+                const int u = __shfl_xor(v[c], off, 64);
+                v[c] = (c & 1) ? max(v[c], u) : min(v[c], u);
             }
+        if ((tid & 63) == 0)
+            for (int c = 0; c < 4; c++) box[tid >> 6][c] = v[c];
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < nt / 64; w++)
+                for (int c = 0; c < 4; c++)
+                    v[c] = (c & 1) ? max(v[c], box[w][c]) : min(v[c], box[w][c]);
+            if (v[0] <= v[1])
+                for (int c = 0; c < 4; c++) sc->bbox[c] = v[c];
         }
     }
+    const double pamp = g.rho_inf * g.cs_inf * g.amp;
+    const bool source = g.src_row && (g.plane_p || g.focused_p);
+    if ((!g.pml_y0 && !source) || (source && eval == 0) || !g.pml_y1)
+        for (int i = 1 + tid; i <= N; i += nt) {
+            if (!g.pml_y0 && !source) p0[frame_off(i, 0, P)] = p0[frame_off(i, 1, P)];
+            if (source && eval == 0) {
+                if (g.plane_p) {
+                    double v = 0.0;
+                    if (fmod(t, ((double)g.on_wave + (double)g.off_wave) / g.freq) <=
+                        ((double)g.on_wave) / g.freq)
+                        v = pamp * sin(g.omega * t);
+                    p0[frame_off(i, 0, P)] = (F)v;
+                }
+                if (g.focused_p)
+                    p0[frame_off(i, 0, P)] =
+                        (F)focused_value(g, i, t, pamp, -0.5 * g.dy, el_amp, el_phase);
+            }
+            if (!g.pml_y1) {
+                // As the reference (kernel.cuh:929-932): rows X..X+1 copy row 2Y+1-j (rows outside [0, M+1] skipped).
+                for (int j = N; j <= N + 1; j++) {
+                    int src = 2 * M + 1 - j;
+                    if (j >= 0 && j <= M + 1 && src >= 0 && src <= M + 1)
+                        p0[frame_off(i, j, P)] = p0[frame_off(i, src, P)];
+                }
+            }
+        }
     __syncthreads();
-    for (int j = tid; j <= M + 1; j += nt) {
-        if (!g.pml_x0) p0[frame_off(0, j, P)] = p0[frame_off(1, j, P)];
-        if (!g.pml_x1) p0[frame_off(N + 1, j, P)] = p0[frame_off(N, j, P)];
+    if (!g.pml_x0 || !g.pml_x1)
+        for (int j = tid; j <= M + 1; j += nt) {
+            if (!g.pml_x0) p0[frame_off(0, j, P)] = p0[frame_off(1, j, P)];
+            if (!g.pml_x1) p0[frame_off(N + 1, j, P)] = p0[frame_off(N, j, P)];
+        }
+    if (tid == 0) {
+        const unsigned long long *m = sc->mark;
+        unsigned long long ph[5];
+        for (int k = 0; k < 5; k++) ph[k] = sc->phase[k];
+        const unsigned long long now = wall_clock64();
+        if (eval == 0) {
+            const unsigned long long motion = m[kMarkMotion] ? m[kMarkMotion] : m[kMarkPressure];
+            ph[0] += motion - m[kMarkVelocity];
+            ph[1] += m[kMarkPressure] - motion;
+            ph[2] += now - m[kMarkPressure];
+        } else {  // an empty window has no evaluation kernel
+            const unsigned long long p = m[kMarkPicard] > m[kMarkRP] ? m[kMarkPicard] : began;
+            ph[4] += m[kMarkQueue] ? m[kMarkRP] - m[kMarkQueue] : 0ull;
+            ph[3] += p - m[kMarkRP];
+            ph[2] += now - p;
+        }
+        sc->mark[kMarkQueue] = 0ull;
+        rep->resid = __longlong_as_double((long long)sc->resid[eval]);
+        for (int k = 0; k < 4; k++) rep->bbox[k] = sc->bbox[k];
+        rep->flags = sc->flags;
+        rep->sub_max = sc->sub_max;
+        rep->sub_sum = sc->sub_sum;
+        rep->done = sc->done;
+        rep->reused = sc->reused;
+        for (int k = 0; k < 5; k++) rep->phase[k] = sc->phase[k] = ph[k];
+        __hip_atomic_store(&rep->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -637,17 +708,17 @@ static bool pressure_small(const GridParams &g) { return (int64_t)g.N * g.M < 30
 template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
                      const int64_t *fgn, Window w, int first_step, const F *cxa, const F *cxb,
-                     const F *cya, const F *cyb) {
+                     const F *cya, const F *cyb, StepScalars *sc) {
     if (velocity_small(g)) {
         hipLaunchKernelGGL(k_velocity_small<F>, dim3((g.N + kBX) / kBX, (g.M + kBY) / kBY),
                            dim3(kBX, kBY), 0, s, g, vx, vy, p0, fgn, w, first_step, cxa, cxb, cya,
-                           cyb);
+                           cyb, sc);
         return;
     }
     dim3 blk(kBX, kBY);  // columns 0..N, rows 0..M
     dim3 grd((g.N + 1 + kBX * kGW - 1) / (kBX * kGW), (g.M + 1 + kGBlockRows - 1) / kGBlockRows);
     hipLaunchKernelGGL(k_velocity<F>, grd, blk, 0, s, g, vx, vy, p0, fgn, w, first_step, cxa,
-                       cxb, cya, cyb);
+                       cxb, cya, cyb, sc);
 }
 
 template <typename F>
@@ -692,10 +763,11 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
 
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
-                            const double *el_phase, double t, const RPTotals *tot, int n_tot,
-                            StepScalars *sc) {
+                            const double *el_phase, double t, int eval, const RPTotals *tot,
+                            int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
+                            StepReport *rep, unsigned long long seq) {
     hipLaunchKernelGGL(k_pressure_ghosts<F>, dim3(1), dim3(1024), 0, s, g, p0, el_amp,
-                       el_phase, t, tot, n_tot, sc);
+                       el_phase, t, eval, tot, n_tot, bbox_blk, n_bbox, sc, rep, seq);
 }
 
 void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
@@ -705,7 +777,7 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
 #define BRP_INST(F)                                                                          \
     template void launch_velocity<F>(hipStream_t, const GridParams &, F *, F *, const F *,   \
                                      const int64_t *, Window, int, const F *, const F *,     \
-                                     const F *, const F *);                                  \
+                                     const F *, const F *, StepScalars *);                   \
     template void launch_velocity_ghosts<F>(hipStream_t, const GridParams &, F *, F *,      \
                                             double, StepScalars *, int);                     \
     template void launch_pressure_first<F>(                                                  \
@@ -717,8 +789,9 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
         F *, F *, const int64_t *, const int64_t *, int64_t *, Window, const F *, const F *, \
         const F *, const F *, const double *, const double *, StepScalars *, int);           \
     template void launch_pressure_ghosts<F>(hipStream_t, const GridParams &, F *,           \
-                                            const double *, const double *, double,          \
-                                            const RPTotals *, int, StepScalars *);
+                                            const double *, const double *, double, int,     \
+                                            const RPTotals *, int, const int *, int,         \
+                                            StepScalars *, StepReport *, unsigned long long);
 
 BRP_INST(double)
 BRP_INST(float)

@@ -40,7 +40,8 @@ __device__ inline double delta_t(double coef_x, double coef_k, int pos, double h
     return coef_x * (1.0 + cos(coef_k * (((double)pos - 0.5) * h - b)));
 }
 
-__global__ void k_zero_window(double *q, Window w, int pitch) {
+__global__ void k_zero_window(double *q, Window w, int pitch, StepScalars *sc) {
+    set_mark(sc, kMarkThermal);
     const int i = w.i0 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int j = w.j0 + (int)blockIdx.y;
     if (i > w.i1 || j > w.j1) return;
@@ -145,8 +146,9 @@ __global__ __launch_bounds__(256) void k_temperature_increment(
     GridParams g, double T_inf, const double *__restrict__ T, const int64_t *__restrict__ fg,
     const int64_t *__restrict__ fgn, int first, const F *__restrict__ px,
     const F *__restrict__ py, const F *__restrict__ pnx, const F *__restrict__ pny,
-    const double *__restrict__ heat, double *__restrict__ dT) {
+    const double *__restrict__ heat, double *__restrict__ dT, StepScalars *sc) {
 #pragma clang fp contract(off)
+    if (sc) set_mark(sc, kMarkThermal);  // no heat kernels ran before
     const int i = 1 + (int)(blockIdx.x * kTX + threadIdx.x);
     const int j = 1 + (int)(blockIdx.y * kTY + threadIdx.y);
     if (i > g.N || j > g.M) return;
@@ -244,7 +246,8 @@ __global__ __launch_bounds__(256) void k_focal_blocks(GridParams g, const double
     }
 }
 
-__global__ __launch_bounds__(256) void k_focal_final(GridParams g, int nblk, StepScalars *sc) {
+__global__ __launch_bounds__(256) void k_focal_final(GridParams g, int nblk, StepScalars *sc,
+                                                     StepReport *rep, unsigned long long seq) {
     __shared__ double sv[256];
     __shared__ int sk[256];
     const int t = threadIdx.x;
@@ -258,36 +261,40 @@ __global__ __launch_bounds__(256) void k_focal_final(GridParams g, int nblk, Ste
     if (t == 0) {
         const int W = g.N + 2;
         const int k = sk[0] == 0x7fffffff ? 0 : sk[0];
-        sc->focal[0] = (double)(k % W) * g.dx;
-        sc->focal[1] = (double)(k / W) * g.dy;
+        rep->focal[0] = sc->focal[0] = (double)(k % W) * g.dx;
+        rep->focal[1] = sc->focal[1] = (double)(k / W) * g.dy;
+        rep->phase[4] = sc->phase[4] += wall_clock64() - sc->mark[kMarkThermal];
+        __hip_atomic_store(&rep->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
 }  // namespace
 
 void launch_focal_point(hipStream_t s, const GridParams &g, const double *dT, const double *heat,
-                        StepScalars *sc) {
+                        StepScalars *sc, StepReport *rep, unsigned long long seq) {
     const int n = (g.N + 2) * (g.M + 2);
     const int nblk = std::min(256, (n + 255) / 256);
     hipLaunchKernelGGL(k_focal_blocks, dim3(nblk), dim3(256), 0, s, g, dT, heat, sc);
-    hipLaunchKernelGGL(k_focal_final, dim3(1), dim3(256), 0, s, g, nblk, sc);
+    hipLaunchKernelGGL(k_focal_final, dim3(1), dim3(256), 0, s, g, nblk, sc, rep, seq);
 }
 
 template <typename F>
 void launch_temperature(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                         const BubbleArrays &b, bool bubbles, Window w, double T_inf, double *T,
                         double *dT, double *heat, const int64_t *fg, const int64_t *fgn,
-                        int first, const F *px, const F *py, const F *pnx, const F *pny) {
-    if (bubbles && w.i0 <= w.i1 && w.j0 <= w.j1) {
+                        int first, const F *px, const F *py, const F *pnx, const F *pny,
+                        StepScalars *sc) {
+    const bool hot = bubbles && w.i0 <= w.i1 && w.j0 <= w.j1;
+    if (hot) {
         hipLaunchKernelGGL(k_zero_window, dim3((w.i1 - w.i0 + 256) / 256, w.j1 - w.j0 + 1),
-                           dim3(256), 0, s, heat, w, g.pitch);
+                           dim3(256), 0, s, heat, w, g.pitch, sc);
         if (b.n > 0)
             hipLaunchKernelGGL(k_bubble_heat, dim3((b.n + 255) / 256), dim3(256), 0, s, g, bp, b,
                                heat);
     }
     const dim3 blk(kTX, kTY), grid((g.N + kTX - 1) / kTX, (g.M + kTY - 1) / kTY);
     hipLaunchKernelGGL(k_temperature_increment<F>, grid, blk, 0, s, g, T_inf, T, fg, fgn, first,
-                       px, py, pnx, pny, heat, dT);
+                       px, py, pnx, pny, heat, dT, hot ? nullptr : sc);
     hipLaunchKernelGGL(k_temperature_add, grid, blk, 0, s, g, T, dT);
     hipLaunchKernelGGL(k_temperature_ghosts, dim3(1), dim3(1024), 0, s, g, T);
 }
@@ -296,11 +303,11 @@ template void launch_temperature<float>(hipStream_t, const GridParams &, const B
                                         const BubbleArrays &, bool, Window, double, double *,
                                         double *, double *, const int64_t *, const int64_t *, int,
                                         const float *, const float *, const float *,
-                                        const float *);
+                                        const float *, StepScalars *);
 template void launch_temperature<double>(hipStream_t, const GridParams &, const BubbleParams &,
                                          const BubbleArrays &, bool, Window, double, double *,
                                          double *, double *, const int64_t *, const int64_t *,
                                          int, const double *, const double *, const double *,
-                                         const double *);
+                                         const double *, StepScalars *);
 
 }  // namespace brp

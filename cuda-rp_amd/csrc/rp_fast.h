@@ -109,7 +109,11 @@ typedef __attribute__((address_space(4))) const double cdouble;
 // where the sub-step uses them rather than held in scalar registers across
 // the sub-step loop; vtab is the kernel's LDS copy of the V and Y tables.
 __device__ inline RPFastShared rp_shared_load(const double *tab, const double *vtab) {
-    cdouble *t = (cdouble *)tab;
+    // one value for the wavefront, also where the pointer came from a vector load
+    const unsigned long long p = (unsigned long long)tab;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)p);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(p >> 32));
+    cdouble *t = (cdouble *)(((unsigned long long)hi << 32) | lo);
     asm volatile("" : "+s"(t));
     return RPFastShared{t[0], t[1], t[2],  t[3],  t[4],  t[5],  t[6], t[7],
                         t[8], t[9], t[10], t[11], t[12], t[13], t[14], vtab};

@@ -68,3 +68,21 @@ def test_both_splits(brp, nx, ny):
     x, y = nx * 1e-4 * r.random(n), ny * 1e-4 * r.random(n)
     cfg = config(brp, nx, ny, 0b1010, SOURCES[1], bubbles=True)
     check(brp, cfg, (x, y, np.full(n, 3e-6), None, 1e-6), steps=2, names=FIELDS + ("fg",))
+
+
+@pytest.mark.parametrize("bubbles,thermal", [(0, 0), (1, 0), (1, 1), (0, 1)])
+def test_phase_times_are_parts_of_the_call(brp, bubbles, thermal):
+    import time
+    cfg = config(brp, 200, 180, 15, SOURCES[1], bubbles=bool(bubbles))
+    cfg.update(thermal=thermal)
+    b = (np.full(1, 8e-3), np.full(1, 9e-3), np.full(1, 3e-6), None, 1e-6) if bubbles else None
+    with cases.make(brp.Simulation, cfg, b) as sim:
+        sim.step(5)
+        t0 = time.perf_counter()
+        n_pic = sum(s["n_pic"] for s in sim.step(40))
+        wall = (time.perf_counter() - t0) * 1e3
+        ph = sim.phase_times()
+    assert all(v >= 0.0 for v in ph.values()) and ph["velocity"] > 0.0 and ph["pressure"] > 0.0
+    assert (ph["motion"] > 0.0) == bool(bubbles) and (ph["bubble_rp"] > 0.0) == (n_pic > 0)
+    assert ph["other"] > 0.0 or not thermal
+    assert 0.2 * wall < sum(ph.values()) < wall, (ph, wall)
