@@ -80,8 +80,9 @@ thread_local std::string g_create_error;
 
 struct Snapshot {
     bool valid = false;
-    std::vector<void *> bufs;   // device copies, same order as the handle's buffer list
-    std::vector<size_t> sizes;
+    char *block = nullptr;  // device copies of the state arrays, one after another
+    size_t capacity = 0;
+    size_t arrays = 0;      // state arrays of the handle when it was taken
     // scalar state
     int pc, fcur, fn, fm, fz, rp_cur, pl_m, pl_n, pl_p, first_step;
     Window W;
@@ -251,7 +252,15 @@ struct brp_handle {
     double phase_ms[5] = {0, 0, 0, 0, 0};
 
     std::vector<void *> allocs;
-    std::vector<size_t> alloc_sizes;
+    // what a snapshot holds: the arrays that a step changes and the source's
+    // elements (void-fraction arrays are zero outside the window's rows, so
+    // their part of it is copied)
+    struct StateArray {
+        void *p;
+        size_t bytes;
+        bool fg;
+    };
+    std::vector<StateArray> state;
     size_t dev_bytes = 0;
     Snapshot snaps[16];
 
@@ -284,7 +293,8 @@ int set_err(brp_handle *h, int code, const char *fmt, ...) {
                            __FILE__, __LINE__);                                          \
     } while (0)
 
-int dalloc(brp_handle *h, void **p, size_t bytes) {
+enum class Keep { kScratch, kState, kVoid };  // whether a snapshot holds the array
+int dalloc(brp_handle *h, void **p, size_t bytes, Keep keep = Keep::kScratch) {
     *p = nullptr;
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(p, bytes);
@@ -294,7 +304,7 @@ int dalloc(brp_handle *h, void **p, size_t bytes) {
     if (e != hipSuccess)
         return set_err(h, BRP_ERR_DEVICE, "hipMemset: %s", hipGetErrorString(e));
     h->allocs.push_back(*p);
-    h->alloc_sizes.push_back(bytes);
+    if (keep != Keep::kScratch) h->state.push_back({*p, bytes, keep == Keep::kVoid});
     h->dev_bytes += bytes;
     return BRP_OK;
 }
@@ -431,11 +441,15 @@ int alloc_bubbles(brp_handle *h, int n) {
     double **arrs[] = {&h->b.x,      &h->b.y,      &h->b.R[0],   &h->b.R[1],   &h->b.Rn[0],
                        &h->b.Rn[1],  &h->b.d1R[0], &h->b.d1R[1], &h->b.PG[0],  &h->b.PG[1],
                        &h->b.bdt[0], &h->b.bdt[1], &h->b.re[0],  &h->b.re[1],  &h->b.R_t,
-                       &h->b.Q_B,    &h->b.PL[0],  &h->b.PL[1],  &h->b.PL[2],  &h->b.n_B,
-                       &h->b.R0,     &h->b.PG0,    &h->b.calpha, &h->b.vx,     &h->b.vy};
+                       &h->b.Q_B,    &h->b.PL[0],  &h->b.PL[1],  &h->b.PL[2],  &h->b.vx,
+                       &h->b.vy};
     for (double **a : arrs)
+        if ((rc = dalloc(h, (void **)a, bytes, Keep::kState))) return rc;
+    double **consts[] = {&h->b.n_B, &h->b.R0, &h->b.PG0, &h->b.calpha};
+    for (double **a : consts)
         if ((rc = dalloc(h, (void **)a, bytes))) return rc;
-    if ((rc = dalloc(h, (void **)&h->b.sub, sizeof(int) * (size_t)std::max(n, 1)))) return rc;
+    if ((rc = dalloc(h, (void **)&h->b.sub, sizeof(int) * (size_t)std::max(n, 1), Keep::kState)))
+        return rc;
     if ((rc = dalloc(h, (void **)&h->b.order, sizeof(int) * (size_t)std::max(n, 1)))) return rc;
     if ((rc = dalloc(h, (void **)&h->b.key, sizeof(int) * (size_t)std::max(n, 1)))) return rc;
     if ((rc = dalloc(h, (void **)&h->b.order_tmp, sizeof(int) * (size_t)std::max(n, 1))) ||
@@ -568,25 +582,45 @@ void field_extent(const brp_handle *h, int field, int *nx, int *ny, int *i0, int
 
 
 // ---- state snapshots (save/restore slots, adjoint checkpoints and tape) ----
-int snap_save(brp_handle *h, Snapshot &sn) {
-    if (!sn.valid && sn.bufs.empty()) {
-        for (size_t k = 0; k < h->allocs.size(); k++) {
-            void *p = nullptr;
-            if (hipMalloc(&p, h->alloc_sizes[k]) != hipSuccess) {
-                for (void *q : sn.bufs) (void)hipFree(q);
-                sn.bufs.clear();
-                sn.sizes.clear();
-                return set_err(h, BRP_ERR_DEVICE, "snapshot allocation failed (%zu bytes)",
-                               h->dev_bytes);
-            }
-            sn.bufs.push_back(p);
-            sn.sizes.push_back(h->alloc_sizes[k]);
+// The copies between the state arrays and a snapshot's block (block null: only
+// their total size, which is returned): whole arrays, and the rows of window w
+// of the void-fraction arrays.
+size_t snap_plan(const brp_handle *h, const Window &w, char *block, bool save, CopyPlan *plan) {
+    size_t at = 0;
+    for (const brp_handle::StateArray &a : h->state) {
+        size_t o = 0, n = a.bytes;
+        if (a.fg) {
+            const size_t row = sizeof(int64_t) * h->pitch;
+            const bool any = w.i0 <= w.i1 && w.j0 <= w.j1;
+            o = any ? row * (w.j0 + 1) : 0;
+            n = any ? row * (w.j1 - w.j0 + 1) : 0;
         }
+        if (block) {
+            char *p = (char *)a.p + o;
+            plan->add(save ? block + at : p, save ? p : block + at, n);
+        }
+        at += (n + 255) & ~size_t(255);
     }
-    if (sn.bufs.size() != h->allocs.size()) return set_err(h, BRP_ERR_STATE, "snapshot layout changed");
-    for (size_t k = 0; k < h->allocs.size(); k++)
-        HIPCHK(h, hipMemcpyAsync(sn.bufs[k], h->allocs[k], sn.sizes[k], hipMemcpyDeviceToDevice, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return at;
+}
+
+int snap_save(brp_handle *h, Snapshot &sn) {
+    const size_t need = snap_plan(h, h->W, nullptr, true, nullptr);
+    if (sn.arrays && sn.arrays != h->state.size())
+        return set_err(h, BRP_ERR_STATE, "snapshot layout changed");
+    if (need > sn.capacity) {
+        char *q = nullptr;
+        if (hipMalloc((void **)&q, need) != hipSuccess)
+            return set_err(h, BRP_ERR_DEVICE, "snapshot allocation failed (%zu bytes)", need);
+        if (sn.block) (void)hipFree(sn.block);
+        sn.block = q;
+        sn.capacity = need;
+    }
+    sn.arrays = h->state.size();
+    CopyPlan plan;
+    snap_plan(h, h->W, sn.block, true, &plan);
+    launch_copy_many(h->stream, plan);
+    HIPCHK(h, hipGetLastError());
     sn.pc = h->pc;
     sn.fcur = h->fcur;
     sn.fn = h->fn;
@@ -609,10 +643,23 @@ int snap_save(brp_handle *h, Snapshot &sn) {
 }
 
 int snap_restore(brp_handle *h, const Snapshot &sn) {
-    if (sn.bufs.size() != h->allocs.size()) return set_err(h, BRP_ERR_STATE, "snapshot layout changed");
-    for (size_t k = 0; k < h->allocs.size(); k++)
-        HIPCHK(h, hipMemcpyAsync(h->allocs[k], sn.bufs[k], sn.sizes[k], hipMemcpyDeviceToDevice, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (sn.arrays != h->state.size()) return set_err(h, BRP_ERR_STATE, "snapshot layout changed");
+    CopyPlan plan;
+    // rows of the present window that the snapshot's does not cover: zeros
+    const Window &w = h->W, &v = sn.W;
+    if (w.i0 <= w.i1 && w.j0 <= w.j1) {
+        const bool any = v.i0 <= v.i1 && v.j0 <= v.j1;
+        const int part[2][2] = {{w.j0, any ? std::min(w.j1, v.j0 - 1) : w.j1},
+                                {any ? std::max(w.j0, v.j1 + 1) : w.j1 + 1, w.j1}};
+        const size_t row = sizeof(int64_t) * h->pitch;
+        for (const brp_handle::StateArray &a : h->state)
+            for (const auto &r : part)
+                if (a.fg && r[0] <= r[1])
+                    plan.add((char *)a.p + row * (r[0] + 1), nullptr, row * (r[1] - r[0] + 1));
+    }
+    snap_plan(h, v, sn.block, false, &plan);
+    launch_copy_many(h->stream, plan);
+    HIPCHK(h, hipGetLastError());
     h->pc = sn.pc;
     h->fcur = sn.fcur;
     h->fn = sn.fn;
@@ -637,16 +684,8 @@ int snap_restore(brp_handle *h, const Snapshot &sn) {
 }
 
 void snap_free(Snapshot &sn) {
-    for (void *q : sn.bufs) (void)hipFree(q);
-    sn.bufs.clear();
-    sn.sizes.clear();
-    sn.valid = false;
-}
-
-size_t snap_bytes(const brp_handle *h) {
-    size_t b = 0;
-    for (size_t z : h->alloc_sizes) b += z;
-    return b;
+    if (sn.block) (void)hipFree(sn.block);
+    sn = Snapshot{};
 }
 
 // Device memory owned by one adjoint call (freed at its end).
@@ -674,17 +713,6 @@ struct AdjMem {
 // Cells of a record rectangle.
 size_t rect_cells(const Window &w) {
     return w.i0 > w.i1 || w.j0 > w.j1 ? 0 : (size_t)(w.i1 - w.i0 + 1) * (size_t)(w.j1 - w.j0 + 1);
-}
-
-// Copies rectangle w of a frame array (elements of `elem` bytes) into a
-// dense buffer.
-int copy_rect(brp_handle *h, void *dst, const void *src, size_t elem, const Window &w) {
-    const size_t cols = (size_t)(w.i1 - w.i0 + 1), rows = (size_t)(w.j1 - w.j0 + 1);
-    if (!rect_cells(w)) return BRP_OK;
-    const char *s0 = (const char *)src + frame_off(w.i0, w.j0, h->pitch) * elem;
-    HIPCHK(h, hipMemcpy2DAsync(dst, cols * elem, s0, (size_t)h->pitch * elem, cols * elem, rows,
-                               hipMemcpyDeviceToDevice, h->stream));
-    return BRP_OK;
 }
 
 int rec_alloc(brp_handle *h, StepRecord *r, size_t bytes, bool bub, void **out) {
@@ -900,8 +928,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         if (rec) {
             int rc = rec_grow(h, rec, 1);
             if (rc) return rc;
-            if (rec->want_grid)
-                HIPCHK(h, hipMemcpyAsync(rec->p0_start, h->p0, sizeof(F) * h->frame, hipMemcpyDeviceToDevice, s));
+            CopyPlan plan;
+            if (rec->want_grid) plan.add(rec->p0_start, h->p0, sizeof(F) * h->frame);
             if (rec->want_bub && h->nb > 0) {
                 const size_t nbb = sizeof(double) * h->nb;
                 const int c = h->rp_cur;
@@ -909,9 +937,9 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                    h->b.bdt[c], h->b.re[c], h->b.PL[h->pl_m], h->b.PL[h->pl_n]};
                 double *dst[10] = {rec->x_start, rec->y_start, rec->rp[0], rec->rp[1], rec->rp[2],
                                    rec->rp[3], rec->rp[4], rec->rp[5], rec->PLm, rec->PLn};
-                for (int q = 0; q < 10; q++)
-                    HIPCHK(h, hipMemcpyAsync(dst[q], src[q], nbb, hipMemcpyDeviceToDevice, s));
+                for (int q = 0; q < 10; q++) plan.add(dst[q], src[q], nbb);
             }
+            launch_copy_many(s, plan);
             rec->first = h->first_step;
             rec->t = h->t;
         }
@@ -936,10 +964,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         if (rec && rec->want_grid) {  // the window is final for this step
             int rc = rec_set_rect(h, rec);
             if (rc) return rc;
-            if ((rc = copy_rect(h, rec->fgC, h->fgb[old_cur], sizeof(int64_t), rec->rect)) ||
-                (rc = copy_rect(h, rec->p0_it[0], p0, sizeof(F), rec->rect)) ||
-                (rc = copy_rect(h, rec->fg_it[0], h->fgb[old_m], sizeof(int64_t), rec->rect)))
-                return rc;
+            RectPlan rp;
+            rp.add(rec->fgC, h->fgb[old_cur], sizeof(int64_t));
+            rp.add(rec->p0_it[0], p0, sizeof(F));
+            rp.add(rec->fg_it[0], h->fgb[old_m], sizeof(int64_t));
+            launch_copy_rects(s, rp, rec->rect, h->pitch);
         }
         int status = BRP_OK;
         long long lost = 0;  // bubbles the RP kernel did not write back
@@ -992,14 +1021,12 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     }
                 }
                 if (h->cfg.tr_cylindrical) launch_cyl_fold(s, h->g, h->fgb[target]);
-                if (rec && rec->want_grid) {
-                    int rc = copy_rect(h, rec->fg_it[loop], h->fgb[target], sizeof(int64_t), rec->rect);
-                    if (rc) return rc;
-                }
                 if (rec && rec->want_bub) {
-                    HIPCHK(h, hipMemcpyAsync(rec->PLp_it[loop], h->b.PL[h->pl_p], sizeof(double) * h->nb, hipMemcpyDeviceToDevice, s));
-                    HIPCHK(h, hipMemcpyAsync(rec->Rt_it[loop], h->b.R_t, sizeof(double) * h->nb, hipMemcpyDeviceToDevice, s));
-                    HIPCHK(h, hipMemcpyAsync(rec->sub_it[loop], h->b.sub, sizeof(int) * h->nb, hipMemcpyDeviceToDevice, s));
+                    CopyPlan plan;
+                    plan.add(rec->PLp_it[loop], h->b.PL[h->pl_p], sizeof(double) * h->nb);
+                    plan.add(rec->Rt_it[loop], h->b.R_t, sizeof(double) * h->nb);
+                    plan.add(rec->sub_it[loop], h->b.sub, sizeof(int) * h->nb);
+                    launch_copy_many(s, plan);
                 }
                 launch_pressure_picard<F>(s, h->g, vx, vy, (F *)h->pb[pn_i][0], (F *)h->pb[pn_i][1],
                                           (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0,
@@ -1008,9 +1035,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
                                           h->b.totals, rp_waves, nullptr, 0, h->sc_d, h->rep,
                                           ++h->rep_seq);
-                if (rec && rec->want_grid) {
-                    int rc = copy_rect(h, rec->p0_it[loop], p0, sizeof(F), rec->rect);
-                    if (rc) return rc;
+                if (rec && rec->want_grid) {  // the iterate that the evaluation read, and its pressure
+                    RectPlan rp;
+                    rp.add(rec->fg_it[loop], h->fgb[target], sizeof(int64_t));
+                    rp.add(rec->p0_it[loop], p0, sizeof(F));
+                    launch_copy_rects(s, rp, rec->rect, h->pitch);
                 }
                 if (int rc = wait_report(h)) return rc;
                 resimax = h->rep->resid / h->P_inf;
@@ -1064,14 +1093,16 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         if (rec) {
             rec->n_pic = loop;
             if (rec->want_grid) {
-                int rc;
-                if ((rc = copy_rect(h, rec->vx_end, vx, sizeof(F), rec->rect)) ||
-                    (rc = copy_rect(h, rec->vy_end, vy, sizeof(F), rec->rect)))
-                    return rc;
+                RectPlan rp;
+                rp.add(rec->vx_end, vx, sizeof(F));
+                rp.add(rec->vy_end, vy, sizeof(F));
+                launch_copy_rects(s, rp, rec->rect, h->pitch);
             }
             if (rec->want_bub && h->nb > 0) {
-                HIPCHK(h, hipMemcpyAsync(rec->x_end, h->b.x, sizeof(double) * h->nb, hipMemcpyDeviceToDevice, s));
-                HIPCHK(h, hipMemcpyAsync(rec->y_end, h->b.y, sizeof(double) * h->nb, hipMemcpyDeviceToDevice, s));
+                CopyPlan plan;
+                plan.add(rec->x_end, h->b.x, sizeof(double) * h->nb);
+                plan.add(rec->y_end, h->b.y, sizeof(double) * h->nb);
+                launch_copy_many(s, plan);
             }
         }
         if (ctl && ctl->npic_out) ctl->npic_out->push_back(loop);
@@ -1108,13 +1139,13 @@ template <typename F>
 int alloc_grid(brp_handle *h) {
     int rc;
     const size_t fb = sizeof(F) * h->frame;
-    if ((rc = dalloc(h, &h->vx, fb)) || (rc = dalloc(h, &h->vy, fb)) || (rc = dalloc(h, &h->p0, fb)))
-        return rc;
+    for (void **f : {&h->vx, &h->vy, &h->p0})
+        if ((rc = dalloc(h, f, fb, Keep::kState))) return rc;
     for (int a = 0; a < 2; a++)
         for (int c = 0; c < 2; c++)
-            if ((rc = dalloc(h, &h->pb[a][c], fb))) return rc;
+            if ((rc = dalloc(h, &h->pb[a][c], fb, Keep::kState))) return rc;
     for (int a = 0; a < 4; a++)
-        if ((rc = dalloc(h, (void **)&h->fgb[a], sizeof(int64_t) * h->frame))) return rc;
+        if ((rc = dalloc(h, (void **)&h->fgb[a], sizeof(int64_t) * h->frame, Keep::kVoid))) return rc;
     return init_coefficients<F>(h);
 }
 
@@ -1438,7 +1469,9 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
         // sub-step counts, per step start/end fields and bubble state
         size_t recb = arena.bytes();
         for (const StepRecord &r : recs) recb += rec_bytes(h, r);
-        stats->memory_bytes = (int64_t)((nseg + 1) * snap_bytes(h) + mem.bytes + recb);
+        size_t snapb = fin.capacity;
+        for (const Snapshot &c : ck) snapb += c.capacity;
+        stats->memory_bytes = (int64_t)(snapb + mem.bytes + recb);
         stats->n_checkpoints = nseg;
         stats->segment = K;
     }
@@ -1607,9 +1640,9 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
     int rc = h->prec == BRP_PREC_FP64 ? alloc_grid<double>(h) : alloc_grid<float>(h);
     if (rc) return fail(rc);
     if (c.thermal &&
-        ((rc = dalloc(h, (void **)&h->T_d, sizeof(double) * h->frame)) ||
-         (rc = dalloc(h, (void **)&h->dT_d, sizeof(double) * h->frame)) ||
-         (rc = dalloc(h, (void **)&h->heat_d, sizeof(double) * h->frame))))
+        ((rc = dalloc(h, (void **)&h->T_d, sizeof(double) * h->frame, Keep::kState)) ||
+         (rc = dalloc(h, (void **)&h->dT_d, sizeof(double) * h->frame, Keep::kState)) ||
+         (rc = dalloc(h, (void **)&h->heat_d, sizeof(double) * h->frame, Keep::kState))))
         return fail(rc);
     if ((rc = dalloc(h, (void **)&h->sc_d, sizeof(StepScalars)))) return fail(rc);
     {
@@ -1656,8 +1689,7 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
 void brp_destroy(brp_handle *h) {
     if (!h) return;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    for (auto &sn : h->snaps)
-        for (void *p : sn.bufs) (void)hipFree(p);
+    for (auto &sn : h->snaps) snap_free(sn);
     for (void *p : h->allocs) (void)hipFree(p);
     h->ring.release();
     if (h->rep) (void)hipHostFree(h->rep);
@@ -1715,8 +1747,8 @@ int brp_set_source(brp_handle *h, int32_t n_elem, const double *amp, const doubl
     std::vector<double> a(amp, amp + n_elem), p(phase, phase + n_elem);
     if (!h->el_amp_d) {
         int rc;
-        if ((rc = dalloc(h, (void **)&h->el_amp_d, sizeof(double) * 4096)) ||
-            (rc = dalloc(h, (void **)&h->el_phase_d, sizeof(double) * 4096)))
+        if ((rc = dalloc(h, (void **)&h->el_amp_d, sizeof(double) * 4096, Keep::kState)) ||
+            (rc = dalloc(h, (void **)&h->el_phase_d, sizeof(double) * 4096, Keep::kState)))
             return rc;
     }
     if (n_elem > 4096) return set_err(h, BRP_ERR_INVALID, "at most 4096 source elements");
@@ -2114,14 +2146,19 @@ int brp_save_state(brp_handle *h, int32_t slot) {
     if (!h || slot < 0 || slot >= 16) return BRP_ERR_INVALID;
     int rc = brp_prepare(h);
     if (rc) return rc;
-    return snap_save(h, h->snaps[slot]);
+    if ((rc = snap_save(h, h->snaps[slot]))) return rc;
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return BRP_OK;
 }
 
 int brp_restore_state(brp_handle *h, int32_t slot) {
     if (!h || slot < 0 || slot >= 16) return BRP_ERR_INVALID;
     Snapshot &sn = h->snaps[slot];
     if (!sn.valid) return set_err(h, BRP_ERR_STATE, "slot %d holds no state", slot);
-    return snap_restore(h, sn);
+    const int rc = snap_restore(h, sn);
+    if (rc) return rc;
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    return BRP_OK;
 }
 
 int brp_adjoint(brp_handle *h, const brp_objective *obj, double *grad_amp, double *grad_phase,

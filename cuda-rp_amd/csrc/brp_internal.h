@@ -314,6 +314,35 @@ struct HostRing {
 hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &src, int64_t rows,
                      double *dst, int64_t ld);
 
+// ---- copies (kernels_copy.hip) ----
+// Arrays to copy in one launch (16-byte aligned, sizes multiples of 4);
+// src null: zeros.
+struct CopyPlan {
+    static constexpr int kMax = 64;
+    int n = 0;
+    unsigned tiles = 0;
+    unsigned tile0[kMax];
+    void *dst[kMax];
+    const void *src[kMax];
+    size_t bytes[kMax];
+    void add(void *d, const void *s, size_t b);
+};
+void launch_copy_many(hipStream_t s, const CopyPlan &c);
+// One rectangle of several frame arrays (elements of 4 or 8 bytes), each into
+// a dense buffer.
+struct RectPlan {
+    int n = 0;
+    void *dst[4];
+    const void *src[4];
+    int elem[4];
+    void add(void *d, const void *s, size_t e) {
+        dst[n] = d;
+        src[n] = s;
+        elem[n++] = (int)e;
+    }
+};
+void launch_copy_rects(hipStream_t s, const RectPlan &r, const Window &w, int pitch);
+
 // ---- temperature (kernels_thermal.hip) ----
 template <typename F>
 void launch_temperature(hipStream_t s, const GridParams &g, const BubbleParams &bp,
