@@ -190,7 +190,12 @@ struct StepCtl {
     const int *force_npic = nullptr;
     StepRecord *rec = nullptr;
     std::vector<int> *npic_out = nullptr;
+    std::vector<Window> *win_out = nullptr;
     const StepRecord *tape_in = nullptr;
+    // With force_npic and tape_in: the step's window in the forward.  Nothing
+    // is then left for the host to decide, and the step is queued without
+    // waiting for any of its reports (the forward's status stands).
+    const Window *win = nullptr;
 };
 
 }  // namespace
@@ -242,6 +247,7 @@ struct brp_handle {
     unsigned long long rep_seq = 0;    // reports asked for so far
     double ms_per_tick = 1e-5;         // of the device's constant-rate clock
     RPLaunch *rpl_h = nullptr, *rpl_d = nullptr;  // the RP kernel's fixed parameters
+    bool rpl_valid = false;                       // rpl_d holds rpl_h
     Window W{1, 0, 1, 0};
     int first_step = 1;
     int64_t nstep = 0;
@@ -891,9 +897,18 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
     const int max_pic = std::min(h->cfg.max_picard > 0 ? h->cfg.max_picard : 1000, kMaxEval - 1);
     const bool bub = h->cfg.bub_enable && h->nb > 0;
     hipStream_t s = h->stream;
-    if (bub) {  // the RP kernel's parameters as of this call (no step is in flight)
-        *h->rpl_h = RPLaunch{h->g, h->bp, h->b};
-        HIPCHK(h, hipMemcpyAsync(h->rpl_d, h->rpl_h, sizeof(RPLaunch), hipMemcpyHostToDevice, s));
+    if (bub) {  // the RP kernel's parameters as of this call, where they have changed
+        RPLaunch now;
+        std::memset(&now, 0, sizeof now);
+        now.g = h->g;
+        now.bp = h->bp;
+        now.b = h->b;
+        if (!h->rpl_valid || std::memcmp(&now, h->rpl_h, sizeof now) != 0) {
+            HIPCHK(h, hipStreamSynchronize(s));
+            std::memcpy(h->rpl_h, &now, sizeof now);
+            HIPCHK(h, hipMemcpyAsync(h->rpl_d, h->rpl_h, sizeof now, hipMemcpyHostToDevice, s));
+            h->rpl_valid = true;
+        }
     }
     F *vx = (F *)h->vx, *vy = (F *)h->vy, *p0 = (F *)h->p0;
     const F *cxa = (const F *)h->cxa, *cxb = (const F *)h->cxb, *cya = (const F *)h->cya,
@@ -918,6 +933,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             h->pl_p = m;
         }
         StepRecord *rec = ctl ? ctl->rec : nullptr;
+        const bool blind = ctl && ctl->force_npic && ctl->tape_in && ctl->win;
         int forced = (ctl && ctl->force_npic) ? ctl->force_npic[step] : -1;
         if (h->sched_mode == 2) {
             if (h->sched_step >= h->sched->npic.size())
@@ -946,18 +962,30 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         launch_velocity<F>(s, h->g, vx, vy, p0, h->fgb[old_cur], h->W, h->first_step, cxa, cxb,
                            cya, cyb, h->sc_d);
         launch_velocity_ghosts<F>(s, h->g, vx, vy, h->t, h->sc_d, max_pic + 1);
-        if (bub) launch_motion<F>(s, h->g, h->bp, h->b, vx, vy, h->sc_d);
+        // a blind replay takes the positions after the motion from the tape
+        BubbleArrays bnow = h->b;
+        if (blind) {
+            bnow.x = ctl->tape_in->x_end;
+            bnow.y = ctl->tape_in->y_end;
+        } else if (bub) {
+            launch_motion<F>(s, h->g, h->bp, h->b, vx, vy, h->sc_d);
+        }
         launch_pressure_first<F>(s, h->g, vx, vy, (F *)h->pb[pn_i][0], (F *)h->pb[pn_i][1],
                                  (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0, h->fgb[old_cur],
                                  h->fgb[old_n], h->fgb[old_m], h->W, ax, bx, ay, by, h->xu_d,
                                  h->rxp_d, h->sc_d);
         launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, 0, nullptr, 0,
-                                  h->b.bbox_blk, bub ? (h->nb + 255) / 256 : 0, h->sc_d, h->rep,
-                                  ++h->rep_seq);
-        if (int rc = wait_report(h)) return rc;
-        double resimax = h->rep->resid / h->P_inf;
+                                  h->b.bbox_blk, bub && !blind ? (h->nb + 255) / 256 : 0, h->sc_d,
+                                  blind ? nullptr : h->rep, blind ? 0 : ++h->rep_seq);
+        double resimax = 0.0;
+        if (blind) {
+            h->W = *ctl->win;
+        } else {
+            if (int rc = wait_report(h)) return rc;
+            resimax = h->rep->resid / h->P_inf;
+        }
         st.resimax0 = resimax;
-        if (bub) {
+        if (bub && !blind) {
             window_union(h->W, h->rep->bbox[0], h->rep->bbox[1], h->rep->bbox[2], h->rep->bbox[3]);
             if (h->cfg.tr_cylindrical && h->W.i0 <= 1 && h->W.i0 <= h->W.i1) h->W.i0 = 0;  // axis fold target
         }
@@ -1000,7 +1028,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 }
                 int rp_waves = 0;  // wavefront records the launch leaves
                 if (tin) {  // replay: the void fraction from the taped radii, no RP
-                    launch_scatter_radii(s, h->g, h->bp, h->b, tin->Rt_it[loop], h->fgb[target], h->sc_d);
+                    launch_scatter_radii(s, h->g, h->bp, bnow, tin->Rt_it[loop], h->fgb[target], h->sc_d);
                 } else if (replay) {  // the recorded step sizes of this RP call
                     if (h->sched_call >= h->sched->calls.size())
                         return set_err(h, BRP_ERR_STATE, "step %lld: the frozen schedule has no "
@@ -1032,14 +1060,20 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                           (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0,
                                           h->fgb[target], h->fgb[old_cur], h->fgb[prev], h->W, ax,
                                           bx, ay, by, h->xu_d, h->rxp_d, h->sc_d, loop);
-                launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
-                                          h->b.totals, rp_waves, nullptr, 0, h->sc_d, h->rep,
-                                          ++h->rep_seq);
+                // blind: only where an iteration changes a ghost cell
+                if (!blind || !pressure_ghosts_fixed(h->g))
+                    launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
+                                              h->b.totals, rp_waves, nullptr, 0, h->sc_d,
+                                              blind ? nullptr : h->rep, blind ? 0 : ++h->rep_seq);
                 if (rec && rec->want_grid) {  // the iterate that the evaluation read, and its pressure
                     RectPlan rp;
                     rp.add(rec->fg_it[loop], h->fgb[target], sizeof(int64_t));
                     rp.add(rec->p0_it[loop], p0, sizeof(F));
                     launch_copy_rects(s, rp, rec->rect, h->pitch);
+                }
+                if (blind) {
+                    std::swap(target, prev);
+                    continue;
                 }
                 if (int rc = wait_report(h)) return rc;
                 resimax = h->rep->resid / h->P_inf;
@@ -1076,10 +1110,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         if (bub && loop == 0) launch_copy_d(s, h->b.PL[h->pl_p], h->b.PL[h->pl_n], h->nb);
         h->pc = p_i;
         h->first_step = 0;
-        if (h->cfg.thermal)
+        if (h->cfg.thermal && !blind)
             if (int rc = wait_report(h)) return rc;
-        for (int q = 0; q < 5; q++) h->phase_ms[q] += (double)h->rep->phase[q] * h->ms_per_tick;
-        const int flags = h->rep->flags;
+        if (!blind)
+            for (int q = 0; q < 5; q++) h->phase_ms[q] += (double)h->rep->phase[q] * h->ms_per_tick;
+        const int flags = blind ? 0 : h->rep->flags;
         if (status == BRP_OK && (flags & 3)) status = BRP_ERR_NONFINITE;
         if (status == BRP_OK && (flags & 4)) status = BRP_ERR_SUBSTEP_CAP;
         st.nstep = h->nstep;
@@ -1106,6 +1141,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             }
         }
         if (ctl && ctl->npic_out) ctl->npic_out->push_back(loop);
+        if (ctl && ctl->win_out) ctl->win_out->push_back(h->W);
+        if (blind) {
+            HIPCHK(h, hipGetLastError());
+            continue;
+        }
         if (h->sched_mode == 1) {
             h->sched->npic.push_back(loop);
             unsigned int mm = 0;
@@ -1158,7 +1198,7 @@ struct AdjState {
     double *LR[4] = {}, *LRs[4] = {};          // RP state adjoints: step end / start
     double *LA = nullptr, *LB = nullptr;       // PL history (PL_p, PL_n of the step end)
     double *Lx = nullptr, *Ly = nullptr;
-    double *lRt = nullptr, *lPLp = nullptr, *lPLn = nullptr, *lPLm = nullptr;
+    double *lPLn = nullptr, *lPLm = nullptr;
     unsigned int *mismatch = nullptr;  // RP replays whose sub-step count differed
     // RP Jacobians of a run of steps (k_adj_rp_jac): columns, iteration
     // descriptors, longest-first order and its bins and queue head
@@ -1188,23 +1228,9 @@ void adjoint_step(brp_handle *h, const StepRecord &rec, const StepRecord &brec, 
     const Window pw{rec.win.i0 - 2, rec.win.i1 + 2, rec.win.j0 - 2, rec.win.j1 + 2};
     const F *ax = (const F *)h->ax, *bx = (const F *)h->bx, *ay = (const F *)h->ay,
             *by = (const F *)h->by;
-    // the bubble arrays as the step saw them: positions after the motion, RP
-    // start state in slot 0, PL history in slots 0 (m) and 1 (n)
-    BubbleArrays bv = h->b;
-    bv.x = brec.x_end;
-    bv.y = brec.y_end;
-    bv.R[0] = brec.rp[0];
-    bv.Rn[0] = brec.rp[1];
-    bv.d1R[0] = brec.rp[2];
-    bv.PG[0] = brec.rp[3];
-    bv.bdt[0] = brec.rp[4];
-    bv.re[0] = brec.rp[5];
-    bv.PL[0] = brec.PLm;
-    bv.PL[1] = brec.PLn;
     if (seed) launch_adj_seed<F>(s, g, fr(rec.p0_it[n]), a.f.p0, box, cJ);
     // start-of-step f_g adjoints: f_gn' = f_g and f_gm' = f_gn of the start
     double *LgC = a.LfN, *LfNs = a.LfM, *LfMs = a.LfC;
-    double *const none[4] = {nullptr, nullptr, nullptr, nullptr};
     for (int k = n; k >= 1; k--) {
         launch_adj_pressure_ghosts(s, g, a.f.p0, h->el_amp_d, h->el_phase_d, rec.t, a.gA, a.gP);
         // before the step's last evaluation, the adjoint inputs are the gather
@@ -1212,34 +1238,32 @@ void adjoint_step(brp_handle *h, const StepRecord &rec, const StepRecord &brec, 
         // zero outside the window grown by the stencil's reach
         launch_adj_pressure<F>(s, g, false, a.f, gr(rec.fg_it[k]), gC, k == n ? a.LfC : nullptr, a.Lf,
                                LgC, nullptr, nullptr, ax, bx, ay, by, k == n ? nullptr : &pw);
-        launch_adj_scatter(s, g, h->bp, bv, brec.Rt_it[k], a.Lf, a.lRt, a.Lx, a.Ly);
-        launch_adj_rp_apply(s, bv.n, jac[k], a.lRt, k == n ? a.LR : none, a.LRs, a.lPLp, a.lPLn,
-                            a.lPLm);
-        launch_adj_gather<F>(s, g, h->bp, bv, fr(rec.p0_it[k - 1]), a.lPLp,
-                             k == n ? a.LA : nullptr, a.f.p0, a.Lx, a.Ly);
+        AdjBubble ab{brec.Rt_it[k], a.Lf, jac[k], {}, {}, a.lPLn, a.lPLm,
+                     k == n ? a.LA : nullptr, a.f.p0, a.Lx, a.Ly};
+        for (int q = 0; q < 4; q++) {
+            ab.LRe[q] = k == n ? a.LR[q] : nullptr;
+            ab.LRs[q] = a.LRs[q];
+        }
+        launch_adj_bubble<F>(s, g, h->bp, h->nb, brec.x_end, brec.y_end, h->b.n_B, ab,
+                             fr(rec.p0_it[k - 1]));
     }
     launch_adj_pressure_ghosts(s, g, a.f.p0, h->el_amp_d, h->el_phase_d, rec.t, a.gA, a.gP);
     launch_adj_pressure<F>(s, g, true, a.f, gr(rec.fg_it[0]), gC, n == 0 ? a.LfC : nullptr, nullptr,
                            LgC, LfNs, LfMs, ax, bx, ay, by, nullptr);
     if (bub)
         launch_adj_motion<F>(s, g, h->bp, h->nb, brec.x_start, brec.y_start, fr(rec.vx_end),
-                             fr(rec.vy_end), a.f.vx, a.f.vy, a.Lx, a.Ly);
+                             fr(rec.vy_end), a.f.vx, a.f.vy, a.Lx, a.Ly,
+                             AdjHistory{n > 0, a.LA, a.LB, a.lPLn, a.lPLm,
+                                        {a.LR[0], a.LR[1], a.LR[2], a.LR[3]}});
     launch_adj_velocity_ghosts(s, g, a.f.vx, a.f.vy);
     launch_adj_velocity<F>(s, g, a.f.vx, a.f.vy, (const F *)rec.p0_start, gC, rec.first,
                            (const F *)h->cxa, (const F *)h->cxb, (const F *)h->cya,
                            (const F *)h->cyb, a.f.p0, LgC);
-    if (bub) {
-        launch_adj_pl_history(s, h->nb, n > 0, a.LA, a.LB, a.lPLn, a.lPLm);
-        if (n > 0)
-            for (int q = 0; q < 4; q++) {
-                std::swap(a.LR[q], a.LRs[q]);
-                launch_fill_d(s, a.LRs[q], (size_t)h->nb, 0.0);
-            }
-    }
+    if (bub && n > 0)
+        for (int q = 0; q < 4; q++) std::swap(a.LR[q], a.LRs[q]);
+    // the first evaluation's transpose left zeros in px and py
     std::swap(a.f.px, a.f.pnx);
     std::swap(a.f.py, a.f.pny);
-    launch_fill_d(s, a.f.pnx, h->frame, 0.0);
-    launch_fill_d(s, a.f.pny, h->frame, 0.0);
     a.LfC = LgC;
     a.LfN = LfNs;
     a.LfM = LfMs;
@@ -1302,6 +1326,9 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
     npic.reserve(n);
     StepCtl fctl;
     fctl.npic_out = &npic;
+    std::vector<Window> wins;
+    wins.reserve(n);
+    fctl.win_out = &wins;
     for (int sg = 0; sg < nseg; sg++) {
         if ((rc = snap_save(h, ck[sg]))) return rc;
         const int s_end = std::min(n, (sg + 1) * K);
@@ -1329,7 +1356,7 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
     if ((rc = mem.get(h, &a.gA, (size_t)h->N + 2)) || (rc = mem.get(h, &a.gP, (size_t)h->N + 2)))
         return rc;
     double **bubs[] = {&a.LR[0], &a.LR[1], &a.LR[2], &a.LR[3], &a.LRs[0], &a.LRs[1], &a.LRs[2],
-                       &a.LRs[3], &a.LA, &a.LB, &a.Lx, &a.Ly, &a.lRt, &a.lPLp, &a.lPLn, &a.lPLm};
+                       &a.LRs[3], &a.LA, &a.LB, &a.Lx, &a.Ly, &a.lPLn, &a.lPLm};
     for (double **q : bubs)
         if ((rc = mem.get(h, q, nb))) return rc;
     if ((rc = mem.get(h, &a.mismatch, 1))) return rc;
@@ -1381,6 +1408,7 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
             c.force_npic = &npic[st - 1];
             c.rec = &recs[st - s0];
             c.tape_in = use_tape ? &tape[st - 1] : nullptr;
+            c.win = &wins[st - 1];
             if ((rc = run_steps<F>(h, 1, nullptr, &c))) return rc;
             if (recs[st - s0].n_pic != npic[st - 1])
                 return set_err(h, BRP_ERR_STATE, "replay of step %d took %d Picard iterations, not %d",

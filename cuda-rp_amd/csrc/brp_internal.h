@@ -104,7 +104,6 @@ struct StepScalars {
     unsigned long long sub_sum;          // sum of RP sub-steps this step
     unsigned int done;                   // bubbles written back by the RP kernel this step
     unsigned int reused;                 // of them, kept from the previous iteration
-    double focal[2];                     // (x, y) of the largest temperature increment
     // The step's phases in ticks of the device's constant-rate clock: marks
     // that kernels set, and the phases' sums (brp_get_phase_times' order).
     unsigned long long mark[kMarks], phase[5];
@@ -114,6 +113,19 @@ struct StepScalars {
 };
 
 #if defined(__HIPCC__)
+// One word of a report.  Report words bypass the caches, one by one: a release
+// at system scope would write back every dirty line of the XCD's L2 first.
+__device__ inline void report_word(unsigned long long *dst, unsigned long long v) {
+    __hip_atomic_store(dst, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The sequence number, after this wavefront's words have arrived.
+__device__ inline void report_seq(StepReport *rep, unsigned long long seq) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+    report_word(&rep->seq, seq);
+}
+
 // Sets a phase's mark (the kernel's first workgroup, one thread).  The store
 // is written out so that the compiler does not take it for one that may
 // change what the kernel reads through its other pointers: after it, uniform
@@ -125,6 +137,90 @@ __device__ inline void set_mark(StepScalars *sc, Mark m) {
         asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(&sc->mark[m]), "v"(now));
     }
 #endif
+}
+#endif
+
+#if defined(__HIPCC__)
+// FP64 contributions of a workgroup's bubble stencils (256 threads) to frame
+// arrays, summed in LDS tiles over the workgroup's bounding box and flushed
+// with one global atomic per touched cell: bubbles are cell-sorted, so a
+// workgroup's stencils cover a small patch, and in dense clouds (hundreds of
+// bubbles per cell) per-contribution global atomics on the same addresses
+// serialise.  A patch larger than `cap` cells falls back to global atomics
+// per contribution.  Every thread calls begin and flush (they synchronise);
+// `any` says whether the thread has a stencil, [i0, i1] x [j0, j1].  The box
+// is reduced by lane moves: atomics on its four corners run as loops over the
+// lanes.
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) double lds_double;
+#else
+typedef double lds_double;  // the host pass only parses kernel bodies
+#endif
+template <int TILES, int CAP>
+struct StencilTiles {
+    double t[TILES][CAP];
+    int red[4][4];
+};
+struct TileBox {
+    int i0, j0, w, h;  // w, h <= 0: no stencil
+    bool binned;
+};
+template <int TILES, int CAP>
+__device__ inline TileBox tiles_begin(StencilTiles<TILES, CAP> &s, bool any, int i0, int i1, int j0,
+                                      int j1) {
+    int lo_i = any ? i0 : 0x7fffffff, hi_i = any ? i1 : -0x7fffffff;
+    int lo_j = any ? j0 : 0x7fffffff, hi_j = any ? j1 : -0x7fffffff;
+    for (int off = 32; off > 0; off >>= 1) {
+        lo_i = min(lo_i, __shfl_xor(lo_i, off, 64));
+        hi_i = max(hi_i, __shfl_xor(hi_i, off, 64));
+        lo_j = min(lo_j, __shfl_xor(lo_j, off, 64));
+        hi_j = max(hi_j, __shfl_xor(hi_j, off, 64));
+    }
+    const int wv = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        s.red[wv][0] = lo_i;
+        s.red[wv][1] = hi_i;
+        s.red[wv][2] = lo_j;
+        s.red[wv][3] = hi_j;
+    }
+    __syncthreads();
+    for (int k = 0; k < 4; k++) {
+        lo_i = min(lo_i, s.red[k][0]);
+        hi_i = max(hi_i, s.red[k][1]);
+        lo_j = min(lo_j, s.red[k][2]);
+        hi_j = max(hi_j, s.red[k][3]);
+    }
+    TileBox b{lo_i, lo_j, 0, 0, false};
+    if (lo_i <= hi_i && lo_j <= hi_j) {
+        b.w = hi_i - lo_i + 1;
+        b.h = hi_j - lo_j + 1;
+        b.binned = (int64_t)b.w * b.h <= CAP;  // workgroup-uniform
+    }
+    if (b.binned)
+        for (int q = 0; q < TILES; q++)
+            for (int k = threadIdx.x; k < b.w * b.h; k += 256) s.t[q][k] = 0.0;
+    __syncthreads();
+    return b;
+}
+template <int TILES, int CAP>
+__device__ inline void tiles_add(StencilTiles<TILES, CAP> &s, int q, const TileBox &b, double *glob,
+                                 int pitch, int i, int j, double v) {
+    if (b.binned)
+        __hip_atomic_fetch_add((lds_double *)&s.t[q][(j - b.j0) * b.w + (i - b.i0)], v,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        atomicAdd(&glob[frame_off(i, j, pitch)], v);
+}
+template <int TILES, int CAP>
+__device__ inline void tiles_flush(StencilTiles<TILES, CAP> &s, const TileBox &b,
+                                   double *const (&glob)[TILES], int pitch) {
+    if (!b.binned) return;
+    __syncthreads();
+    for (int k = threadIdx.x; k < b.w * b.h; k += 256) {
+        const int64_t o = frame_off(b.i0 + k % b.w, b.j0 + k / b.w, pitch);
+        for (int q = 0; q < TILES; q++)
+            if (const double v = s.t[q][k]; v != 0.0) atomicAdd(&glob[q][o], v);
+    }
 }
 #endif
 
@@ -233,6 +329,12 @@ void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const dou
                             const double *el_phase, double t, int eval, const RPTotals *tot,
                             int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
                             StepReport *rep, unsigned long long seq);
+// Whether a Picard iteration's evaluation changes no ghost cell of p0: they
+// hold the source row, or nothing, and mirror no wall.
+inline bool pressure_ghosts_fixed(const GridParams &g) {
+    const bool source = g.src_row && (g.plane_p || g.focused_p);
+    return g.pml_x0 && g.pml_x1 && g.pml_y1 && (g.pml_y0 || source);
+}
 template <typename F>
 void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                    const BubbleArrays &b, const F *vx, const F *vy, StepScalars *sc);
@@ -393,17 +495,27 @@ template <typename F>
 void launch_adj_velocity(hipStream_t s, const GridParams &g, double *Lvx, double *Lvy,
                          const F *p0, Rect<int64_t> fgn, int first, const F *cxa, const F *cxb,
                          const F *cya, const F *cyb, double *Lp0, double *LfC);
-void launch_adj_scatter(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                        const BubbleArrays &b, const double *Rt, const double *Lf, double *lRt,
-                        double *Lx, double *Ly);
+// The adjoints that k_adj_bubble reads and adds to (see there).
+struct AdjBubble {
+    const double *Rt, *Lf, *jac;
+    const double *LRe[4];  // null before the step's last iteration
+    double *LRs[4], *lPLn, *lPLm;
+    const double *lPL_extra;
+    double *Lp0, *Lx, *Ly;
+};
+// What k_adj_motion carries across the step boundary (see there).
+struct AdjHistory {
+    int picard;
+    double *LA, *LB, *lPLn, *lPLm, *LR[4];
+};
 template <typename F>
-void launch_adj_gather(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                       const BubbleArrays &b, Rect<F> p0, const double *lPL,
-                       const double *lPL_extra, double *Lp0, double *Lx, double *Ly);
+void launch_adj_bubble(hipStream_t s, const GridParams &g, const BubbleParams &bp, int n,
+                       const double *x, const double *y, const double *n_B, const AdjBubble &A,
+                       Rect<F> p0);
 template <typename F>
 void launch_adj_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp, int n,
                        const double *xs, const double *ys, Rect<F> vx, Rect<F> vy, double *Lvx,
-                       double *Lvy, double *Lx, double *Ly);
+                       double *Lvy, double *Lx, double *Ly, const AdjHistory &H);
 // One Picard iteration of one step for the RP Jacobians of the reverse
 // sweep: the step's RP start state and pressure history, the iteration's
 // gathered pressure and the forward's sub-step counts (taped), and where its
@@ -430,12 +542,4 @@ void launch_adj_rp_jacobians(hipStream_t s, const BubbleParams &bp, const Bubble
 // and the reverse-mode state buffer a grid of `blocks` workgroups needs.
 int adj_rp_jac_per_cu();
 size_t adj_rp_jac_buf_doubles(int blocks);
-// The transpose of one iteration's RP map: LRe (the adjoint of the step's
-// final RP state) only for the last iteration, else null.
-void launch_adj_rp_apply(hipStream_t s, int nb, const double *jac, const double *lRt,
-                         double *const LRe[4], double *const LRs[4], double *lPLp, double *lPLn,
-                         double *lPLm);
-void launch_adj_pl_history(hipStream_t s, int n, int picard, double *LA, double *LB,
-                           double *lPLn, double *lPLm);
-void launch_fill_d(hipStream_t s, double *p, size_t n, double v);
 }  // namespace brp

@@ -8,11 +8,11 @@
 //   k_adj_pressure_ghosts / k_adj_velocity_ghosts   the boundary kernels,
 //                    their writes undone in reverse program order
 //   k_adj_velocity_a / _b   VelocityKernel
-//   k_adj_scatter / k_adj_gather / k_adj_motion   the bubble-grid coupling,
+//   k_adj_bubble / k_adj_motion   the bubble-grid coupling,
 //                    including the derivative of the smooth-delta weights with
 //                    respect to the bubble position (bins are piecewise
 //                    constant and not differentiated)
-//   k_adj_rp_jac / k_adj_rp_apply   Rayleigh-Plesset over one mixture step
+//   k_adj_rp_jac / k_adj_bubble   Rayleigh-Plesset over one mixture step
 //                    at the frozen sub-step schedule: Jacobian columns from
 //                    seven tangent lanes per bubble, then their transpose
 // Grid adjoints are FP64 in both precision modes; scatter-type transposes
@@ -32,13 +32,25 @@ constexpr int kAX = 64, kAY = 4;
 
 __device__ inline double fgd(int64_t v) { return (double)v * kFgInvScale; }
 
-__device__ inline double wdelta(double c, double k, int pos, double h, double b) {
-    return c * (1.0 + cos(k * (((double)pos - 0.5) * h - b)));
-}
-// d/db of wdelta
-__device__ inline double wdelta_db(double c, double k, int pos, double h, double b) {
-    return c * k * sin(k * (((double)pos - 0.5) * h - b));
-}
+// A stencil's nb weights along one axis and their derivatives, each cosine
+// and sine taken once (NB: nb, or the largest band where nb is only known at
+// run time).  With the weights of the inner axis taken again for every outer
+// one, the trigonometry of one bubble was the whole kernel's time where there
+// are few bubbles (1024: k_adj_motion 26 -> 8.4 us).
+template <int NB>
+struct AxisW {
+    double w[NB], d[NB];
+    __device__ AxisW(double c, double k, int first, int nb, double h, double b) {
+#pragma unroll
+        for (int a = 0; a < NB; a++) {
+            if (a >= nb) break;
+            double sn, cn;
+            sincos(k * (((double)(first + a) - 0.5) * h - b), &sn, &cn);
+            w[a] = c * (1.0 + cn);
+            d[a] = c * k * sn;
+        }
+    }
+};
 
 __device__ inline int bin_idx(double x, double rdx, double c) {
 #pragma clang fp contract(off)
@@ -353,153 +365,110 @@ __global__ void k_adj_velocity_b(GridParams g, double *Lvx, double *Lvy, const F
     if (i >= 1) Lvy[o] *= (double)cya[j + 1] / (double)cyb[j + 1];
 }
 
-// Adjoint of the scatter of iteration k: lRt = dJ/dR_t, and the position
-// adjoints of the weights.
-__global__ __launch_bounds__(256) void k_adj_scatter(GridParams g, BubbleParams bp,
-                                                      BubbleArrays b, const double *Rt,
-                                                      const double *__restrict__ Lf, double *lRt,
-                                                      double *Lx, double *Ly) {
+// The bubble side of Picard iteration k, reversed, one bubble per thread:
+//   the scatter of R_t (Lf: the void-fraction adjoint): dJ/dR_t and the
+//     position adjoints of the weights;
+//   the RP map by its Jacobian columns (k_adj_rp_jac; 35 with the adjoints
+//     LRe of the step's final RP state, in its last iteration, else 7) into the
+//     adjoints of the step's start state and pressure history;
+//   the gather PL_p = sum p0 w (p0: the previous evaluation's pressure, lPL_extra:
+//     the history's adjoint of PL_p): FP64 sums into Lp0 through the
+//     workgroup's tile, position adjoints.
+// One launch instead of three (1024 bubbles: 23.9 -> 9.2 us of kernels an iteration,
+// with the tile's box reduced by lane moves).
+template <typename F, int NB>
+__global__ __launch_bounds__(256) void k_adj_bubble(GridParams g, BubbleParams bp, int n,
+                                                     const double *xs, const double *ys,
+                                                     const double *n_B, AdjBubble A, Rect<F> p0) {
+    __shared__ StencilTiles<1, 4096> tiles;
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= b.n) return;
-    const double x = b.x[idx], y = b.y[idx], R = Rt[idx];
+    const bool valid = idx < n;
+    const int nb = NB == 2 ? 2 : bp.mbe - bp.mbs + 1;
+    const double x = valid ? xs[idx] : 0.0, y = valid ? ys[idx] : 0.0;
     const int ibnx = bin_idx(x, g.rdx, 0.5), ibny = bin_idx(y, g.rdy, 0.5);
-    const int nb = bp.mbe - bp.mbs + 1;
-    double s = 0.0, sx = 0.0, sy = 0.0;
-    for (int a = 0; a < nb; a++) {
-        const int i = ibnx + bp.mbs + a;
-        const double wx = wdelta(bp.dcx, bp.dcy, i, g.dx, x);
-        const double dwx = wdelta_db(bp.dcx, bp.dcy, i, g.dx, x);
-        for (int c = 0; c < nb; c++) {
-            const int j = ibny + bp.mbs + c;
-            if (i >= 0 && i <= g.N + 1 && j >= 0 && j <= g.M + 1) {
-                const double wy = wdelta(bp.dcx, bp.dcz, j, g.dy, y);
-                const double dwy = wdelta_db(bp.dcx, bp.dcz, j, g.dy, y);
-                const double l = Lf[frame_off(i, j, g.pitch)];
-                s += l * wx * wy;
-                sx += l * dwx * wy;
-                sy += l * wx * dwy;
-            }
-        }
-    }
-    const double base = bp.pi4r3 * b.n_B[idx] * g.rdx * g.rdy;  // fg_temp = base R^3
-    lRt[idx] = s * 3.0 * base * R * R;
-    const double ft = base * R * R * R;
-    Lx[idx] += ft * sx;
-    Ly[idx] += ft * sy;
-}
-
-// FP64 contributions of a workgroup's bubble stencils to a frame array,
-// summed in an LDS tile over the workgroup's bounding box and flushed with
-// one global atomic per touched cell: bubbles are cell-sorted, so a
-// workgroup's stencils cover a small patch, and in dense clouds (hundreds
-// of bubbles per cell) per-contribution global atomics on the same
-// addresses serialise.  A patch larger than the tile falls back to global
-// atomics per contribution.  Every thread of the workgroup calls begin and
-// end (they synchronise); `any` says whether the thread has a stencil.
-constexpr int kAdjTile = 4096;  // cells (32 KB of LDS)
-struct TileAcc {
-    double *tile;
-    int bx0, by0, bw;
-    bool binned;
-};
-__device__ inline TileAcc tile_begin(double *tile, int *box, bool any, int i0, int i1, int j0,
-                                     int j1) {
-    __syncthreads();  // the previous use of box / tile has finished
-    if (threadIdx.x == 0) {
-        box[0] = 0x7fffffff;
-        box[1] = -0x7fffffff;
-        box[2] = 0x7fffffff;
-        box[3] = -0x7fffffff;
-    }
-    __syncthreads();
-    if (any) {
-        atomicMin(&box[0], i0);
-        atomicMax(&box[1], i1);
-        atomicMin(&box[2], j0);
-        atomicMax(&box[3], j1);
-    }
-    __syncthreads();
-    TileAcc t{tile, box[0], box[2], box[1] - box[0] + 1, false};
-    const int bh = box[3] - box[2] + 1;
-    t.binned = t.bw > 0 && bh > 0 && (int64_t)t.bw * bh <= kAdjTile;  // workgroup-uniform
-    if (t.binned) {
-        for (int k = threadIdx.x; k < t.bw * bh; k += blockDim.x) tile[k] = 0.0;
-        __syncthreads();
-    }
-    return t;
-}
-__device__ inline void tile_add(const TileAcc &t, double *glob, int pitch, int i, int j, double v) {
-    if (t.binned)
-        atomicAdd(&t.tile[(j - t.by0) * t.bw + (i - t.bx0)], v);
-    else
-        atomicAdd(&glob[frame_off(i, j, pitch)], v);
-}
-__device__ inline void tile_end(const TileAcc &t, const int *box, double *glob, int pitch) {
-    if (!t.binned) return;
-    __syncthreads();
-    const int n = t.bw * (box[3] - box[2] + 1);
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        const double v = t.tile[k];
-        if (v != 0.0) atomicAdd(&glob[frame_off(t.bx0 + k % t.bw, t.by0 + k / t.bw, pitch)], v);
-    }
-}
-
-// Adjoint of the gather PL_p = sum p0 w of iteration k (p0 = the previous
-// evaluation's pressure): FP64 atomics into Lp0 (through the workgroup's
-// LDS tile), position adjoints.
-template <typename F>
-__global__ __launch_bounds__(256) void k_adj_gather(GridParams g, BubbleParams bp,
-                                                     BubbleArrays b, Rect<F> p0,
-                                                     const double *lPL, const double *lPL_extra,
-                                                     double *Lp0, double *Lx, double *Ly) {
-    __shared__ double tile[kAdjTile];
-    __shared__ int box[4];
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = idx < b.n;
-    double lam = 0.0, x = 0.0, y = 0.0;
-    int ibnx = 0, ibny = 0;
-    if (valid) {
-        lam = lPL[idx] + (lPL_extra ? lPL_extra[idx] : 0.0);
-        x = b.x[idx];
-        y = b.y[idx];
-        ibnx = bin_idx(x, g.rdx, 0.5);
-        ibny = bin_idx(y, g.rdy, 0.5);
-    }
+    const AxisW<NB> X(bp.dcx, bp.dcy, ibnx + bp.mbs, nb, g.dx, x);
+    const AxisW<NB> Y(bp.dcx, bp.dcz, ibny + bp.mbs, nb, g.dy, y);
     const int i0 = max(ibnx + bp.mbs, 0), i1 = min(ibnx + bp.mbe, g.N + 1);
     const int j0 = max(ibny + bp.mbs, 0), j1 = min(ibny + bp.mbe, g.M + 1);
-    const bool any = valid && lam != 0.0 && i0 <= i1 && j0 <= j1;
-    const TileAcc t = tile_begin(tile, box, any, i0, i1, j0, j1);
-    double sx = 0.0, sy = 0.0;
+    double lx = 0.0, ly = 0.0, lam4 = 0.0;
     if (valid) {
-        for (int i = i0; i <= i1; i++) {
-            const double wx = wdelta(bp.dcx, bp.dcy, i, g.dx, x);
-            const double dwx = wdelta_db(bp.dcx, bp.dcy, i, g.dx, x);
-            for (int j = j0; j <= j1; j++) {
-                const double wy = wdelta(bp.dcx, bp.dcz, j, g.dy, y);
-                const double dwy = wdelta_db(bp.dcx, bp.dcz, j, g.dy, y);
-                if (any) tile_add(t, Lp0, g.pitch, i, j, lam * wx * wy);
-                const double p = (double)p0.at(i, j);
-                sx += p * dwx * wy;
-                sy += p * wx * dwy;
+        double s = 0.0, sx = 0.0, sy = 0.0;
+#pragma unroll
+        for (int a = 0; a < NB; a++) {
+#pragma unroll
+            for (int c = 0; c < NB; c++) {
+                const int i = ibnx + bp.mbs + a, j = ibny + bp.mbs + c;
+                if (a >= nb || c >= nb || i < i0 || i > i1 || j < j0 || j > j1) continue;
+                const double l = A.Lf[frame_off(i, j, g.pitch)];
+                s += l * X.w[a] * Y.w[c];
+                sx += l * X.d[a] * Y.w[c];
+                sy += l * X.w[a] * Y.d[c];
             }
         }
-        Lx[idx] += lam * sx;
-        Ly[idx] += lam * sy;
+        const double R = A.Rt[idx];
+        const double base = bp.pi4r3 * n_B[idx] * g.rdx * g.rdy;  // fg_temp = base R^3
+        const double lr = s * 3.0 * base * R * R;                  // dJ/dR_t
+        const double ft = base * R * R * R;
+        lx = A.Lx[idx] + ft * sx;
+        ly = A.Ly[idx] + ft * sy;
+        const double *J = A.jac + idx;
+        const size_t m = (size_t)n;
+        double lam[7];
+#pragma unroll
+        for (int d = 0; d < 7; d++) lam[d] = lr * J[d * m];
+        if (A.LRe[0]) {
+            const double e0 = A.LRe[0][idx], e1 = A.LRe[1][idx], e2 = A.LRe[2][idx],
+                         e3 = A.LRe[3][idx];
+#pragma unroll
+            for (int d = 0; d < 7; d++)
+                lam[d] += e0 * J[(7 + d) * m] + e1 * J[(14 + d) * m] + e2 * J[(21 + d) * m] +
+                          e3 * J[(28 + d) * m];
+        }
+#pragma unroll
+        for (int d = 0; d < 4; d++) A.LRs[d][idx] += lam[d];
+        A.lPLn[idx] += lam[5];
+        A.lPLm[idx] += lam[6];
+        lam4 = lam[4] + (A.lPL_extra ? A.lPL_extra[idx] : 0.0);
     }
-    tile_end(t, box, Lp0, g.pitch);
+    const bool any = valid && lam4 != 0.0 && i0 <= i1 && j0 <= j1;
+    const TileBox t = tiles_begin(tiles, any, i0, i1, j0, j1);
+    if (valid) {
+        double sx = 0.0, sy = 0.0;
+#pragma unroll
+        for (int a = 0; a < NB; a++) {
+#pragma unroll
+            for (int c = 0; c < NB; c++) {
+                const int i = ibnx + bp.mbs + a, j = ibny + bp.mbs + c;
+                if (a >= nb || c >= nb || i < i0 || i > i1 || j < j0 || j > j1) continue;
+                if (any) tiles_add(tiles, 0, t, A.Lp0, g.pitch, i, j, lam4 * X.w[a] * Y.w[c]);
+                const double p = (double)p0.at(i, j);
+                sx += p * X.d[a] * Y.w[c];
+                sy += p * X.w[a] * Y.d[c];
+            }
+        }
+        A.Lx[idx] = lx + lam4 * sx;
+        A.Ly[idx] = ly + lam4 * sy;
+    }
+    double *const glob[1] = {A.Lp0};
+    tiles_flush(tiles, t, glob, g.pitch);
 }
 
 // Adjoint of k_motion: x' = x + dt vLx(x, y; vx), y' = y + dt vLy(x, y; vy)
 // at the step's start positions (xs, ys); Lx, Ly hold dJ/dx', dJ/dy' and
 // become dJ/dx, dJ/dy.  The node adjoints Lvx, Lvy are summed through the
-// workgroup's LDS tile, one array after the other.
-template <typename F>
+// workgroup's LDS tiles, both in one pass.  Also carries the liquid-pressure
+// history's adjoints across the step boundary:
+//   Picard ran:  LA <- lPLn + LB,  LB <- lPLm, and the RP adjoints of the step's
+//                end, LR, were consumed: zeros, for the step before to
+//                accumulate in (they become its start's after a swap)
+//   no Picard:   LA <- LA + LB,    LB <- 0        (PL_p was copied from PL_n)
+template <typename F, int NB>
 __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams bp, int n,
                                                      const double *xs, const double *ys,
                                                      Rect<F> vx, Rect<F> vy, double *Lvx,
-                                                     double *Lvy, double *Lx, double *Ly) {
-    __shared__ double tile[kAdjTile];
-    __shared__ int box[4];
+                                                     double *Lvy, double *Lx, double *Ly,
+                                                     AdjHistory H) {
+    __shared__ StencilTiles<2, 2048> tiles;  // vx and vy nodes
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = idx < n;
     double x = 0.0, y = 0.0, lx = 0.0, ly = 0.0;
@@ -515,50 +484,67 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
         ibnx = bin_idx(x, g.rdx, 0.5);
         ibny = bin_idx(y, g.rdy, 0.5);
     }
+    const int nb = NB == 2 ? 2 : bp.mbe - bp.mbs + 1;
+    const AxisW<NB> Xm(bp.dcx, bp.dcy, ibmx + bp.nbs, nb, g.dx, x);
+    const AxisW<NB> Yn(bp.dcx, bp.dcz, ibny + bp.mbs, nb, g.dy, y);
+    const AxisW<NB> Xn(bp.dcx, bp.dcy, ibnx + bp.mbs, nb, g.dx, x);
+    const AxisW<NB> Ym(bp.dcx, bp.dcz, ibmy + bp.nbs, nb, g.dy, y);
     double dvx_dx = 0.0, dvx_dy = 0.0, dvy_dx = 0.0, dvy_dy = 0.0;
-    {  // vx nodes: columns ibm + [nbs, nbe] in [-1, N+1], rows ibn + [mbs, mbe] in [0, M+1]
-        const int i0 = max(ibmx + bp.nbs, -1), i1 = min(ibmx + bp.nbe, g.N + 1);
-        const int j0 = max(ibny + bp.mbs, 0), j1 = min(ibny + bp.mbe, g.M + 1);
-        const bool any = valid && lx != 0.0 && i0 <= i1 && j0 <= j1;
-        const TileAcc t = tile_begin(tile, box, any, i0, i1, j0, j1);
-        if (valid)
-            for (int i = i0; i <= i1; i++) {
-                const double Dx = wdelta(bp.dcx, bp.dcy, i, g.dx, x);
-                const double dDx = wdelta_db(bp.dcx, bp.dcy, i, g.dx, x);
-                for (int j = j0; j <= j1; j++) {
-                    const double Dy = wdelta(bp.dcx, bp.dcz, j, g.dy, y);
-                    const double dDy = wdelta_db(bp.dcx, bp.dcz, j, g.dy, y);
-                    if (any) tile_add(t, Lvx, g.pitch, i, j, dt * lx * Dx * Dy);
+    // vx nodes: columns ibm + [nbs, nbe] in [-1, N+1], rows ibn + [mbs, mbe] in
+    // [0, M+1]; vy nodes: columns ibn + [mbs, mbe] in [0, N+1], rows ibm +
+    // [nbs, nbe] in [-1, M+1]
+    const int xi0 = max(ibmx + bp.nbs, -1), xi1 = min(ibmx + bp.nbe, g.N + 1);
+    const int xj0 = max(ibny + bp.mbs, 0), xj1 = min(ibny + bp.mbe, g.M + 1);
+    const int yi0 = max(ibnx + bp.mbs, 0), yi1 = min(ibnx + bp.mbe, g.N + 1);
+    const int yj0 = max(ibmy + bp.nbs, -1), yj1 = min(ibmy + bp.nbe, g.M + 1);
+    const bool any_x = valid && lx != 0.0 && xi0 <= xi1 && xj0 <= xj1;
+    const bool any_y = valid && ly != 0.0 && yi0 <= yi1 && yj0 <= yj1;
+    const int big = 0x7fffffff;
+    const TileBox t =
+        tiles_begin(tiles, any_x || any_y, min(any_x ? xi0 : big, any_y ? yi0 : big),
+                    max(any_x ? xi1 : -big, any_y ? yi1 : -big),
+                    min(any_x ? xj0 : big, any_y ? yj0 : big),
+                    max(any_x ? xj1 : -big, any_y ? yj1 : -big));
+    if (valid) {
+#pragma unroll
+        for (int a = 0; a < NB; a++) {
+#pragma unroll
+            for (int c = 0; c < NB; c++) {
+                if (a >= nb || c >= nb) continue;
+                const int i = ibmx + bp.nbs + a, j = ibny + bp.mbs + c;
+                if (i >= xi0 && i <= xi1 && j >= xj0 && j <= xj1) {
+                    if (any_x) tiles_add(tiles, 0, t, Lvx, g.pitch, i, j, dt * lx * Xm.w[a] * Yn.w[c]);
                     const double v = (double)vx.at(i, j);
-                    dvx_dx += v * dDx * Dy;
-                    dvx_dy += v * Dx * dDy;
+                    dvx_dx += v * Xm.d[a] * Yn.w[c];
+                    dvx_dy += v * Xm.w[a] * Yn.d[c];
+                }
+                const int k = ibnx + bp.mbs + a, l = ibmy + bp.nbs + c;
+                if (k >= yi0 && k <= yi1 && l >= yj0 && l <= yj1) {
+                    if (any_y) tiles_add(tiles, 1, t, Lvy, g.pitch, k, l, dt * ly * Xn.w[a] * Ym.w[c]);
+                    const double v = (double)vy.at(k, l);
+                    dvy_dx += v * Xn.d[a] * Ym.w[c];
+                    dvy_dy += v * Xn.w[a] * Ym.d[c];
                 }
             }
-        tile_end(t, box, Lvx, g.pitch);
+        }
     }
-    {  // vy nodes: columns ibn + [mbs, mbe] in [0, N+1], rows ibm + [nbs, nbe] in [-1, M+1]
-        const int i0 = max(ibnx + bp.mbs, 0), i1 = min(ibnx + bp.mbe, g.N + 1);
-        const int j0 = max(ibmy + bp.nbs, -1), j1 = min(ibmy + bp.nbe, g.M + 1);
-        const bool any = valid && ly != 0.0 && i0 <= i1 && j0 <= j1;
-        const TileAcc t = tile_begin(tile, box, any, i0, i1, j0, j1);
-        if (valid)
-            for (int i = i0; i <= i1; i++) {
-                const double Dx = wdelta(bp.dcx, bp.dcy, i, g.dx, x);
-                const double dDx = wdelta_db(bp.dcx, bp.dcy, i, g.dx, x);
-                for (int j = j0; j <= j1; j++) {
-                    const double Dy = wdelta(bp.dcx, bp.dcz, j, g.dy, y);
-                    const double dDy = wdelta_db(bp.dcx, bp.dcz, j, g.dy, y);
-                    if (any) tile_add(t, Lvy, g.pitch, i, j, dt * ly * Dx * Dy);
-                    const double v = (double)vy.at(i, j);
-                    dvy_dx += v * dDx * Dy;
-                    dvy_dy += v * Dx * dDy;
-                }
-            }
-        tile_end(t, box, Lvy, g.pitch);
-    }
+    double *const glob[2] = {Lvx, Lvy};
+    tiles_flush(tiles, t, glob, g.pitch);
     if (valid) {
         Lx[idx] = lx + dt * (lx * dvx_dx + ly * dvy_dx);
         Ly[idx] = ly + dt * (lx * dvx_dy + ly * dvy_dy);
+        const double lb = H.LB[idx];
+        if (H.picard) {
+            H.LA[idx] = H.lPLn[idx] + lb;
+            H.LB[idx] = H.lPLm[idx];
+#pragma unroll
+            for (int q = 0; q < 4; q++) H.LR[q][idx] = 0.0;
+        } else {
+            H.LA[idx] += lb;
+            H.LB[idx] = 0.0;
+        }
+        H.lPLn[idx] = 0.0;
+        H.lPLm[idx] = 0.0;
     }
 }
 
@@ -568,7 +554,7 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
 // its Jacobian is computed for every Picard iteration of a run of steps in
 // one launch (k_adj_rp_jac, after the items are ordered by k_jac_rank), and
 // each reverse step applies its transpose to the step's adjoints
-// (k_adj_rp_apply).  Without it every iteration's integration would be a
+// (k_adj_bubble).  Without it every iteration's integration would be a
 // launch of its own, bounded by that iteration's longest chain.
 
 // Keys of the item order (k_jac_rank): first the items of more than
@@ -768,62 +754,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// Transpose of one Picard iteration's RP map applied to its adjoints:
-//   lam_d = lRt dR_t/dIn_d (+ sum_o LRe_o dOut_o/dIn_d in the last iteration)
-// then LRs[d] += lam_d (d < 4), lPLp = lam_4, lPLn += lam_5, lPLm += lam_6.
-__global__ __launch_bounds__(256) void k_adj_rp_apply(int nb, const double *jac, const double *lRt,
-                                                       const double *LRe0, const double *LRe1,
-                                                       const double *LRe2, const double *LRe3,
-                                                       double *LRs0, double *LRs1, double *LRs2,
-                                                       double *LRs3, double *lPLp, double *lPLn,
-                                                       double *lPLm) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nb) return;
-    const double *J = jac + idx;
-    const size_t n = (size_t)nb;
-    const double lr = lRt[idx];
-    double lam[7];
-#pragma unroll
-    for (int d = 0; d < 7; d++) lam[d] = lr * J[d * n];
-    if (LRe0) {
-        const double e0 = LRe0[idx], e1 = LRe1[idx], e2 = LRe2[idx], e3 = LRe3[idx];
-#pragma unroll
-        for (int d = 0; d < 7; d++)
-            lam[d] += e0 * J[(7 + d) * n] + e1 * J[(14 + d) * n] + e2 * J[(21 + d) * n] +
-                      e3 * J[(28 + d) * n];
-    }
-    LRs0[idx] += lam[0];
-    LRs1[idx] += lam[1];
-    LRs2[idx] += lam[2];
-    LRs3[idx] += lam[3];
-    lPLp[idx] = lam[4];
-    lPLn[idx] += lam[5];
-    lPLm[idx] += lam[6];
-}
-
-// Liquid-pressure history adjoints across the step boundary:
-//   Picard ran:  LA <- lPLn + LB,  LB <- lPLm
-//   no Picard:   LA <- LA + LB,    LB <- 0        (PL_p was copied from PL_n)
-__global__ void k_adj_pl_history(int n, int picard, double *LA, double *LB, double *lPLn,
-                                 double *lPLm) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n) return;
-    if (picard) {
-        LA[idx] = lPLn[idx] + LB[idx];
-        LB[idx] = lPLm[idx];
-    } else {
-        LA[idx] = LA[idx] + LB[idx];
-        LB[idx] = 0.0;
-    }
-    lPLn[idx] = 0.0;
-    lPLm[idx] = 0.0;
-}
-
-__global__ void k_fill_d(double *p, size_t n, double v) {
-    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) p[k] = v;
-}
-
 __global__ void k_fill_i(int *p, int n) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) p[k] = 0;
@@ -897,30 +827,26 @@ void launch_adj_velocity(hipStream_t s, const GridParams &g, double *Lvx, double
     hipLaunchKernelGGL(k_adj_velocity_b<F>, gb, blk, 0, s, g, Lvx, Lvy, cxa, cxb, cya, cyb);
 }
 
-void launch_adj_scatter(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                        const BubbleArrays &b, const double *Rt, const double *Lf, double *lRt,
-                        double *Lx, double *Ly) {
-    if (b.n <= 0) return;
-    hipLaunchKernelGGL(k_adj_scatter, dim3((b.n + 255) / 256), dim3(256), 0, s, g, bp, b, Rt, Lf,
-                       lRt, Lx, Ly);
-}
+constexpr int kAdjBand = 8;  // the largest smooth_delta_band (checked at set-up)
+static bool band2(const BubbleParams &bp) { return bp.mbe - bp.mbs + 1 == 2; }
 
 template <typename F>
-void launch_adj_gather(hipStream_t s, const GridParams &g, const BubbleParams &bp,
-                       const BubbleArrays &b, Rect<F> p0, const double *lPL,
-                       const double *lPL_extra, double *Lp0, double *Lx, double *Ly) {
-    if (b.n <= 0) return;
-    hipLaunchKernelGGL(k_adj_gather<F>, dim3((b.n + 255) / 256), dim3(256), 0, s, g, bp, b, p0,
-                       lPL, lPL_extra, Lp0, Lx, Ly);
+void launch_adj_bubble(hipStream_t s, const GridParams &g, const BubbleParams &bp, int n,
+                       const double *x, const double *y, const double *n_B, const AdjBubble &A,
+                       Rect<F> p0) {
+    if (n <= 0) return;
+    const auto k = band2(bp) ? k_adj_bubble<F, 2> : k_adj_bubble<F, kAdjBand>;
+    hipLaunchKernelGGL(k, dim3((n + 255) / 256), dim3(256), 0, s, g, bp, n, x, y, n_B, A, p0);
 }
 
 template <typename F>
 void launch_adj_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp, int n,
                        const double *xs, const double *ys, Rect<F> vx, Rect<F> vy, double *Lvx,
-                       double *Lvy, double *Lx, double *Ly) {
+                       double *Lvy, double *Lx, double *Ly, const AdjHistory &H) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_adj_motion<F>, dim3((n + 255) / 256), dim3(256), 0, s, g, bp, n, xs, ys,
-                       vx, vy, Lvx, Lvy, Lx, Ly);
+    const auto k = band2(bp) ? k_adj_motion<F, 2> : k_adj_motion<F, kAdjBand>;
+    hipLaunchKernelGGL(k, dim3((n + 255) / 256), dim3(256), 0, s, g, bp, n, xs, ys, vx, vy, Lvx, Lvy,
+                       Lx, Ly, H);
 }
 
 size_t adj_rp_jac_buf_doubles(int blocks) {
@@ -955,27 +881,6 @@ void launch_adj_rp_jacobians(hipStream_t s, const BubbleParams &bp, const Bubble
                        ord, n_items, bins, head, mismatch, buf);
 }
 
-void launch_adj_rp_apply(hipStream_t s, int nb, const double *jac, const double *lRt,
-                         double *const LRe[4], double *const LRs[4], double *lPLp, double *lPLn,
-                         double *lPLm) {
-    if (nb <= 0) return;
-    hipLaunchKernelGGL(k_adj_rp_apply, dim3((nb + 255) / 256), dim3(256), 0, s, nb, jac, lRt,
-                       LRe[0], LRe[1], LRe[2], LRe[3], LRs[0], LRs[1], LRs[2], LRs[3], lPLp, lPLn,
-                       lPLm);
-}
-
-void launch_adj_pl_history(hipStream_t s, int n, int picard, double *LA, double *LB,
-                           double *lPLn, double *lPLm) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_adj_pl_history, dim3((n + 255) / 256), dim3(256), 0, s, n, picard, LA, LB,
-                       lPLn, lPLm);
-}
-
-void launch_fill_d(hipStream_t s, double *p, size_t n, double v) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_fill_d, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
-}
-
 #define BRP_ADJ_INSTANTIATE(F)                                                                  \
     template void launch_box_sumsq<F>(hipStream_t, const GridParams &, const F *, const int[4], \
                                       double *);                                                \
@@ -988,12 +893,13 @@ void launch_fill_d(hipStream_t s, double *p, size_t n, double v) {
     template void launch_adj_velocity<F>(hipStream_t, const GridParams &, double *, double *,   \
                                          const F *, Rect<int64_t>, int, const F *, const F *,   \
                                          const F *, const F *, double *, double *);             \
-    template void launch_adj_gather<F>(hipStream_t, const GridParams &, const BubbleParams &,   \
-                                       const BubbleArrays &, Rect<F>, const double *,           \
-                                       const double *, double *, double *, double *);           \
+    template void launch_adj_bubble<F>(hipStream_t, const GridParams &, const BubbleParams &, int, \
+                                       const double *, const double *, const double *,         \
+                                       const AdjBubble &, Rect<F>);                             \
     template void launch_adj_motion<F>(hipStream_t, const GridParams &, const BubbleParams &,   \
                                        int, const double *, const double *, Rect<F>, Rect<F>,   \
-                                       double *, double *, double *, double *);
+                                       double *, double *, double *, double *,                  \
+                                       const AdjHistory &);
 BRP_ADJ_INSTANTIATE(float)
 BRP_ADJ_INSTANTIATE(double)
 

@@ -9,6 +9,7 @@
 #include "brp_internal.h"
 
 #include <math.h>
+#include <stddef.h>
 
 #include <algorithm>
 
@@ -658,6 +659,8 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             if (!g.pml_x0) p0[frame_off(0, j, P)] = p0[frame_off(1, j, P)];
             if (!g.pml_x1) p0[frame_off(N + 1, j, P)] = p0[frame_off(N, j, P)];
         }
+    if (!rep) return;  // nobody waits
+    __shared__ StepReport out;
     if (tid == 0) {
         const unsigned long long *m = sc->mark;
         unsigned long long ph[5];
@@ -674,16 +677,23 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             ph[3] += p - m[kMarkRP];
             ph[2] += now - p;
         }
+        out.resid = __longlong_as_double((long long)sc->resid[eval]);
+        for (int k = 0; k < 4; k++) out.bbox[k] = sc->bbox[k];
+        out.flags = sc->flags;
+        out.sub_max = sc->sub_max;
+        out.sub_sum = sc->sub_sum;
+        out.done = sc->done;
+        out.reused = sc->reused;
+        for (int k = 0; k < 5; k++) out.phase[k] = sc->phase[k] = ph[k];
         sc->mark[kMarkQueue] = 0ull;
-        rep->resid = __longlong_as_double((long long)sc->resid[eval]);
-        for (int k = 0; k < 4; k++) rep->bbox[k] = sc->bbox[k];
-        rep->flags = sc->flags;
-        rep->sub_max = sc->sub_max;
-        rep->sub_sum = sc->sub_sum;
-        rep->done = sc->done;
-        rep->reused = sc->reused;
-        for (int k = 0; k < 5; k++) rep->phase[k] = sc->phase[k] = ph[k];
-        __hip_atomic_store(&rep->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+    constexpr int words = offsetof(StepReport, focal) / 8;
+    static_assert(words <= 64 && offsetof(StepReport, focal) % 8 == 0, "one wavefront's words");
+    if (tid < 64) {
+        if (tid < words)
+            report_word((unsigned long long *)rep + tid, ((const unsigned long long *)&out)[tid]);
+        if (tid == 0) report_seq(rep, seq);
     }
 }
 
