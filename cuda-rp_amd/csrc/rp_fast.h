@@ -144,10 +144,12 @@ struct cx_d {
 // k = floor(8 s), t = 16 s - (2k + 1), Horner in t for the real and
 // imaginary parts (two independent chains); with dpr/dpi also d/ds.
 __device__ inline cx_d v_poly(double s, const double *ftab, double *dpr = nullptr,
-                              double *dpi = nullptr) {
+                              double *dpi = nullptr, double *outside = nullptr) {
     static_assert(kVPerUnit == 8, "t below scales s by 2^4");
-    const int k = max(0, min((int)ldexp(s, 3), kVIntervals - 1));
-    const double t = ldexp(s, 4) - (2.0 * k + 1.0);  // exact product, one rounding
+    // (outside: interval 0 is left out, and |t| > 1 beyond either end)
+    const int k = max(outside ? 1 : 0, min((int)ldexp(s, 3), kVIntervals - 1));
+    const double t = fma(16.0, s, -(2.0 * k + 1.0));
+    if (outside) *outside = fmax(*outside, fabs(t));
     ldouble *c = (ldouble *)ftab + k * (2 * (kVDegree + 1));
     double cr[kVDegree + 1], ci[kVDegree + 1];
 #pragma unroll
@@ -229,28 +231,32 @@ __device__ inline bool cond(bool c) {
 // s = 20 (k3 is the simulation's; the table was built for it); beyond it
 // coth alpha = 1 to below an ulp, so U = (alpha - 1) / alpha^2 =
 // (is / 2) (1 + i (is - 1)).
-template <typename T, bool UNI = false>
+template <typename T>
+__device__ inline cx<T> v_of_u(cx<T> u, double k3) {
+    const T dr = fma_(T(k3), u.re, T(1.0)), di = k3 * u.im;
+    const T f = rcp_(fma_(dr, dr, di * di));
+    return cx<T>{dr * f, di * f};
+}
+template <typename T>
+__device__ inline cx<T> upsilon_far(T is, double k3) {
+    const T h = 0.5 * is;
+    return v_of_u(cx<T>{h, h * (is - T(1.0))}, k3);
+}
+template <typename T>
 __device__ inline cx<T> upsilon_g(T s, T is, double k3, const double *vtab) {
-    cx<T> v;
-    const bool far = cond<UNI>(val(s) > 20.0), small = cond<UNI>(small_alpha(s));
-    if (!far && !small) {  // the table
-        v = v_table(s, vtab);
-    } else {
-        cx<T> u;
-        if (far) {
-            const T h = 0.5 * is;
-            u = cx<T>{h, h * (is - T(1.0))};
-        } else {  // 1/3 + a^2 (-1/45 + a^2 (2/945 - a^2/4725)), a^2 = i q
-            const T q = 2.0 * (s * s);
-            const T ur = T(2.0 / 945.0), ui = -(q * (1.0 / 4725.0));
-            const T nr = fma_(-q, ui, T(-1.0 / 45.0)), ni = q * ur;
-            u = cx<T>{fma_(-q, ni, T(1.0 / 3.0)), q * nr};
-        }
-        const T dr = fma_(T(k3), u.re, T(1.0)), di = k3 * u.im;
-        const T f = rcp_(fma_(dr, dr, di * di));
-        v = cx<T>{dr * f, di * f};
+    const bool far = val(s) > 20.0, small = small_alpha(s);
+    if (!far && !small) return v_table(s, vtab);
+    cx<T> u;
+    if (far) {
+        const T h = 0.5 * is;
+        u = cx<T>{h, h * (is - T(1.0))};
+    } else {  // 1/3 + a^2 (-1/45 + a^2 (2/945 - a^2/4725)), a^2 = i q
+        const T q = 2.0 * (s * s);
+        const T ur = T(2.0 / 945.0), ui = -(q * (1.0 / 4725.0));
+        const T nr = fma_(-q, ui, T(-1.0 / 45.0)), ni = q * ur;
+        u = cx<T>{fma_(-q, ni, T(1.0 / 3.0)), q * nr};
     }
-    return v;
+    return v_of_u(u, k3);
 }
 
 // solveLp (bubble_CUDA_kernel.cuh:314-320) as solvePG uses it
@@ -260,15 +266,19 @@ __device__ inline cx<T> upsilon_g(T s, T is, double k3, const double *vtab) {
 // Y = conj(N) / conj(D) with N = alpha^2 (alpha - 1), D = alpha^2 - 3 alpha + 3,
 // both divided by s^2: conj(N)/s^2 = -2s - 2i(s - 1),
 // conj(D)/s^2 = 3 is (is - 1) - i (2 - 3 is).
-template <typename T, bool UNI = false>
+template <typename T>
+__device__ inline cx<T> lp_inv_far(T s, T is) {
+    const T a = -2.0 * s, b = -2.0 * (s - T(1.0));
+    const T c = (3.0 * is) * (is - T(1.0)), d = fma_(T(3.0), is, T(-2.0));
+    const T id = rcp_(fma_(c, c, d * d));
+    return cx<T>{fma_(a, c, b * d) * id, fma_(b, c, -(a * d)) * id};
+}
+template <typename T>
 __device__ inline cx<T> lp_inv_g(T s, T is, T iR, const double *vtab) {
     cx<T> y;
-    const bool far = cond<UNI>(val(s) > 20.0), small = cond<UNI>(small_alpha(s));
+    const bool far = val(s) > 20.0, small = small_alpha(s);
     if (far) {
-        const T a = -2.0 * s, b = -2.0 * (s - T(1.0));
-        const T c = (3.0 * is) * (is - T(1.0)), d = fma_(T(3.0), is, T(-2.0));
-        const T id = rcp_(fma_(c, c, d * d));
-        y = cx<T>{fma_(a, c, b * d) * id, fma_(b, c, -(a * d)) * id};
+        y = lp_inv_far(s, is);
     } else if (small) {  // W = 1/5 + a^2 (-1/175 + a^2 (2/7875 - 37 a^2 / 3031875))
         const T q = 2.0 * (s * s);
         const T ur = T(2.0 / 7875.0), ui = -(q * (37.0 / 3031875.0));
@@ -326,15 +336,13 @@ __device__ inline void rp_begin_g(RPLaneF<T> &L, T Rp, T Rn, T d1R, T PG, double
 // |dR/dt| and by 10 % of R over sqrt|R d2R/dt2| (each limit only where its
 // denominator exceeds DBL_EPSILON).  The two limits share one reciprocal
 // square root: min(0.01 R / |dR/dt|, 0.1 R / sqrt|R d2R/dt2|) =
-// R / sqrt(max(1e4 (dR/dt)^2, 100 |R d2R/dt2|)).
-template <bool UNI = false>
+// R / sqrt(max(1e4 (dR/dt)^2, 100 |R d2R/dt2|)).  Where neither holds that is
+// NaN (drsqrt(0)), which fmin passes over.
 __device__ inline double rp_dtp(double dtm, double Rn, double d1R, double Rnd2R,
                                 const RPFastShared &s) {
-    double dtp = fmin(1.01 * dtm, s.dt0);
     const double ad = fabs(d1R), aa = fabs(Rnd2R);
     const double m = fmax(ad > kDblEps ? 1.0e4 * (ad * ad) : 0.0, aa > kDblEps ? 100.0 * aa : 0.0);
-    if (__builtin_expect(cond<UNI>(m > 0.0), 1)) dtp = fmin(dtp, Rn * drsqrt(m));
-    return dtp;
+    return fmin(fmin(1.01 * dtm, s.dt0), Rn * drsqrt(m));
 }
 
 // solveOmegaN at (PGn, Rn) (bubble_CUDA_kernel.cuh:263-289) and solveLp as
@@ -344,8 +352,12 @@ __device__ inline double rp_dtp(double dtm, double Rn, double d1R, double Rnd2R,
 // Upsilon.re coef1 coef2 = (Upsilon.re / 3 gam) A and
 // Upsilon.im coef1 PGn / 4 = (-Upsilon.im / 3 gam) B with A = A0 / Rn^3,
 // B = B0 / Rn^3 (rp_fast_const), so both depend on Rn alone.
-template <typename T, bool UNI = false>
-__device__ inline void omega_lp_g(T Rn, T iRn, const RPFastConst &k, const RPFastShared &s,
+// RANGE other than kRangeAny (T = double): all four impedances are taken in
+// that form, without a branch, and the return value says whether they were
+// all in its range; if not, the results are not to be used.
+enum ImpedanceRange { kRangeAny, kRangeFar, kRangeTable };
+template <typename T, int RANGE = kRangeAny>
+__device__ inline bool omega_lp_g(T Rn, T iRn, const RPFastConst &k, const RPFastShared &s,
                                   cx<T> *Ln, T *iom_out) {
     const T iRn2 = iRn * iRn;
     const T iRn3 = iRn2 * iRn;
@@ -357,17 +369,39 @@ __device__ inline void omega_lp_g(T Rn, T iRn, const RPFastConst &k, const RPFas
     T eta = A + fma_(T(-s.mu2), coef3, value1);
     T x, iom;  // x = c_alpha omega / Rn = s^2
     omega_g(eta, xscale, iscale, &x, &iom);
+    double in = RANGE == kRangeFar ? 1.0e300 : 0.0;  // the least s, or the largest |t|
 #pragma unroll
     for (int it = 0; it < 3; it++) {
         const T isa = rsqrt_(x);
-        const cx<T> ups = upsilon_g<T, UNI>(x * isa, isa, s.k3, s.vtab);
+        const T sa = x * isa;
+        cx<T> ups;
+        if constexpr (RANGE == kRangeFar) {
+            ups = upsilon_far(isa, s.k3);
+            in = fmin(in, sa);
+        } else if constexpr (RANGE == kRangeTable) {
+            const cx_d v = v_poly(sa, s.vtab, nullptr, nullptr, &in);
+            ups = cx<T>{v.re, v.im};
+        } else {
+            ups = upsilon_g(sa, isa, s.k3, s.vtab);
+        }
         const T mu_eff = fma_(ups.im * B, iom, T(s.mu));  // mu + ui PG / (4 omega)
         eta = fma_(ups.re, A, fma_(-(mu_eff * mu_eff), coef3, value1));
         omega_g(eta, xscale, iscale, &x, &iom);
     }
-    const T isa = rsqrt_(x);
-    *Ln = lp_inv_g<T, UNI>(x * isa, isa, iRn, s.vtab);
+    const T isa = rsqrt_(x), sa = x * isa;
     *iom_out = iom;
+    if constexpr (RANGE == kRangeFar) {
+        const cx<T> y = lp_inv_far(sa, isa);
+        *Ln = cx<T>{y.re * iRn, y.im * iRn};
+        return fmin(in, sa) > 20.0;
+    } else if constexpr (RANGE == kRangeTable) {
+        const cx_d y = v_poly(sa, s.vtab + kRpVFunc, nullptr, nullptr, &in);
+        *Ln = cx<T>{y.re * iRn, y.im * iRn};
+        return in <= 1.0;
+    } else {
+        *Ln = lp_inv_g(sa, isa, iRn, s.vtab);
+        return true;
+    }
 }
 
 // solveRayleighPlesset (bubble_CUDA_kernel.cuh:227-260) and the clock of the
@@ -378,20 +412,20 @@ template <typename T>
 struct RPMove {
     T Rn, iRn, PGn;
 };
-template <typename T, bool FORCED = false, bool UNI = false>
-__device__ inline RPMove<T> rp_advance_g(RPLaneF<T> &L, const RPFastShared &s,
+// iRn = 1 / L.Rp.  LAST: the sub-step may reach the sync time.
+template <typename T, bool FORCED = false, bool UNI = false, bool LAST = true>
+__device__ inline RPMove<T> rp_advance_g(RPLaneF<T> &L, T iRn, const RPFastShared &s,
                                          double forced_dtp = 0.0) {
     const T PGn = L.PG;
     const double t = L.time;
     const T PL = fma_(L.PC2, T(t * t), fma_(L.PC1, T(t), L.PC0));
     const T Rm = L.Rn;
     const T Rn = L.Rp;
-    const T iRn = rcp_(Rn);
     T d1R = L.d1R;
     const T sv = iRn * fma_(T(s.four_mu), d1R, T(s.two_sig));  // (2 sig + 4 mu dR) / R
     const T Rnd2R = fma_(-1.5 * d1R, d1R, (PGn - PL - sv) * s.irho);
     const double dtm = L.dtL;
-    double dtp = rp_dtp<UNI>(dtm, val(Rn), val(d1R), val(Rnd2R), s);
+    double dtp = rp_dtp(dtm, val(Rn), val(d1R), val(Rnd2R), s);
     if constexpr (FORCED) dtp = forced_dtp;
     const double idtm = drcp(dtm);
     const double r = dtp * idtm;
@@ -401,12 +435,12 @@ __device__ inline RPMove<T> rp_advance_g(RPLaneF<T> &L, const RPFastShared &s,
     const double iden = drcp(dtm * dtp * (dtm + dtp));
     d1R = fma_(fma_(T(dm2), Rp, fma_(T(dp2 - dm2), Rn, -dp2 * Rm)), T(iden), acc);
     const double dtL = dtp;
-    if (__builtin_expect(cond<UNI>(dtp >= L.remain), 0)) {  // last sub-step: R_t at the sync time
+    if (LAST && __builtin_expect(cond<UNI>(dtp >= L.remain), 0)) {  // last sub-step: R_t at the sync time
         const double d = L.remain;
         const double r2 = d * idtm;
         L.Rt = fma_((d * Rnd2R) * iRn, T(0.5 * (d + dtm)), fma_(T(1.0 + r2), Rn, -r2 * Rm));
         dtp = d;
-    } else {
+    } else if (LAST) {
         L.Rt = Rp;
     }
     L.remain -= dtp;
@@ -455,14 +489,13 @@ __device__ inline void rp_gas_g(RPLaneF<T> &L, const RPMove<T> &mv, cx<T> Ln, T 
 // FORCED: the step size is forced_dtp instead of the step-size control's
 // (the replay of a recorded schedule; the rest of the sub-step is unchanged).
 // HEAT: accumulate the heat and viscous dissipation of Q_B (T = double).
-// UNI: one lane runs the sub-step alone (branches on the scalar unit, cond).
-template <typename T, bool FORCED = false, bool HEAT = true, bool UNI = false>
+template <typename T, bool FORCED = false, bool HEAT = true>
 __device__ inline void rp_substep_g(RPLaneF<T> &L, const RPFastConst &k, const RPFastShared &s,
                                     double forced_dtp = 0.0) {
-    const RPMove<T> mv = rp_advance_g<T, FORCED, UNI>(L, s, forced_dtp);
+    const RPMove<T> mv = rp_advance_g<T, FORCED>(L, rcp_(L.Rp), s, forced_dtp);
     cx<T> Ln;  // Lp / |Lp|^2
     T iom;
-    omega_lp_g<T, UNI>(mv.Rn, mv.iRn, k, s, &Ln, &iom);
+    omega_lp_g(mv.Rn, mv.iRn, k, s, &Ln, &iom);
     rp_gas_g<T, HEAT>(L, mv, Ln, iom, k, s);
 }
 
@@ -490,23 +523,59 @@ __device__ inline double from_odd(double v) { return quad_move<0xF5>(v); }   // 
 template <bool UNI>
 __device__ inline void rp_pair_pass(RPLaneF<double> &L, const RPFastConst &k,
                                     const RPFastShared &s, bool odd, int max_substeps) {
-    const RPMove<double> m0 = rp_advance_g<double, false, UNI>(L, s);
+    const RPMove<double> m0 = rp_advance_g<double, false, UNI>(L, drcp(L.Rp), s);
     const double R = odd ? L.Rp : m0.Rn;
+    const double iR = drcp(R);
     cx<double> Ln;
     double iom;
-    omega_lp_g<double>(R, drcp(R), k, s, &Ln, &iom);
+    omega_lp_g(R, iR, k, s, &Ln, &iom);
     rp_gas_g<double>(L, m0, cx<double>{from_even(Ln.re), from_even(Ln.im)}, from_even(iom), k, s);
     if (cond<UNI>(L.remain > 0.0 && L.counter < max_substeps)) {
-        const RPMove<double> m1 = rp_advance_g<double, false, UNI>(L, s);
+        const RPMove<double> m1 = rp_advance_g<double, false, UNI>(L, from_odd(iR), s);
         rp_gas_g<double>(L, m1, cx<double>{from_odd(Ln.re), from_odd(Ln.im)}, from_odd(iom), k, s);
     }
+}
+
+// Passes of the one bubble that a wavefront's lane pair holds, without a
+// branch but the two at their end, while neither sub-step of a pass can reach
+// the sync time (a step is at most 1.01 times the one before) and the
+// impedances stay in RANGE.  A wavefront of its own issues an instruction
+// every 4 cycles, dependent or not, and a branch on a comparison just made
+// costs 30 (45 if taken); a pass had some twenty.  A collapse spends half of
+// its sub-steps beyond the tables and most of the others within them.  RP
+// launch with branches at each impedance against without: 11 bubbles 1240 /
+// 965 us, 30 011 1810 / 1640, 2^20 2185 / 2142, 2^22 2600 / 2523.
+template <int RANGE>
+__device__ inline void rp_pair_run(RPLaneF<double> &L, const RPFastConst &k,
+                                   const RPFastShared &s, bool odd, int max_substeps) {
+    while (cond<true>(L.remain > 2.1 * L.dtL && L.counter + 1 < max_substeps)) {
+        const RPMove<double> m0 = rp_advance_g<double, false, true, false>(L, drcp(L.Rp), s);
+        const double R = odd ? L.Rp : m0.Rn;
+        const double iR = drcp(R);
+        cx<double> Ln;
+        double iom;
+        const bool in = omega_lp_g<double, RANGE>(R, iR, k, s, &Ln, &iom);
+        const bool out = cond<true>(!in);
+        if (__builtin_expect(out, 0)) omega_lp_g(R, iR, k, s, &Ln, &iom);
+        rp_gas_g<double>(L, m0, cx<double>{from_even(Ln.re), from_even(Ln.im)}, from_even(iom), k,
+                         s);
+        const RPMove<double> m1 = rp_advance_g<double, false, true, false>(L, from_odd(iR), s);
+        rp_gas_g<double>(L, m1, cx<double>{from_odd(Ln.re), from_odd(Ln.im)}, from_odd(iom), k, s);
+        if (__builtin_expect(out, 0)) break;
+    }
+    L.Rt = L.Rp;
 }
 
 // The whole integration of the one bubble that a wavefront's lane pair holds.
 __device__ inline void rp_integrate_pair(RPLaneF<double> &L, const RPFastConst &k,
                                          const RPFastShared &s, bool odd, int max_substeps) {
-    while (cond<true>(L.remain > 0.0 && L.counter < max_substeps))
-        rp_pair_pass<true>(L, k, s, odd, max_substeps);
+    while (cond<true>(L.remain > 0.0 && L.counter < max_substeps)) {
+        rp_pair_run<kRangeFar>(L, k, s, odd, max_substeps);
+        rp_pair_run<kRangeTable>(L, k, s, odd, max_substeps);
+        if (cond<true>(!(L.remain > 2.1 * L.dtL && L.counter + 1 < max_substeps)) &&
+            cond<true>(L.remain > 0.0 && L.counter < max_substeps))
+            rp_pair_pass<true>(L, k, s, odd, max_substeps);
+    }
 }
 
 // ---- reverse mode: adjoints of the RP map of one Picard iteration ----------
