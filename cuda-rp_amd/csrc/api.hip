@@ -463,7 +463,7 @@ int alloc_bubbles(brp_handle *h, int n) {
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.part, sizeof(int) * 2 * (size_t)((n + 255) / 256 + 1))))
         return rc;
-    if ((rc = dalloc(h, (void **)&h->b.heads, sizeof(unsigned int) * kQueueHeads * kHeadStride)))
+    if ((rc = dalloc(h, (void **)&h->b.heads, sizeof(unsigned int) * 2 * kQueueHeads * kHeadStride)))
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.totals, sizeof(RPTotals) * 4 * (size_t)(h->cus * h->per_cu))))
         return rc;
@@ -1037,11 +1037,11 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     launch_rp_replay<F>(s, h->rpl_d, h->nb, h->rp_cur, h->pl_m, h->pl_n, h->pl_p,
                                         p0, h->fgb[target], h->sc_d, cl.off, cl.dts);
                 } else {
-                    const bool lean = bubble_step_lean(h->last_sub_max, h->last_sub_per_launch,
-                                                       h->bp.extreme_threshold, h->cus);
-                    st.rp_lean_launches += lean ? 1 : 0;
+                    const RPGrid shape = bubble_step_grid(h->last_sub_max, h->last_sub_per_launch,
+                                                          h->bp.extreme_threshold, h->cus);
+                    st.rp_lean_launches += shape == kRPLean ? 1 : 0;
                     rp_waves = launch_bubble_step<F>(s, *h->rpl_h, h->rpl_d, h->rp_cur, h->pl_m, h->pl_n,
-                                          h->pl_p, p0, h->fgb[target], h->sc_d, loop, lean, h->cus,
+                                          h->pl_p, p0, h->fgb[target], h->sc_d, loop, shape, h->cus,
                                           h->per_cu);
                     if (h->sched_mode == 1) {
                         int rc = schedule_record_call(h);

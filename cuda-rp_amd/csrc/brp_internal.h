@@ -241,7 +241,8 @@ struct BubbleArrays {
     int *part;            // partition scratch: per-block extreme and heavy offsets + totals
     int *bbox_blk;        // per-block stencil bounding boxes of k_motion (4 ints each)
     RPTotals *totals;     // per wavefront of the RP launch
-    unsigned int *heads;  // kQueueHeads work-queue heads, kHeadStride apart
+    unsigned int *heads;  // kQueueHeads work-queue heads, kHeadStride apart, twice
+                          // (the second for the extreme entries on lane pairs)
 };
 
 // Bubble physics constants shared by every bubble.
@@ -338,13 +339,17 @@ inline bool pressure_ghosts_fixed(const GridParams &g) {
 template <typename F>
 void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                    const BubbleArrays &b, const F *vx, const F *vy, StepScalars *sc);
+// Shape of an RP launch: bound by its longest chains (one workgroup per
+// compute unit), with long chains but bound by the work of all bubbles (as
+// many workgroups as fit), or without long chains (the same).
+enum RPGrid { kRPLean, kRPFull, kRPLight };
 // The RP launch of Picard iteration `slot` over the queue order, with the
 // gathered pressures of launch_queue_keys in PL[plp].
 // Returns the number of wavefronts launched (their records in b.totals).
 template <typename F>
 int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
                         int plm, int pln, int plp, const F *p0, int64_t *fg_target, StepScalars *sc,
-                        int slot, bool lean, int cus, int per_cu);
+                        int slot, RPGrid shape, int cus, int per_cu);
 // Whether the launch runs every bubble on a lane pair, and whether it then
 // needs no queue (it gathers the pressures itself).
 bool bubble_step_pairs(const RPLaunch &host, int cus);
@@ -353,10 +358,9 @@ bool bubble_step_unordered(const RPLaunch &host, int cus);
 // compute unit (its occupancy limit), queried once per handle.
 void rp_grid_query(int device, int *cus, int *per_cu);
 int bubble_step_blocks(int n_bubbles, bool lean, int cus, int per_cu);
-// Whether the next RP launch is bound by its longest chains (lean grid): the
-// longest chain of the last launch is long and the sub-steps per lane of a
-// one-workgroup-per-CU grid are few against it.
-bool bubble_step_lean(int sub_max, double sub_per_launch, int extreme_threshold, int cus);
+// The shape of the next RP launch, from the last one's longest chain and its
+// sub-steps in all.
+RPGrid bubble_step_grid(int sub_max, double sub_per_launch, int extreme_threshold, int cus);
 // Pressure gather of a Picard iteration's bubbles into PL[plp] and its queue
 // keys (predicted or previous sub-step counts; -1: the previous iteration's
 // results stand).

@@ -311,6 +311,21 @@ __device__ inline bool queue_batch(unsigned int *heads, int lane, int n, int siz
     return false;
 }
 
+// Where a wavefront of k_bubble_persistent takes its bubbles from and how it
+// holds them: long ones on lane pairs, the others a lane each, its last ones
+// on lane pairs again.
+enum RPPhase { kOnPairs, kOnLanes, kSpread };
+
+// The integration state of lane src, in every lane.
+__device__ inline void spread_lane(RPLaneF<double> &L, RPFastConst &k, int src) {
+    double *p[] = {&L.Rp,   &L.Rn,  &L.d1R,  &L.PG,      &L.Rt,     &L.PC0, &L.PC1, &L.PC2,
+                   &L.dtL,  &L.remain, &L.time, &L.SumHeat, &L.SumVis,
+                   &k.iR0,  &k.PG0, &k.iPG0, &k.calpha_irho, &k.PG0R03, &k.T0_PG0R03, &k.A0, &k.B0};
+#pragma unroll
+    for (double *q : p) *q = __shfl(*q, src, 64);
+    L.counter = __shfl(L.counter, src, 64);
+}
+
 // One Picard iteration for every bubble, fused (after k_queue_keys gathered
 // PL_p, BubbleInterpolationScalarKernel, kernel.cuh:361-395):
 //   BubbleRadiusKernel              (RP from the step's start state, 471-554)
@@ -343,13 +358,25 @@ __device__ inline crpl *rpl(const RPLaunch *p) {
     return q;
 }
 
+// PAIRS (launches with long chains): the queue's extreme entries after the
+// dedicated ones run on lane pairs of the shared wavefronts, spread over all
+// of them (at most 32 to a wavefront), before the others are taken a lane
+// each; and once the queue is empty a wavefront with at most 32 bubbles left
+// moves them onto lane pairs.  A pair does a sub-step in 0.7 of a lane's time,
+// and a chain of the 257th rank is nearly as long as the first: RP launch of
+// 2^20 bubbles 2142 -> 1476 us, 2^22 (with the full grid) 2523 -> 2060,
+// 30 011 1640 -> 1510; 65 536 at the onset of cavitation 1207 -> 1250.  256
+// VGPRs, so that two wavefronts fit a SIMD; held to that by the attribute for
+// two the compiler spills nine, and a launch without long chains took 12 %
+// more.
+//
 // A shared wavefront holds at most `quota` bubbles (64 but for a population
 // too small to give every wavefront 64), takes as many from the queue at a
 // time, and leaves the sub-step loop to write back and refill when half of
 // them have finished (4096^2 clustered on the lean grid, quota 64, ms per step
 // for 16 / 24 / 32 / 40 / 48 finished lanes: 24.5 / 23.3 / 23.0 / 23.2 / 24.2;
 // 2048^2 equal within 1 % from 24 to 48).
-template <typename F, bool FAST>
+template <typename F, bool FAST, bool PAIRS>
 __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, int max_substeps,
                                                             const double *rp_shared, int cur,
                                                             int plm, int pln, int plp,
@@ -364,7 +391,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     WaveAgg &agg = agg_all[threadIdx.x >> 6];
     agg_clear(agg, lane);
     // The shared RP constants go through LDS into vector registers, held for
-    // the whole kernel (247 VGPRs, two wavefronts per SIMD still fit): read
+    // the whole kernel (two wavefronts per SIMD still fit): read
     // from the constant table instead, each sub-step waited on its scalar
     // loads (no scalar registers are free to hold them).
     __shared__ double shc[16];
@@ -395,12 +422,18 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     // 2.65 ms at 4096^2 with 2^22, against one lane).  Lane 0 writes back.
     // The wavefront runs at raised issue priority until that bubble is done,
     // then joins the shared queue, which starts after the E dedicated entries.
-    int E, nb;
+    int E, nb, X;
     {
         const BubbleArrays &b = rpl(kp)->b;
         nb = b.n;
-        E = min(min(b.part[(b.n + 255) / 256], (int)gridDim.x), solo_cap);
+        X = b.part[(b.n + 255) / 256];
+        E = min(min(X, (int)gridDim.x), solo_cap);
+        if (!PAIRS) X = E;
     }
+    // lane pairs of a shared wavefront for the entries [E, X)
+    const int quota_x = min(32, (X - E + 4 * (int)gridDim.x - 1 - E) / (4 * (int)gridDim.x - E));
+    RPPhase phase = PAIRS && X > E ? kOnPairs : kOnLanes;  // wave-uniform
+    const bool odd = lane & 1;
     int idx = -1;                  // bubble of this lane, -1 when idle
     bool reuse = false;            // idx keeps its previous iteration's results
     bool pre = false;
@@ -416,11 +449,9 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
     RPLane L;              // operation-by-operation path
     RPLaneF<double> LF;    // shortened-chain path
     RPConst k{0.0, 0.0, 0.0, 0.0};
-    double x = 0.0, y = 0.0;
-    int ibnx = 0, ibny = 0;
     int sub_max = 0;
-    unsigned long long sub_sum = 0;
-    unsigned int done = 0;  // bubbles this lane wrote back
+    unsigned int sub_sum = 0;  // 2^32 sub-steps of a lane would take half an hour
+    unsigned int done = 0;  // bubbles this wavefront wrote back
     unsigned int kept = 0;  // of them, with the previous iteration's results
     bool bad = false, capped_any = false;
     while (true) {
@@ -429,7 +460,14 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
             __builtin_amdgcn_s_setprio(0);
         }
         // ---- refill idle lanes from the wave's batch / the global queue
-        bool need = idx < 0 && !solo && lane < quota;
+        if (PAIRS && phase == kOnPairs && !solo && exhausted && __ballot(idx >= 0) == 0ull) {
+            phase = kOnLanes;
+            exhausted = false;
+            batch_next = batch_end = 0;
+            head = (int)blockIdx.x & (kQueueHeads - 1);
+        }
+        const bool pairs = FAST && (phase != kOnLanes || solo);  // wave-uniform
+        bool need = idx < 0 && !solo && (pairs ? !odd && (lane >> 1) < quota_x : lane < quota);
         {
         crpl *P = rpl(kp);
         const GridParams &g = P->g;
@@ -440,30 +478,39 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         pre = false;
         while (m != 0ull && !exhausted) {
             if (batch_next >= batch_end &&
-                !queue_batch(b.heads, lane, nb - E, quota, head, batch_next, batch_end)) {
+                !queue_batch(b.heads + (pairs ? kQueueHeads * kHeadStride : 0), lane,
+                             pairs ? X - E : nb - X, pairs ? quota_x : quota, head, batch_next,
+                             batch_end)) {
                 exhausted = true;
                 break;
             }
             const int avail = batch_end - batch_next;
             const int rank = __popcll(m & lanemask_lt(lane));
             if (need && rank < avail) {
-                idx = b.order[E + batch_next + rank];
+                idx = b.order[(pairs ? E : X) + batch_next + rank];
                 need = false;
                 fresh = true;
             }
             batch_next += min(avail, __popcll(m));
             m = __ballot(need);
         }
+        if (PAIRS && pairs && !solo) {  // the even lane took it, its partner copies
+            idx = __shfl(idx, lane & ~1, 64);
+            fresh = __shfl((int)fresh, lane & ~1, 64) != 0;
+        }
         if (fresh) {
-            x = b.x[idx];
-            y = b.y[idx];
-            ibnx = bin_index(x, g.rdx, 0.5);
-            ibny = bin_index(y, g.rdy, 0.5);
             const double PL = b.PL[plp][idx];  // gathered by k_queue_keys
             reuse = b.key[idx] < 0;            // the previous iteration's results stand
             const double R0 = b.R0[idx];
             k = RPConst{R0, R0 * R0 * R0, b.PG0[idx], b.calpha[idx]};
-            if (FAST) fk = rp_fast_const(R0, k.PG0, k.calpha, bp.T0, fsh);
+            if (FAST) {
+                // (g3 from LDS: a register less through the sub-steps)
+                ldouble *q = (ldouble *)shc;
+                asm volatile("" : "+v"(q));
+                RPFastShared f = fsh;
+                f.g3 = q[6];
+                fk = rp_fast_const(R0, k.PG0, k.calpha, bp.T0, f);
+            }
             if (reuse) {
                 LF.remain = 0.0;
                 LF.counter = 0;
@@ -481,7 +528,10 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         }
         }
         const bool active = idx >= 0;
-        if (__ballot(active) == 0ull) break;
+        if (__ballot(active) == 0ull) {
+            if (PAIRS && phase == kOnPairs) continue;
+            break;
+        }
         // ---- sub-steps until half of the quota's bubbles have reached the
         // sync time (or the sub-step cap), or no active lane is left
         // running; finished lanes idle meanwhile.  The refill and write-back
@@ -493,15 +543,24 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         // 46.1 -> 29.2 with a batch of 24 on the full grid).
         bool fin, capped;
         double remain;
-        if (FAST && solo) {
-            // a dedicated wavefront: lanes 0 and 1 run its bubble to the sync
-            // time without the batch bookkeeping of the shared loop below
-            // (both hold one bubble: its conditions are wave-uniform)
-            if (active) rp_integrate_pair(LF, fk, fsh, lane & 1, max_substeps);
-            if (lane == 1) idx = -1;  // lane 0 writes back
+        if (FAST && pairs) {
+            while (true) {
+                const bool run = active && LF.remain > 0.0 && LF.counter < max_substeps;
+                const unsigned long long rm = __ballot(run);
+                if (rm == 0ull || (!exhausted && !solo && __popcll(rm) <= quota_x)) break;
+                if (__popcll(rm) == 2) {  // one bubble: to the end
+                    if (run) rp_integrate_pair(LF, fk, fsh, odd, max_substeps);
+                } else if (run) {
+                    rp_pair_pass<false>(LF, fk, fsh, odd, max_substeps);
+                }
+            }
             capped = active && LF.counter >= max_substeps;
             remain = active ? LF.remain : 0.0;
-            fin = idx >= 0;
+            fin = active && (!(remain > 0.0) || capped);
+            if (odd && fin) {
+                fin = false;  // the even lane writes back
+                idx = -1;
+            }
         } else
         while (true) {
             capped = false;
@@ -521,8 +580,11 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
             const unsigned long long fm = __ballot(fin);
             if (fm != 0ull && (2 * __popcll(fm) >= quota || __ballot(active && !fin) == 0ull))
                 break;
+            if (PAIRS && exhausted && __popcll(__ballot(active && !fin)) <= 32) break;
         }
         // ---- write back the bubbles that reached the sync time
+        done += (unsigned int)__popcll(__ballot(fin));
+        kept += (unsigned int)__popcll(__ballot(fin && reuse));
         if (idx >= 0) {
             crpl *P = rpl(kp);
             const GridParams &g = P->g;
@@ -532,10 +594,10 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
                 double R_t;
                 if (reuse) {  // the previous iteration's results are in place
                     R_t = b.R_t[idx];
-                    kept++;
                 } else {
                     RPState out;
                     double Q_B;
+                    LF.re_n = b.re[cur][idx];
                     if (FAST)
                         rp_end_g(LF, g.dt, &out, &R_t, &Q_B);
                     else
@@ -551,21 +613,37 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
                     b.Q_B[idx] = Q_B;
                     b.sub[idx] = cnt;
                     sub_max = max(sub_max, cnt);
-                    sub_sum += (unsigned long long)cnt;
+                    sub_sum += (unsigned int)cnt;
                     capped_any |= capped && remain > 0.0;
                 }
-                done++;
                 bad |= !isfinite(R_t);
-                scatter_bubble_agg(g, bp, x, y, ibnx, ibny,
+                const double x = b.x[idx], y = b.y[idx];
+                scatter_bubble_agg(g, bp, x, y, bin_index(x, g.rdx, 0.5), bin_index(y, g.rdy, 0.5),
                                    fg_temp_of(g, bp, b.n_B[idx], R_t, x), agg, fg_target, &bad);
                 idx = -1;
                 reuse = false;
             }
         }
         if (__builtin_amdgcn_readfirstlane(agg.count) > kAggSlots / 2) agg_flush(agg, lane, fg_target);
+        // ---- nothing is left to take and at most 32 bubbles run: onto pairs
+        if (PAIRS && phase == kOnLanes && !solo && exhausted) {
+            const unsigned long long m = __ballot(idx >= 0);
+            if (m != 0ull && __popcll(m) <= 32) {
+                phase = kSpread;
+                int src = __builtin_amdgcn_ds_permute(
+                    (idx >= 0 ? 2 * __popcll(m & lanemask_lt(lane)) : 63) * 4, lane);
+                src = __shfl(src, lane & ~1, 64);
+                const bool mine = (lane >> 1) < __popcll(m);
+                spread_lane(LF, fk, src);
+                idx = __shfl(idx, src, 64);
+                reuse = __shfl((int)reuse, src, 64) != 0;
+                if (!mine) idx = -1;
+            }
+        }
     }
     agg_flush(agg, lane, fg_target);
-    rp_launch_totals(rpl(kp)->b.totals, lane, sub_max, sub_sum, done, kept, bad, capped_any);
+    rp_launch_totals(rpl(kp)->b.totals, lane, sub_max, sub_sum, lane ? 0u : done, lane ? 0u : kept, bad,
+                     capped_any);
 }
 
 // The same launch for a population that the chip can hold at once on lane
@@ -986,26 +1064,25 @@ void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
 }
 
 // Workgroups of the persistent RP kernel: as many as fit (two per CU) when
-// the launch is throughput-bound; one per CU ("lean") when a few long
-// sub-step chains bound it, so that each dedicated wavefront has a SIMD of
-// its own and fewer shared-queue wavefronts compete with it.  Measured with
-// the void-fraction scatter aggregated in LDS: 2048^2, 2^20 bubbles during
-// cavitation (a 3500-sub-step chain, 430 sub-steps per lean-grid lane):
-// lean 23.0 vs full 26.2 ms of RP per step; 4096^2, 2^22 clustered bubbles
-// at 3 MPa (a 4000-sub-step chain, several thousand per lane): lean 84 vs
-// full 60 ms.  bubble_step_lean decides from the previous launch.
+// the launch is bound by the work of all bubbles; one per CU ("lean") when a
+// few long sub-step chains bound it, so that each wavefront has a SIMD of its
+// own.  Collapsing bubbles, ms per step on the lean / full grid: 2^20 (2500
+// sub-steps in the longest chain, 0.14 of that in a lane of the lean grid on
+// average) 6.3 / 7.4; 2^22 (2700, 0.49) 13.4 / 11.2.  bubble_step_grid decides
+// from the previous launch.
 void rp_grid_query(int device, int *cus, int *per_cu) {
     int c = 0, p = 0;
     (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, device);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, k_bubble_persistent<float, true>, 256,
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, k_bubble_persistent<float, true, true>, 256,
                                                        0);
     *cus = std::max(1, c);
     *per_cu = std::max(1, p);
 }
 
-bool bubble_step_lean(int sub_max, double sub_per_launch, int extreme_threshold, int cus) {
+RPGrid bubble_step_grid(int sub_max, double sub_per_launch, int extreme_threshold, int cus) {
     const double lanes = 256.0 * cus;  // lanes of the lean grid
-    return sub_max >= 2 * extreme_threshold && sub_per_launch < 0.6 * lanes * sub_max;
+    if (sub_max < 2 * extreme_threshold) return kRPLight;
+    return sub_per_launch < 0.2 * lanes * sub_max ? kRPLean : kRPFull;
 }
 
 // A lean launch spreads a small population over all its compute units (30 011
@@ -1036,7 +1113,7 @@ bool bubble_step_unordered(const RPLaunch &host, int cus) {
 template <typename F>
 int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
                         int plm, int pln, int plp, const F *p0, int64_t *fg_target,
-                        StepScalars *sc, int slot, bool lean, int cus, int per_cu) {
+                        StepScalars *sc, int slot, RPGrid shape, int cus, int per_cu) {
     if (host.b.n <= 0) return 0;
     const int cap = host.bp.max_substeps;
     if (bubble_step_pairs(host, cus)) {
@@ -1052,25 +1129,20 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
                                (n + waves - 1) / waves, cus);
         return 4 * blocks;
     }
+    const bool lean = shape == kRPLean;
     const dim3 grid(bubble_step_blocks(host.b.n, lean, cus, per_cu));
     const int quota = std::max(8, std::min(64, (host.b.n + 4 * (int)grid.x - 1) / (4 * (int)grid.x)));
     // Dedicated wavefronts: up to one per workgroup on the lean grid, where
-    // the longest chains bound the launch; CUs / 8 on the full grid, which
-    // is chosen when the total work bounds it: a wavefront with one active
-    // lane still takes its SIMD's issue slots, so every dedicated wavefront
-    // costs a SIMD of throughput there.  4096^2, 2^22 clustered bubbles
-    // (full grid): 512 dedicated 49.8, 128 46.8, 32 46.4, 0 46.2 ms/step;
-    // with refills batched: 128 29.6, 64 29.2, 32 29.3,
-    // 0 30.8; 2048^2 (lean grid): 256 17.2, 32 17.4, 0 19.1 ms/step.
-    const int solo_cap = lean ? (int)grid.x : std::max(1, cus / 8);
-    if (host.bp.rp_exact)
-        hipLaunchKernelGGL((k_bubble_persistent<F, false>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, quota,
-                           solo_cap);
-    else
-        hipLaunchKernelGGL((k_bubble_persistent<F, true>), grid, dim3(256), 0, s, dev, cap,
-                           host.bp.rp_shared, cur, plm, pln, plp, fg_target, sc, quota,
-                           solo_cap);
+    // the longest chains bound the launch.  On the full grid, bound by the
+    // work, every one costs a SIMD of throughput: 2^22 clustered bubbles with
+    // 16 / 32 / 64 / 128 / 256 of them 183.9 / 183.4 / 183.4 / 186.7 / 193 ms
+    // for 16 steps.
+    const int solo_cap = lean ? (int)grid.x : std::max(1, cus / (shape == kRPFull ? 4 : 8));
+    const auto k = host.bp.rp_exact    ? k_bubble_persistent<F, false, false>
+                   : shape == kRPLight ? k_bubble_persistent<F, true, false>
+                                       : k_bubble_persistent<F, true, true>;
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, s, dev, cap, host.bp.rp_shared, cur, plm, pln, plp,
+                       fg_target, sc, quota, solo_cap);
     return 4 * (int)grid.x;
 }
 
@@ -1089,7 +1161,7 @@ __global__ __launch_bounds__(256) void k_part_count(const int *sub, int n, int e
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (blockIdx.x == 0) {
         for (int k = threadIdx.x; k < kSortBins; k += 256) sort_hist[k] = 0;
-        if (threadIdx.x < kQueueHeads) heads[threadIdx.x * kHeadStride] = 0u;
+        if (threadIdx.x < 2 * kQueueHeads) heads[threadIdx.x * kHeadStride] = 0u;
     }
     const int v = idx < n ? sub[idx] : 0;
     const int ce = __syncthreads_count(idx < n && v >= ext);
@@ -1392,10 +1464,10 @@ template void launch_motion<float>(hipStream_t, const GridParams &, const Bubble
                                    const BubbleArrays &, const float *, const float *,
                                    StepScalars *);
 template int launch_bubble_step<double>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
-                                         int, int, const double *, int64_t *, StepScalars *, int, bool, int,
+                                         int, int, const double *, int64_t *, StepScalars *, int, RPGrid, int,
                                          int);
 template int launch_bubble_step<float>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
-                                         int, int, const float *, int64_t *, StepScalars *, int, bool, int,
+                                         int, int, const float *, int64_t *, StepScalars *, int, RPGrid, int,
                                          int);
 
 }  // namespace brp
