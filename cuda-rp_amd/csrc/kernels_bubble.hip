@@ -24,6 +24,25 @@ __device__ inline double delta_w(double coef_x, double coef_k, int pos, double h
     return coef_x * (1.0 + cos(coef_k * (((double)pos - 0.5) * h - b)));
 }
 
+// A stencil's weights along one axis, each cosine taken once.  NB = 2: the
+// usual band, known at compile time, so that the stencil's loops unroll and
+// its loads and cosines overlap; NB = 0: any band up to kMaxBand.  (The
+// gather took the inner axis's cosines again for every outer one:
+// k_queue_keys over 2^22 bubbles 70 -> 51 us, 2^20 22.8 -> 17.)
+template <int NB>
+struct Weights {
+    double w[NB ? NB : kMaxBand];
+    __device__ Weights(double coef_x, double coef_k, int first, int nb, double h, double b) {
+        if constexpr (NB > 0) {
+#pragma unroll
+            for (int a = 0; a < NB; a++) w[a] = delta_w(coef_x, coef_k, first + a, h, b);
+        } else {
+            for (int a = 0; a < nb; a++) w[a] = delta_w(coef_x, coef_k, first + a, h, b);
+        }
+    }
+    __device__ double operator[](int a) const { return w[a]; }
+};
+
 __device__ inline int64_t to_fixed(double v, bool *bad) {
     double s = v * kFgScale;
     if (!(fabs(s) < 4.611686018427388e18)) {  // |v| < 4, NaN rejected
@@ -71,7 +90,10 @@ __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *o
 // BubbleInterpolationVelocityKernel + v_B <- v_L + BubbleMotionKernel
 // (bubble_CUDA_kernel.cuh:398-468, 1282-1297), fused per bubble; also the
 // bounding box of the new scatter stencils for the Picard window.
-template <typename F>
+// Bound by its eight cosines rather than its 96 bytes a bubble (2^22 bubbles:
+// 131 us with the band known at run time only, 112 with NB = 2; 80 to move
+// the bytes).
+template <typename F, int NB>
 __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, BubbleArrays b,
                                                  const F *__restrict__ vx,
                                                  const F *__restrict__ vy, StepScalars *sc) {
@@ -84,25 +106,26 @@ __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, B
         const int ibnx = bin_index(x, g.rdx, 0.5), ibny = bin_index(y, g.rdy, 0.5);
         // the four weight sets (x at ibm / ibn columns, y at ibn / ibm rows),
         // each evaluated once
-        const int nb = bp.mbe - bp.mbs + 1;
-        double wxm[kMaxBand], wyn[kMaxBand], wxn[kMaxBand], wym[kMaxBand];
-        for (int a = 0; a < nb; a++) {
-            wxm[a] = delta_w(bp.dcx, bp.dcy, ibmx + bp.nbs + a, g.dx, x);
-            wxn[a] = delta_w(bp.dcx, bp.dcy, ibnx + bp.mbs + a, g.dx, x);
-            wyn[a] = delta_w(bp.dcx, bp.dcz, ibny + bp.mbs + a, g.dy, y);
-            wym[a] = delta_w(bp.dcx, bp.dcz, ibmy + bp.nbs + a, g.dy, y);
-        }
+        const int nb = NB ? NB : bp.mbe - bp.mbs + 1;
+        const Weights<NB> wxm(bp.dcx, bp.dcy, ibmx + bp.nbs, nb, g.dx, x);
+        const Weights<NB> wxn(bp.dcx, bp.dcy, ibnx + bp.mbs, nb, g.dx, x);
+        const Weights<NB> wyn(bp.dcx, bp.dcz, ibny + bp.mbs, nb, g.dy, y);
+        const Weights<NB> wym(bp.dcx, bp.dcz, ibmy + bp.nbs, nb, g.dy, y);
         double vLx = 0.0, vLy = 0.0;
+#pragma unroll
         for (int a = 0; a < nb; a++) {
             const int i = ibmx + bp.nbs + a;
+#pragma unroll
             for (int c = 0; c < nb; c++) {
                 const int j = ibny + bp.mbs + c;
                 if (i >= -1 && i <= g.N + 1 && j >= 0 && j <= g.M + 1)
                     vLx += (double)vx[frame_off(i, j, g.pitch)] * wxm[a] * wyn[c];
             }
         }
+#pragma unroll
         for (int a = 0; a < nb; a++) {
             const int i = ibnx + bp.mbs + a;
+#pragma unroll
             for (int c = 0; c < nb; c++) {
                 const int j = ibmy + bp.nbs + c;
                 if (i >= 0 && i <= g.N + 1 && j >= -1 && j <= g.M + 1)
@@ -146,24 +169,32 @@ __device__ inline double fg_temp_of(const GridParams &g, const BubbleParams &bp,
 
 // Gather of p0 at a bubble (BubbleInterpolationScalarKernel,
 // bubble_CUDA_kernel.cuh:361-395) and the bubble's B x B stencil weights.
-template <typename F>
-__device__ inline double gather_p0(const GridParams &g, const BubbleParams &bp, const F *p0,
-                                   double x, double y, int ibnx, int ibny) {
-    const int nb = bp.mbe - bp.mbs + 1;
+template <int NB, typename F>
+__device__ inline double gather_band(const GridParams &g, const BubbleParams &bp, const F *p0,
+                                     double x, double y, int ibnx, int ibny) {
+    const int nb = NB ? NB : bp.mbe - bp.mbs + 1;
+    const Weights<NB> Dx(bp.dcx, bp.dcy, ibnx + bp.mbs, nb, g.dx, x);
+    const Weights<NB> Dy(bp.dcx, bp.dcz, ibny + bp.mbs, nb, g.dy, y);
     double PL = 0.0;
+#pragma unroll
     for (int a = 0; a < nb; a++) {
         const int i = ibnx + bp.mbs + a;
-        const double Dx = delta_w(bp.dcx, bp.dcy, i, g.dx, x);
+#pragma unroll
         for (int c = 0; c < nb; c++) {
             const int j = ibny + bp.mbs + c;
-            const double Dy = delta_w(bp.dcx, bp.dcz, j, g.dy, y);
             if (i >= 0 && i <= g.N + 1 && j >= 0 && j <= g.M + 1) {
 #pragma clang fp contract(off)
-                PL += (double)p0[frame_off(i, j, g.pitch)] * Dx * Dy;
+                PL += (double)p0[frame_off(i, j, g.pitch)] * Dx[a] * Dy[c];
             }
         }
     }
     return PL;
+}
+template <typename F>
+__device__ inline double gather_p0(const GridParams &g, const BubbleParams &bp, const F *p0,
+                                   double x, double y, int ibnx, int ibny) {
+    return bp.mbe - bp.mbs == 1 ? gather_band<2>(g, bp, p0, x, y, ibnx, ibny)
+                                : gather_band<0>(g, bp, p0, x, y, ibnx, ibny);
 }
 
 // Per-wavefront aggregation of the void-fraction scatter in LDS: an
@@ -231,15 +262,13 @@ __device__ inline void agg_flush(WaveAgg &A, int lane, int64_t *fg) {
 // VoidFractionReverseLookupKernel's per-bubble scatter (bubble_CUDA_kernel.cuh:
 // 576-619): fg_temp times the B x B smooth-delta weights, as int64 fixed
 // point, added to the wavefront's table.
-__device__ inline void scatter_bubble_agg(const GridParams &g, const BubbleParams &bp, double x,
-                                          double y, int ibnx, int ibny, double fg_temp,
-                                          WaveAgg &A, int64_t *fg, bool *bad) {
-    const int nb = bp.mbe - bp.mbs + 1;
-    double wx[kMaxBand], wy[kMaxBand];
-    for (int a = 0; a < nb; a++) {
-        wx[a] = delta_w(bp.dcx, bp.dcy, ibnx + bp.mbs + a, g.dx, x);
-        wy[a] = delta_w(bp.dcx, bp.dcz, ibny + bp.mbs + a, g.dy, y);
-    }
+template <int NB>
+__device__ inline void scatter_band(const GridParams &g, const BubbleParams &bp, double x,
+                                    double y, int ibnx, int ibny, double fg_temp, WaveAgg &A,
+                                    int64_t *fg, bool *bad) {
+    const int nb = NB ? NB : bp.mbe - bp.mbs + 1;
+    const Weights<NB> wx(bp.dcx, bp.dcy, ibnx + bp.mbs, nb, g.dx, x);
+    const Weights<NB> wy(bp.dcx, bp.dcz, ibny + bp.mbs, nb, g.dy, y);
     for (int a = 0; a < nb; a++) {
         const int i = ibnx + bp.mbs + a;
         for (int c = 0; c < nb; c++) {
@@ -255,6 +284,14 @@ __device__ inline void scatter_bubble_agg(const GridParams &g, const BubbleParam
             }
         }
     }
+}
+__device__ inline void scatter_bubble_agg(const GridParams &g, const BubbleParams &bp, double x,
+                                          double y, int ibnx, int ibny, double fg_temp,
+                                          WaveAgg &A, int64_t *fg, bool *bad) {
+    if (bp.mbe - bp.mbs == 1)
+        scatter_band<2>(g, bp, x, y, ibnx, ibny, fg_temp, A, fg, bad);
+    else
+        scatter_band<0>(g, bp, x, y, ibnx, ibny, fg_temp, A, fg, bad);
 }
 
 __device__ inline unsigned long long lanemask_lt(int lane) {
@@ -1060,7 +1097,10 @@ void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                    const BubbleArrays &b, const F *vx, const F *vy, StepScalars *sc) {
     if (b.n <= 0) return;
     const int nblk = (b.n + 255) / 256;
-    hipLaunchKernelGGL(k_motion<F>, dim3(nblk), dim3(256), 0, s, g, bp, b, vx, vy, sc);
+    if (bp.mbe - bp.mbs == 1)
+        hipLaunchKernelGGL((k_motion<F, 2>), dim3(nblk), dim3(256), 0, s, g, bp, b, vx, vy, sc);
+    else
+        hipLaunchKernelGGL((k_motion<F, 0>), dim3(nblk), dim3(256), 0, s, g, bp, b, vx, vy, sc);
 }
 
 // Workgroups of the persistent RP kernel: as many as fit (two per CU) when
