@@ -396,14 +396,15 @@ __device__ inline crpl *rpl(const RPLaunch *p) {
 }
 
 // PAIRS (launches with long chains): the queue's extreme entries after the
-// dedicated ones run on lane pairs of the shared wavefronts, spread over all
-// of them (at most 32 to a wavefront), before the others are taken a lane
-// each; and once the queue is empty a wavefront with at most 32 bubbles left
+// dedicated ones run on lane pairs of the shared wavefronts, 32 to a wavefront
+// (spread thinner over all of them they leave lanes idle and end no sooner:
+// 1, 8, 16, 24 or 32 at least to a wavefront, ms for 16 steps of 2^22 bubbles:
+// 189 / 188 / - / 178 / 178, 10 of 65 536: 46.7 / 42.3 / 40.5 / 39.6 / 40.5),
+// before the others are taken a lane each; and once the queue is empty a wavefront with at most 32 bubbles left
 // moves them onto lane pairs.  A pair does a sub-step in 0.7 of a lane's time,
 // and a chain of the 257th rank is nearly as long as the first: RP launch of
-// 2^20 bubbles 2142 -> 1476 us, 2^22 (with the full grid) 2523 -> 2060,
-// 30 011 1640 -> 1510; 65 536 at the onset of cavitation 1207 -> 1250.  256
-// VGPRs, so that two wavefronts fit a SIMD; held to that by the attribute for
+// 2^20 bubbles 2142 -> 1476 us, 2^22 (with the full grid) 2523 -> 1907,
+// 30 011 1640 -> 1460, 65 536 1207 -> 1110.  At most 256 VGPRs, so that two wavefronts fit a SIMD; held to that by the attribute for
 // two the compiler spills nine, and a launch without long chains took 12 %
 // more.
 //
@@ -467,8 +468,7 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         E = min(min(X, (int)gridDim.x), solo_cap);
         if (!PAIRS) X = E;
     }
-    // lane pairs of a shared wavefront for the entries [E, X)
-    const int quota_x = min(32, (X - E + 4 * (int)gridDim.x - 1 - E) / (4 * (int)gridDim.x - E));
+    constexpr int quota_x = 32;  // lane pairs of a shared wavefront, for the entries [E, X)
     RPPhase phase = PAIRS && X > E ? kOnPairs : kOnLanes;  // wave-uniform
     const bool odd = lane & 1;
     int idx = -1;                  // bubble of this lane, -1 when idle
