@@ -469,7 +469,18 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         if (!PAIRS) X = E;
     }
     constexpr int quota_x = 32;  // lane pairs of a shared wavefront, for the entries [E, X)
-    RPPhase phase = PAIRS && X > E ? kOnPairs : kOnLanes;  // wave-uniform
+    // The first batch of extreme entries of each shared wavefront is its own by
+    // its place, a workgroup after the other, the rest are drawn: the second
+    // workgroup of a compute unit holds long chains only when the first of
+    // every one does.
+    const int waves_x = 4 * (int)gridDim.x - E;  // shared wavefronts
+    const int w = (int)(threadIdx.x >> 6);
+    int batch_next =
+        quota_x * ((int)blockIdx.x * 4 + w - min((int)blockIdx.x + (w > 0), E));  // wave-uniform
+    int batch_end = min(batch_next + quota_x, X - E);
+    const bool solo_start = w == 0 && (int)blockIdx.x < E;
+    if (solo_start || batch_next >= batch_end) batch_next = batch_end = 0;
+    RPPhase phase = PAIRS && (batch_end > 0 || X - E > quota_x * waves_x) ? kOnPairs : kOnLanes;
     const bool odd = lane & 1;
     int idx = -1;                  // bubble of this lane, -1 when idle
     bool reuse = false;            // idx keeps its previous iteration's results
@@ -478,9 +489,8 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         idx = rpl(kp)->b.order[blockIdx.x];
         pre = true;
     }
-    bool solo = threadIdx.x < 64 && (int)blockIdx.x < E;  // wave-uniform
+    bool solo = solo_start;  // wave-uniform
     if (solo) __builtin_amdgcn_s_setprio(3);
-    int batch_next = 0, batch_end = 0;  // wave-uniform
     int head = (int)blockIdx.x & (kQueueHeads - 1);  // wave-uniform
     bool exhausted = false;             // wave-uniform
     RPLane L;              // operation-by-operation path
@@ -514,12 +524,16 @@ __global__ __launch_bounds__(256) void k_bubble_persistent(const RPLaunch *kp, i
         bool fresh = pre;
         pre = false;
         while (m != 0ull && !exhausted) {
-            if (batch_next >= batch_end &&
-                !queue_batch(b.heads + (pairs ? kQueueHeads * kHeadStride : 0), lane,
-                             pairs ? X - E : nb - X, pairs ? quota_x : quota, head, batch_next,
-                             batch_end)) {
-                exhausted = true;
-                break;
+            if (batch_next >= batch_end) {
+                const int first = pairs ? quota_x * waves_x : 0;  // the first batches went by place
+                if (!queue_batch(b.heads + (pairs ? kQueueHeads * kHeadStride : 0), lane,
+                                 (pairs ? X - E : nb - X) - first, pairs ? quota_x : quota, head,
+                                 batch_next, batch_end)) {
+                    exhausted = true;
+                    break;
+                }
+                batch_next += first;
+                batch_end += first;
             }
             const int avail = batch_end - batch_next;
             const int rank = __popcll(m & lanemask_lt(lane));
