@@ -112,7 +112,16 @@ struct StepScalars {
     int focal_i[256];
 };
 
+// Picard iterations go on while the residual over the ambient pressure is
+// above this (bubble_CUDA.cu:243).
+constexpr double kPicardTol = (double)1.0e-7f;
+
 #if defined(__HIPCC__)
+// Whether a step needs its first Picard iteration, for kernels queued before
+// the host knows: its own test (p_inf = 0: the host has decided).
+__device__ inline bool picard_needed(const StepScalars *sc, double p_inf) {
+    return p_inf == 0.0 || __longlong_as_double((long long)sc->resid[0]) / p_inf > kPicardTol;
+}
 // One word of a report.  Report words bypass the caches, one by one: a release
 // at system scope would write back every dirty line of the XCD's L2 first.
 __device__ inline void report_word(unsigned long long *dst, unsigned long long v) {
@@ -346,10 +355,12 @@ enum RPGrid { kRPLean, kRPFull, kRPLight };
 // The RP launch of Picard iteration `slot` over the queue order, with the
 // gathered pressures of launch_queue_keys in PL[plp].
 // Returns the number of wavefronts launched (their records in b.totals).
+// p_inf as in picard_needed: where no iteration is needed, the launch and
+// launch_queue_keys leave everything as it is.
 template <typename F>
 int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
                         int plm, int pln, int plp, const F *p0, int64_t *fg_target, StepScalars *sc,
-                        int slot, RPGrid shape, int cus, int per_cu);
+                        int slot, RPGrid shape, int cus, int per_cu, double p_inf);
 // Whether the launch runs every bubble on a lane pair, and whether it then
 // needs no queue (it gathers the pressures itself).
 bool bubble_step_pairs(const RPLaunch &host, int cus);
@@ -367,9 +378,9 @@ RPGrid bubble_step_grid(int sub_max, double sub_per_launch, int extreme_threshol
 template <typename F>
 void launch_queue_keys(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                        const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext,
-                       StepScalars *sc);
+                       StepScalars *sc, double p_inf);
 void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key, int threshold,
-                            int ext);
+                            int ext, const StepScalars *sc, double p_inf);
 void launch_scatter_initial(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                             const BubbleArrays &b, int64_t *fg_target, StepScalars *sc);
 void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg);

@@ -712,7 +712,7 @@ __global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int ma
                                                       int pln, int plp, const F *__restrict__ p0,
                                                       int64_t *__restrict__ fg_target,
                                                       StepScalars *sc, int slot, int quota,
-                                                      int solo_cap) {
+                                                      int solo_cap, double p_inf) {
     set_mark(sc, kMarkRP);
     const int lane = threadIdx.x & 63;
     const bool odd = lane & 1;
@@ -722,9 +722,11 @@ __global__ __launch_bounds__(256) void k_bubble_pairs(const RPLaunch *kp, int ma
     __shared__ double shc[16];
     WaveAgg &agg = agg_all[threadIdx.x >> 6];
     agg_clear(agg, lane);
+    const bool needed = ORDERED || picard_needed(sc, p_inf);  // ORDERED: the queue is empty
     rp_vtab_stage(rp_shared, vtab);
     if (threadIdx.x < 15) shc[threadIdx.x] = rp_shared[threadIdx.x];
     __syncthreads();
+    if (!needed) return;
     const ldouble *t = (const ldouble *)shc;
     const RPFastShared fsh{t[0], t[1], t[2],  t[3],  t[4],  t[5],  t[6], t[7],
                            t[8], t[9], t[10], t[11], t[12], t[13], t[14], vtab};
@@ -1167,7 +1169,8 @@ bool bubble_step_unordered(const RPLaunch &host, int cus) {
 template <typename F>
 int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev, int cur,
                         int plm, int pln, int plp, const F *p0, int64_t *fg_target,
-                        StepScalars *sc, int slot, RPGrid shape, int cus, int per_cu) {
+                        StepScalars *sc, int slot, RPGrid shape, int cus, int per_cu,
+                        double p_inf) {
     if (host.b.n <= 0) return 0;
     const int cap = host.bp.max_substeps;
     if (bubble_step_pairs(host, cus)) {
@@ -1176,11 +1179,11 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
         if (n <= waves)
             hipLaunchKernelGGL((k_bubble_pairs<F, false>), dim3(blocks), dim3(256), 0, s,
                                dev, cap, host.bp.rp_shared, cur, plm, pln, plp, p0, fg_target, sc,
-                               slot, 1, 0);
+                               slot, 1, 0, p_inf);
         else
             hipLaunchKernelGGL((k_bubble_pairs<F, true>), dim3(blocks), dim3(256), 0, s, dev, cap,
                                host.bp.rp_shared, cur, plm, pln, plp, p0, fg_target, sc, slot,
-                               (n + waves - 1) / waves, cus);
+                               (n + waves - 1) / waves, cus, p_inf);
         return 4 * blocks;
     }
     const bool lean = shape == kRPLean;
@@ -1211,13 +1214,16 @@ constexpr int kSortBins = 2048;  // bins of the extreme-class sort
 
 __global__ __launch_bounds__(256) void k_part_count(const int *sub, int n, int ext, int thr,
                                                     int *cntE, int *cntH, int *sort_hist,
-                                                    unsigned int *heads) {
+                                                    unsigned int *heads, const StepScalars *sc,
+                                                    double p_inf) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
+    // not needed: an empty queue (no classes, and the heads past any end)
+    const bool needed = picard_needed(sc, p_inf);
     if (blockIdx.x == 0) {
         for (int k = threadIdx.x; k < kSortBins; k += 256) sort_hist[k] = 0;
-        if (threadIdx.x < 2 * kQueueHeads) heads[threadIdx.x * kHeadStride] = 0u;
+        if (threadIdx.x < 2 * kQueueHeads) heads[threadIdx.x * kHeadStride] = needed ? 0u : 0x40000000u;
     }
-    const int v = idx < n ? sub[idx] : 0;
+    const int v = idx < n && needed ? sub[idx] : 0;
     const int ce = __syncthreads_count(idx < n && v >= ext);
     const int ch = __syncthreads_count(idx < n && v >= thr && v < ext);
     if (threadIdx.x == 0) {
@@ -1395,7 +1401,9 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const int *sub, const int 
 template <typename F>
 __global__ __launch_bounds__(256) void k_queue_keys(GridParams g, BubbleParams bp, BubbleArrays b,
                                                     const F *__restrict__ p0, int cur, int plp,
-                                                    int slot, int ext, StepScalars *sc) {
+                                                    int slot, int ext, StepScalars *sc,
+                                                    double p_inf) {
+    if (!picard_needed(sc, p_inf)) return;
     set_mark(sc, kMarkQueue);
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= b.n) return;
@@ -1433,25 +1441,25 @@ __global__ __launch_bounds__(256) void k_queue_keys(GridParams g, BubbleParams b
 template <typename F>
 void launch_queue_keys(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                        const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext,
-                       StepScalars *sc) {
+                       StepScalars *sc, double p_inf) {
     if (b.n <= 0) return;
     hipLaunchKernelGGL(k_queue_keys<F>, dim3((b.n + 255) / 256), dim3(256), 0, s, g, bp, b, p0,
-                       cur, plp, slot, ext, sc);
+                       cur, plp, slot, ext, sc, p_inf);
 }
 template void launch_queue_keys<double>(hipStream_t, const GridParams &, const BubbleParams &,
                                         const BubbleArrays &, const double *, int, int, int, int,
-                                        StepScalars *);
+                                        StepScalars *, double);
 template void launch_queue_keys<float>(hipStream_t, const GridParams &, const BubbleParams &,
                                        const BubbleArrays &, const float *, int, int, int, int,
-                                       StepScalars *);
+                                       StepScalars *, double);
 
 void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key, int threshold,
-                            int ext) {
+                            int ext, const StepScalars *sc, double p_inf) {
     if (b.n <= 0) return;
     const int nblk = (b.n + 255) / 256;
     int *cntE = b.part, *cntH = b.part + (nblk + 1);
     hipLaunchKernelGGL(k_part_count, dim3(nblk), dim3(256), 0, s, key, b.n, ext, threshold,
-                       cntE, cntH, b.sort_hist, b.heads);
+                       cntE, cntH, b.sort_hist, b.heads, sc, p_inf);
     hipLaunchKernelGGL(k_part_scan, dim3(2), dim3(1024), 0, s, cntE, nblk);
     hipLaunchKernelGGL(k_part_scatter, dim3(nblk), dim3(256), 0, s, key, b.n, ext, threshold,
                        cntE, cntH, nblk, b.order, b.order_tmp);
@@ -1534,9 +1542,9 @@ template void launch_motion<float>(hipStream_t, const GridParams &, const Bubble
                                    StepScalars *);
 template int launch_bubble_step<double>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
                                          int, int, const double *, int64_t *, StepScalars *, int, RPGrid, int,
-                                         int);
+                                         int, double);
 template int launch_bubble_step<float>(hipStream_t, const RPLaunch &, const RPLaunch *, int, int,
                                          int, int, const float *, int64_t *, StepScalars *, int, RPGrid, int,
-                                         int);
+                                         int, double);
 
 }  // namespace brp
