@@ -45,6 +45,7 @@ struct GridParams {
     double fp_x, fp_y, fdist;  // control point and focal distance
     int ap_lo, ap_hi, n_elem;  // aperture cells and element count (E4)
     double s3;           // dt * rho_l * c * c   (MixturePressureKernel)
+    int ahead = 0;  // queued before the host knows the step before (halted)
 };
 
 __host__ __device__ inline int64_t frame_off(int i, int j, int pitch) {
@@ -107,6 +108,7 @@ struct StepScalars {
     // The step's phases in ticks of the device's constant-rate clock: marks
     // that kernels set, and the phases' sums (brp_get_phase_times' order).
     unsigned long long mark[kMarks], phase[5];
+    int halt;                            // the last evaluation's flags & 3
     unsigned long long resid[kMaxEval];  // max |dp0| bit patterns (>= 0 doubles)
     double focal_v[256];                 // per-block maxima of the focal-point search
     int focal_i[256];
@@ -117,6 +119,11 @@ struct StepScalars {
 constexpr double kPicardTol = (double)1.0e-7f;
 
 #if defined(__HIPCC__)
+// Whether the step before has failed, for kernels queued before the host knows:
+// they leave everything as that step left it.
+__device__ inline bool halted(const GridParams &g, const StepScalars *sc) {
+    return g.ahead && sc->halt != 0;
+}
 // Whether a step needs its first Picard iteration, for kernels queued before
 // the host knows: its own test (p_inf = 0: the host has decided).
 __device__ inline bool picard_needed(const StepScalars *sc, double p_inf) {

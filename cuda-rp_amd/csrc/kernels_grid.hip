@@ -88,6 +88,7 @@ __global__ __launch_bounds__(256) void k_velocity(GridParams g, F *__restrict__ 
                                                    const F *__restrict__ cxb,
                                                    const F *__restrict__ cya,
                                                    const F *__restrict__ cyb, StepScalars *sc) {
+    if (halted(g, sc)) return;
     set_mark(sc, kMarkVelocity);
     typedef typename Vec4<F>::type V;
     const int lane = threadIdx.x;
@@ -171,6 +172,7 @@ __global__ __launch_bounds__(256) void k_velocity_small(GridParams g, F *__restr
                                                         const F *__restrict__ cya,
                                                         const F *__restrict__ cyb,
                                                         StepScalars *sc) {
+    if (halted(g, sc)) return;
     set_mark(sc, kMarkVelocity);
     const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
     if (i > g.N || j > g.M) return;
@@ -242,6 +244,7 @@ __device__ inline double focused_value(const GridParams &g, int i, double t, dou
 template <typename F>
 __global__ __launch_bounds__(256) void k_velocity_ghosts(GridParams g, F *vx, F *vy, double t,
                                                          StepScalars *sc, int nslots) {
+    if (halted(g, sc)) return;
     const int N = g.N, M = g.M, P = g.pitch;
     const int k = blockIdx.x * 256 + threadIdx.x;
     for (int q = k; q < nslots; q += gridDim.x * 256) sc->resid[q] = 0ull;
@@ -336,6 +339,7 @@ __global__ __launch_bounds__(256) void k_pressure_first(
     int64_t *__restrict__ fg_mp, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
     const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
     const double *__restrict__ rxp, StepScalars *sc) {
+    if (halted(g, sc)) return;
     set_mark(sc, kMarkPressure);
     typedef typename Vec4<F>::type V;
     const int lane = threadIdx.x;
@@ -449,6 +453,7 @@ __global__ __launch_bounds__(256) void k_pressure_first_small(
     int64_t *__restrict__ fg_mp, Window w, const F *__restrict__ ax, const F *__restrict__ bx,
     const F *__restrict__ ay, const F *__restrict__ by, const double *__restrict__ xu,
     const double *__restrict__ rxp, StepScalars *sc) {
+    if (halted(g, sc)) return;
     set_mark(sc, kMarkPressure);
     const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
     double rmax = 0.0;
@@ -579,6 +584,7 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           const int *bbox_blk, int n_bbox,
                                                           StepScalars *sc, StepReport *rep,
                                                           unsigned long long seq) {
+    if (halted(g, sc)) return;
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
     const unsigned long long began = wall_clock64();
@@ -686,6 +692,7 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
         out.reused = sc->reused;
         for (int k = 0; k < 5; k++) out.phase[k] = sc->phase[k] = ph[k];
         sc->mark[kMarkQueue] = 0ull;
+        sc->halt = sc->flags & 3;
     }
     __syncthreads();
     constexpr int words = offsetof(StepReport, focal) / 8;
