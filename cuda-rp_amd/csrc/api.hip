@@ -898,6 +898,14 @@ int schedule_record_call(brp_handle *h) {
     return BRP_OK;
 }
 
+// The clock: compensated sum (bubble_CUDA.cu:208-212).
+void advance_clock(const brp_handle *h, double &t, double &tx) {
+    const double s1 = t;
+    t = t + h->dt + tx;
+    const double s2 = t - s1;
+    tx = h->dt + tx - s2;
+}
+
 template <typename F>
 int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullptr) {
     const int max_pic = std::min(h->cfg.max_picard > 0 ? h->cfg.max_picard : 1000, kMaxEval - 1);
@@ -951,18 +959,24 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         return set_err(h, st.status, "step %lld: %s (flags %d, Picard %d)", (long long)h->nstep,
                        "non-finite value or void fraction out of range", r->flags, 0);
     };
+    // A step's launches up to the bubbles' motion.
+    const auto launch_first = [&](const GridParams &g, const int64_t *fg, int first, double t,
+                                  bool motion) {
+        launch_velocity<F>(s, g, vx, vy, p0, fg, h->W, first, cxa, cxb, cya, cyb, h->sc_d);
+        launch_velocity_ghosts<F>(s, g, vx, vy, t, h->sc_d, max_pic + 1);
+        if (bub && motion) launch_motion<F>(s, g, h->bp, h->b, vx, vy, h->sc_d);
+    };
+    int started = 0;  // iterations after which the next step's were queued ahead
     for (int step = 0; step < k; step++) {
         if (ahead_steps && step >= kStepsAhead)
             if (int rc = read_behind(step - kStepsAhead)) return rc;
         GridParams g = h->g;
         g.ahead = ahead_steps && step > 0;
         brp_step_stats st{};
-        // clock: compensated sum (bubble_CUDA.cu:208-212)
         h->nstep++;
-        const double s1 = h->t;
-        h->t = h->t + h->dt + h->tx;
-        const double s2 = h->t - s1;
-        h->tx = h->dt + h->tx - s2;
+        advance_clock(h, h->t, h->tx);
+        const int started_before = started;
+        started = 0;
         // store_variables (kernel.cuh:1229-1262) as renamings: pn <- p,
         // (f_gm, f_gn, f_g) <- (f_gn, f_g, prediction), PL history shift.
         const int pn_i = h->pc, p_i = h->pc ^ 1;
@@ -1000,17 +1014,14 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             rec->first = h->first_step;
             rec->t = h->t;
         }
-        launch_velocity<F>(s, g, vx, vy, p0, h->fgb[old_cur], h->W, h->first_step, cxa, cxb,
-                           cya, cyb, h->sc_d);
-        launch_velocity_ghosts<F>(s, g, vx, vy, h->t, h->sc_d, max_pic + 1);
         // a blind replay takes the positions after the motion from the tape
         BubbleArrays bnow = h->b;
         if (blind) {
             bnow.x = ctl->tape_in->x_end;
             bnow.y = ctl->tape_in->y_end;
-        } else if (bub) {
-            launch_motion<F>(s, h->g, h->bp, h->b, vx, vy, h->sc_d);
         }
+        if (started_before == 0 || started_before != h->last_n_pic)
+            launch_first(g, h->fgb[old_cur], h->first_step, h->t, !blind);
         launch_pressure_first<F>(s, g, vx, vy, (F *)h->pb[pn_i][0], (F *)h->pb[pn_i][1],
                                  (F *)h->pb[p_i][0], (F *)h->pb[p_i][1], p0, h->fgb[old_cur],
                                  h->fgb[old_n], h->fgb[old_m], h->W, ax, bx, ay, by, h->xu_d,
@@ -1020,7 +1031,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                   blind         ? nullptr
                                   : ahead_steps ? h->rep_ahead + step % kStepsAhead
                                                 : h->rep,
-                                  blind ? 0 : ++h->rep_seq);
+                                  blind ? 0 : ++h->rep_seq, 0u);
         // A Picard iteration's RP call, up to the new void fraction: the window
         // is not needed yet, so the first iteration's is queued before the
         // report above is there, while the host would wait for it (p_inf: it
@@ -1136,7 +1147,20 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 if (!blind || !pressure_ghosts_fixed(h->g))
                     launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
                                               h->b.totals, rp_waves, nullptr, 0, h->sc_d,
-                                              blind ? nullptr : h->rep, blind ? 0 : ++h->rep_seq);
+                                              blind ? nullptr : h->rep, blind ? 0 : ++h->rep_seq,
+                                              (unsigned)h->nb * (unsigned)loop);
+                // The step probably ends here, as the one before did: the next
+                // one's first launches, which halt on the device if it does not
+                // (256^2 with 1024 bubbles at rest 84 -> 75 us a step)
+                if (!ctl && !h->cfg.thermal && h->sched_mode == 0 && step + 1 < k &&
+                    loop == h->last_n_pic && h->P_inf != 0.0) {
+                    double t = h->t, tx = h->tx;
+                    advance_clock(h, t, tx);
+                    GridParams gn = h->g;
+                    gn.ahead = 1;
+                    launch_first(gn, h->fgb[target], 0, t, true);
+                    started = loop;
+                }
                 if (rec && rec->want_grid) {  // the iterate that the evaluation read, and its pressure
                     RectPlan rp;
                     rp.add(rec->fg_it[loop], h->fgb[target], sizeof(int64_t));

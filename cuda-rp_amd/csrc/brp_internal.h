@@ -45,7 +45,7 @@ struct GridParams {
     double fp_x, fp_y, fdist;  // control point and focal distance
     int ap_lo, ap_hi, n_elem;  // aperture cells and element count (E4)
     double s3;           // dt * rho_l * c * c   (MixturePressureKernel)
-    int ahead = 0;  // queued before the host knows the step before (halted)
+    int ahead = 0;  // queued before the host knows how the step before ends (halted)
 };
 
 __host__ __device__ inline int64_t frame_off(int i, int j, int pitch) {
@@ -108,7 +108,7 @@ struct StepScalars {
     // The step's phases in ticks of the device's constant-rate clock: marks
     // that kernels set, and the phases' sums (brp_get_phase_times' order).
     unsigned long long mark[kMarks], phase[5];
-    int halt;                            // the last evaluation's flags & 3
+    int halt;                            // the step does not end with the last evaluation
     unsigned long long resid[kMaxEval];  // max |dp0| bit patterns (>= 0 doubles)
     double focal_v[256];                 // per-block maxima of the focal-point search
     int focal_i[256];
@@ -119,8 +119,8 @@ struct StepScalars {
 constexpr double kPicardTol = (double)1.0e-7f;
 
 #if defined(__HIPCC__)
-// Whether the step before has failed, for kernels queued before the host knows:
-// they leave everything as that step left it.
+// Whether the step before goes on or has failed, for kernels of the next step
+// queued before the host knows: they leave everything as it is.
 __device__ inline bool halted(const GridParams &g, const StepScalars *sc) {
     return g.ahead && sc->halt != 0;
 }
@@ -345,7 +345,7 @@ template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
                             const double *el_phase, double t, int eval, const RPTotals *tot,
                             int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
-                            StepReport *rep, unsigned long long seq);
+                            StepReport *rep, unsigned long long seq, unsigned int done_want);
 // Whether a Picard iteration's evaluation changes no ghost cell of p0: they
 // hold the source row, or nothing, and mirror no wall.
 inline bool pressure_ghosts_fixed(const GridParams &g) {

@@ -97,6 +97,7 @@ template <typename F, int NB>
 __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, BubbleArrays b,
                                                  const F *__restrict__ vx,
                                                  const F *__restrict__ vy, StepScalars *sc) {
+    const bool stop = halted(g, sc);  // tested where it writes: the load's time passes meanwhile
     set_mark(sc, kMarkMotion);
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     int imin = 0x7fffffff, imax = -0x7fffffff, jmin = 0x7fffffff, jmax = -0x7fffffff;
@@ -132,16 +133,20 @@ __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, B
                     vLy += (double)vy[frame_off(i, j, g.pitch)] * wxn[a] * wym[c];
             }
         }
-        b.vx[idx] = vLx;
-        b.vy[idx] = vLy;
+        if (!stop) {
+            b.vx[idx] = vLx;
+            b.vy[idx] = vLy;
+        }
         double nx, ny;
         {
 #pragma clang fp contract(off)
             nx = x + vLx * g.dt;
             ny = y + vLy * g.dt;
         }
-        b.x[idx] = nx;
-        b.y[idx] = ny;
+        if (!stop) {
+            b.x[idx] = nx;
+            b.y[idx] = ny;
+        }
         const int kx = bin_index(nx, g.rdx, 0.5), ky = bin_index(ny, g.rdy, 0.5);
         imin = max(kx + bp.mbs, 0);
         imax = min(kx + bp.mbe, g.N + 1);
@@ -154,6 +159,7 @@ __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, B
             jmax = -0x7fffffff;
         }
     }
+    if (stop) return;
     block_bbox(imin, imax, jmin, jmax, b.bbox_blk);
 }
 

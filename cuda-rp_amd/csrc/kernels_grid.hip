@@ -583,7 +583,8 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           int eval, const RPTotals *tot, int n_tot,
                                                           const int *bbox_blk, int n_bbox,
                                                           StepScalars *sc, StepReport *rep,
-                                                          unsigned long long seq) {
+                                                          unsigned long long seq,
+                                                          unsigned int done_want) {
     if (halted(g, sc)) return;
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -692,7 +693,10 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
         out.reused = sc->reused;
         for (int k = 0; k < 5; k++) out.phase[k] = sc->phase[k] = ph[k];
         sc->mark[kMarkQueue] = 0ull;
-        sc->halt = sc->flags & 3;
+        // the host's own tests of whether the step ends here, without error
+        sc->halt = eval == 0 ? out.flags & 3
+                             : out.flags != 0 || out.done != done_want ||
+                                   out.resid / g.P_inf > kPicardTol;
     }
     __syncthreads();
     constexpr int words = offsetof(StepReport, focal) / 8;
@@ -782,9 +786,9 @@ template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
                             const double *el_phase, double t, int eval, const RPTotals *tot,
                             int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
-                            StepReport *rep, unsigned long long seq) {
+                            StepReport *rep, unsigned long long seq, unsigned int done_want) {
     hipLaunchKernelGGL(k_pressure_ghosts<F>, dim3(1), dim3(1024), 0, s, g, p0, el_amp,
-                       el_phase, t, eval, tot, n_tot, bbox_blk, n_bbox, sc, rep, seq);
+                       el_phase, t, eval, tot, n_tot, bbox_blk, n_bbox, sc, rep, seq, done_want);
 }
 
 void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
@@ -808,7 +812,8 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
     template void launch_pressure_ghosts<F>(hipStream_t, const GridParams &, F *,           \
                                             const double *, const double *, double, int,     \
                                             const RPTotals *, int, const int *, int,         \
-                                            StepScalars *, StepReport *, unsigned long long);
+                                            StepScalars *, StepReport *, unsigned long long,  \
+                                            unsigned int);
 
 BRP_INST(double)
 BRP_INST(float)
