@@ -962,8 +962,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
     // A step's launches up to the bubbles' motion.
     const auto launch_first = [&](const GridParams &g, const int64_t *fg, int first, double t,
                                   bool motion) {
-        launch_velocity<F>(s, g, vx, vy, p0, fg, h->W, first, cxa, cxb, cya, cyb, h->sc_d);
-        launch_velocity_ghosts<F>(s, g, vx, vy, t, h->sc_d, max_pic + 1);
+        launch_velocity<F>(s, g, vx, vy, p0, fg, h->W, first, cxa, cxb, cya, cyb, t, h->sc_d,
+                           max_pic + 1);
         if (bub && motion) launch_motion<F>(s, g, h->bp, h->b, vx, vy, h->sc_d);
     };
     int started = 0;  // iterations after which the next step's were queued ahead

@@ -321,14 +321,11 @@ inline void rp_table_values(const BubbleParams &bp, double v[kRpTable]) {
 
 // Kernel launchers (kernels_*.hip).  All run on stream s.
 namespace brp {
+// Velocity and its boundary at time t; clears the step's scalars.
 template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
-                     const int64_t *fgn, Window w, int first_step, const F *cvx_a,
-                     const F *cvx_b, const F *cvy_a, const F *cvy_b, StepScalars *sc);
-template <typename F>
-// Also clears the step's scalars (resid[0, nslots)).
-void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t,
-                            StepScalars *sc, int nslots);
+                     const int64_t *fgn, Window w, int first_step, const F *cxa, const F *cxb,
+                     const F *cya, const F *cyb, double t, StepScalars *sc, int nslots);
 template <typename F>
 void launch_pressure_first(hipStream_t s, const GridParams &g, const F *vx, const F *vy,
                            const F *pnx, const F *pny, F *px, F *py, F *p0,

@@ -159,41 +159,6 @@ __global__ __launch_bounds__(256) void k_velocity(GridParams g, F *__restrict__ 
     }
 }
 
-// The same update for a grid that k_velocity would cover with too few
-// wavefronts (velocity_small): one cell per thread, so that no thread walks rows
-// one after another (256^2 FP64 beside a cloud: 16.3 -> 4.1 us).
-template <typename F>
-__global__ __launch_bounds__(256) void k_velocity_small(GridParams g, F *__restrict__ vx,
-                                                        F *__restrict__ vy,
-                                                        const F *__restrict__ p0,
-                                                        const int64_t *__restrict__ fgn, Window w,
-                                                        int first, const F *__restrict__ cxa,
-                                                        const F *__restrict__ cxb,
-                                                        const F *__restrict__ cya,
-                                                        const F *__restrict__ cyb,
-                                                        StepScalars *sc) {
-    if (halted(g, sc)) return;
-    set_mark(sc, kMarkVelocity);
-    const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
-    if (i > g.N || j > g.M) return;
-    const int64_t o = frame_off(i, j, g.pitch);
-    const F dt = (F)g.dt, rdx = (F)g.rdx, half = (F)0.5;
-    const F dt_rho = dt / (((F)g.rho_inf + (F)g.rho_inf) * half);
-    const bool in_w = !first && j + 1 >= w.j0 && j <= w.j1 && i + 1 >= w.i0 && i <= w.i1;
-    const F pc = p0[o], pe = p0[o + 1], pn = p0[o + g.pitch];
-    const F rc = in_w ? rho_m_at<F>(g, fgn, w, first, i, j) : (F)g.rho_inf;
-    if (j >= 1) {
-        const F s2 = (-pc + pe) * rdx;
-        const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i + 1, j)) * half) : dt_rho;
-        vx[o] = (vx[o] * cxa[i + 1] - q * s2) / cxb[i + 1];
-    }
-    if (i >= 1) {
-        const F s2 = (-pc + pn) * rdx;  // rdx, as the reference (kernel.cuh:671)
-        const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i, j + 1)) * half) : dt_rho;
-        vy[o] = (vy[o] * cya[j + 1] - q * s2) / cyb[j + 1];
-    }
-}
-
 __device__ inline void clear_scalars(StepScalars *sc) {
     sc->bbox[0] = 0x7fffffff;
     sc->bbox[1] = -0x7fffffff;
@@ -230,6 +195,13 @@ __device__ inline double focused_value(const GridParams &g, int i, double t, dou
         }
         return 0.0;
     }
+    return 0.0;
+}
+
+// The plane velocity source at time t.
+__device__ inline double plane_value(const GridParams &g, double t) {
+    if (fmod(t, ((double)g.on_wave + (double)g.off_wave) / g.freq) <= ((double)g.on_wave) / g.freq)
+        return g.amp * sin(g.omega * t);
     return 0.0;
 }
 
@@ -288,13 +260,7 @@ __global__ __launch_bounds__(256) void k_velocity_ghosts(GridParams g, F *vx, F 
             vm1 = v0;
         }
         if (g.src_row) {
-            if (g.plane_v) {
-                double v = 0.0;
-                if (fmod(t, ((double)g.on_wave + (double)g.off_wave) / g.freq) <=
-                    ((double)g.on_wave) / g.freq)
-                    v = g.amp * sin(g.omega * t);
-                v0 = (F)v;
-            }
+            if (g.plane_v) v0 = (F)plane_value(g, t);
             if (g.focused_v) v0 = (F)focused_value(g, i, t, g.amp, 0.0, nullptr, nullptr);
         }
         if (!g.pml_y1) {
@@ -319,6 +285,113 @@ __global__ __launch_bounds__(256) void k_velocity_ghosts(GridParams g, F *vx, F 
         else if (N <= M + 1)
             q = vy[frame_off(N, N, P)];
         vy[frame_off(N + 1, j, P)] = q;
+    }
+}
+
+// The velocity of a small grid (velocity_small), one cell per thread, so that
+// no thread walks rows one after another, with the boundary of
+// k_velocity_ghosts in the same launch: the thread that has a cell's new value
+// writes it to the ghost cells that copy it as well, so that none waits for
+// another (256^2 FP64: 7.3 us a step in two launches, 3.9 in one; 16.3 and 3.9
+// with k_velocity's split).  The right ghost column copies one cell in every
+// row: the workgroup of that cell writes the column.
+template <typename F>
+__global__ __launch_bounds__(256) void k_velocity_small(GridParams g, F *__restrict__ vx,
+                                                        F *__restrict__ vy,
+                                                        const F *__restrict__ p0,
+                                                        const int64_t *__restrict__ fgn, Window w,
+                                                        int first, const F *__restrict__ cxa,
+                                                        const F *__restrict__ cxb,
+                                                        const F *__restrict__ cya,
+                                                        const F *__restrict__ cyb, double t,
+                                                        StepScalars *sc, int nslots) {
+    if (halted(g, sc)) return;
+    set_mark(sc, kMarkVelocity);
+    const int N = g.N, M = g.M, P = g.pitch;
+    const int tid = threadIdx.y * kBX + threadIdx.x;
+    const bool origin = blockIdx.x == 0 && blockIdx.y == 0;
+    if (origin) {
+        for (int q = tid; q < nslots; q += 256) sc->resid[q] = 0ull;
+        if (tid == 0) clear_scalars(sc);
+    }
+    // the row of column N whose vy the right ghost column copies, -1 for none
+    const int jq = N == M + 1 && !g.pml_y1            ? M - 1
+                   : N < M || (N == M && g.pml_y1)    ? N
+                                                      : -1;
+    __shared__ F right;
+    const int i = blockIdx.x * kBX + threadIdx.x, j = blockIdx.y * kBY + threadIdx.y;
+    if (i <= N && j <= M) {
+        const int64_t o = frame_off(i, j, P);
+        const F dt = (F)g.dt, rdx = (F)g.rdx, half = (F)0.5;
+        const F dt_rho = dt / (((F)g.rho_inf + (F)g.rho_inf) * half);
+        const bool in_w = !first && j + 1 >= w.j0 && j <= w.j1 && i + 1 >= w.i0 && i <= w.i1;
+        const F pc = p0[o], pe = p0[o + 1], pn = p0[o + P];
+        const F rc = in_w ? rho_m_at<F>(g, fgn, w, first, i, j) : (F)g.rho_inf;
+        if (j >= 1) {
+            const F s2 = (-pc + pe) * rdx;
+            const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i + 1, j)) * half) : dt_rho;
+            const F v = (vx[o] * cxa[i + 1] - q * s2) / cxb[i + 1];
+            const auto rows = [&](int ii, F u) {  // rows 0 and M + 1 copy rows 1 and M
+                if (j == 1) vx[frame_off(ii, 0, P)] = u;
+                if (j == M) vx[frame_off(ii, M + 1, P)] = u;
+            };
+            const bool wall = (!g.pml_x0 && i == 0) || (!g.pml_x1 && i == N);
+            vx[o] = wall ? (F)0 : v;
+            rows(i, wall ? (F)0 : v);
+            if (!g.pml_x0 && i == 1) {
+                vx[frame_off(-1, j, P)] = v;
+                rows(-1, v);
+            }
+            if (!g.pml_x1 && i == N - 1) {
+                vx[frame_off(N + 1, j, P)] = -v;
+                rows(N + 1, -v);
+            }
+            if (j == 1 || j == M) {  // columns that no step writes
+                if (g.pml_x0 && i == 0) rows(-1, vx[frame_off(-1, j, P)]);
+                if (g.pml_x1 && i == N) rows(N + 1, vx[frame_off(N + 1, j, P)]);
+            }
+        }
+        if (i >= 1) {
+            const F s2 = (-pc + pn) * rdx;  // rdx, as the reference (kernel.cuh:671)
+            const F q = in_w ? dt / ((rc + rho_m_at<F>(g, fgn, w, first, i, j + 1)) * half) : dt_rho;
+            F v = (vy[o] * cya[j + 1] - q * s2) / cyb[j + 1];
+            const auto put = [&](int jj, F u) {  // column 0 copies column 1
+                vy[frame_off(i, jj, P)] = u;
+                if (i == 1) vy[frame_off(0, jj, P)] = u;
+            };
+            if (j == 0) {
+                F below = vy[frame_off(i, -1, P)];
+                if (!g.pml_y0) {
+                    if (!g.plane_p && !g.focused_p) v = (F)0;
+                    below = v;
+                }
+                if (g.src_row) {
+                    if (g.plane_v) v = (F)plane_value(g, t);
+                    if (g.focused_v) v = (F)focused_value(g, i, t, g.amp, 0.0, nullptr, nullptr);
+                }
+                put(-1, below);
+            }
+            if (j == M) {
+                if (!g.pml_y1)
+                    v = (F)0;
+                else
+                    put(M + 1, vy[frame_off(i, M + 1, P)]);
+            }
+            if (j == M - 1 && !g.pml_y1) put(M + 1, v);
+            put(j, v);
+            if (i == N && j == jq) right = v;
+        }
+    }
+    // vy(N + 1, j) = vy(N, N) in every row: the reference reads row
+    // vy_width*i with the loop variable i (bubble_CUDA_kernel.cuh:808)
+    const bool here = jq < 0 ? origin
+                             : (int)blockIdx.x == N / kBX && (int)blockIdx.y == jq / kBY;
+    if (here) {  // workgroup-uniform
+        __syncthreads();
+        const F q = jq >= 0                      ? right
+                    : N == M + 1 && g.pml_y1     ? vy[frame_off(N, N, P)]
+                                                 : (F)0;
+        for (int jj = tid - 1; jj <= M + 1; jj += 256) vy[frame_off(N + 1, jj, P)] = q;
     }
 }
 
@@ -719,7 +792,7 @@ __global__ void k_zero_scalars(StepScalars *sc, int nslots) {
 // Where one cell per thread is the better split: the four-cell, four-row
 // threads are fewer than a wavefront per SIMD (1024 on 256 compute units)
 // below a million cells, but they load each pressure row and velocity once.
-// With the ghost launch after it, us, four-row against one-cell threads:
+// With the ghost launch after either, us, four-row against one-cell threads:
 // velocity 256^2 15.4 / 12.9, 777^2 16.8 / 16.6 (FP32 15.3 / 13.2), 1400^2
 // 22.4 / 22.3, 2048^2 FP32 22.8 / 25.8; pressure 256^2 17.0 / 11.5, 400^2 16.4
 // / 14.1, 600^2 17.7 / 19.1, 1000^2 20.2 / 22.7.
@@ -729,22 +802,17 @@ static bool pressure_small(const GridParams &g) { return (int64_t)g.N * g.M < 30
 template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
                      const int64_t *fgn, Window w, int first_step, const F *cxa, const F *cxb,
-                     const F *cya, const F *cyb, StepScalars *sc) {
-    if (velocity_small(g)) {
+                     const F *cya, const F *cyb, double t, StepScalars *sc, int nslots) {
+    if (velocity_small(g) && std::min(g.N, g.M) >= 4) {  // (one thread for each wall)
         hipLaunchKernelGGL(k_velocity_small<F>, dim3((g.N + kBX) / kBX, (g.M + kBY) / kBY),
                            dim3(kBX, kBY), 0, s, g, vx, vy, p0, fgn, w, first_step, cxa, cxb, cya,
-                           cyb, sc);
+                           cyb, t, sc, nslots);
         return;
     }
     dim3 blk(kBX, kBY);  // columns 0..N, rows 0..M
     dim3 grd((g.N + 1 + kBX * kGW - 1) / (kBX * kGW), (g.M + 1 + kGBlockRows - 1) / kGBlockRows);
     hipLaunchKernelGGL(k_velocity<F>, grd, blk, 0, s, g, vx, vy, p0, fgn, w, first_step, cxa,
                        cxb, cya, cyb, sc);
-}
-
-template <typename F>
-void launch_velocity_ghosts(hipStream_t s, const GridParams &g, F *vx, F *vy, double t,
-                            StepScalars *sc, int nslots) {
     const int n = std::max(g.N, g.M) + 3;  // columns and rows -1 .. N + 1, M + 1
     hipLaunchKernelGGL(k_velocity_ghosts<F>, dim3((n + 255) / 256), dim3(256), 0, s, g, vx, vy, t,
                        sc, nslots);
@@ -798,9 +866,7 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
 #define BRP_INST(F)                                                                          \
     template void launch_velocity<F>(hipStream_t, const GridParams &, F *, F *, const F *,   \
                                      const int64_t *, Window, int, const F *, const F *,     \
-                                     const F *, const F *, StepScalars *);                   \
-    template void launch_velocity_ghosts<F>(hipStream_t, const GridParams &, F *, F *,      \
-                                            double, StepScalars *, int);                     \
+                                     const F *, const F *, double, StepScalars *, int);      \
     template void launch_pressure_first<F>(                                                  \
         hipStream_t, const GridParams &, const F *, const F *, const F *, const F *, F *,   \
         F *, F *, const int64_t *, const int64_t *, int64_t *, Window, const F *, const F *, \
