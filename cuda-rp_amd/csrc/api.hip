@@ -1046,6 +1046,9 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
         const auto rp_call = [&](int loop, double p_inf) -> int {
             const bool replay = h->sched_mode == 2;
             rp_waves = 0;
+            shape = tin || replay ? kRPLight
+                                  : bubble_step_grid(h->last_sub_max, h->last_sub_per_launch,
+                                                     h->bp.extreme_threshold, h->cus);
             if (!tin && !replay && !bubble_step_unordered(*h->rpl_h, h->cus)) {
                 // the pressure gather, then the queue: the first iteration's
                 // from the start state (the previous step's counts do not
@@ -1055,7 +1058,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 launch_queue_keys<F>(s, h->g, h->bp, h->b, p0, h->rp_cur, h->pl_p, loop,
                                      h->bp.extreme_threshold, h->sc_d, p_inf);
                 launch_order_partition(s, h->b, h->b.key, h->bp.heavy_threshold,
-                                       h->bp.extreme_threshold, h->sc_d, p_inf);
+                                       h->bp.extreme_threshold, shape != kRPLight, h->sc_d, p_inf);
             }
             if (tin) {  // replay: the void fraction from the taped radii, no RP
                 launch_scatter_radii(s, h->g, h->bp, bnow, tin->Rt_it[loop], h->fgb[target], h->sc_d);
@@ -1067,8 +1070,6 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 launch_rp_replay<F>(s, h->rpl_d, h->nb, h->rp_cur, h->pl_m, h->pl_n, h->pl_p,
                                     p0, h->fgb[target], h->sc_d, cl.off, cl.dts);
             } else {
-                shape = bubble_step_grid(h->last_sub_max, h->last_sub_per_launch,
-                                         h->bp.extreme_threshold, h->cus);
                 rp_waves = launch_bubble_step<F>(s, *h->rpl_h, h->rpl_d, h->rp_cur, h->pl_m, h->pl_n,
                                                  h->pl_p, p0, h->fgb[target], h->sc_d, loop, shape,
                                                  h->cus, h->per_cu, p_inf);

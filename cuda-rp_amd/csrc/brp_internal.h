@@ -384,7 +384,7 @@ void launch_queue_keys(hipStream_t s, const GridParams &g, const BubbleParams &b
                        const BubbleArrays &b, const F *p0, int cur, int plp, int slot, int ext,
                        StepScalars *sc, double p_inf);
 void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key, int threshold,
-                            int ext, const StepScalars *sc, double p_inf);
+                            int ext, bool sort, const StepScalars *sc, double p_inf);
 void launch_scatter_initial(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                             const BubbleArrays &b, int64_t *fg_target, StepScalars *sc);
 void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg);
