@@ -1047,8 +1047,8 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
             const bool replay = h->sched_mode == 2;
             rp_waves = 0;
             shape = tin || replay ? kRPLight
-                                  : bubble_step_grid(h->last_sub_max, h->last_sub_per_launch,
-                                                     h->bp.extreme_threshold, h->cus);
+                                  : bubble_step_grid(h->last_sub_max, h->last_sub_per_launch, h->cus);
+            const int ext = bubble_step_extreme(h->last_sub_max, h->bp.extreme_threshold);
             if (!tin && !replay && !bubble_step_unordered(*h->rpl_h, h->cus)) {
                 // the pressure gather, then the queue: the first iteration's
                 // from the start state (the previous step's counts do not
@@ -1056,9 +1056,9 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 // previous iteration's counts, bubbles whose gathered
                 // pressure did not change last
                 launch_queue_keys<F>(s, h->g, h->bp, h->b, p0, h->rp_cur, h->pl_p, loop,
-                                     h->bp.extreme_threshold, h->sc_d, p_inf);
+                                     ext, h->sc_d, p_inf);
                 launch_order_partition(s, h->b, h->b.key, h->bp.heavy_threshold,
-                                       h->bp.extreme_threshold, shape != kRPLight, h->sc_d, p_inf);
+                                       ext, shape != kRPLight, h->sc_d, p_inf);
             }
             if (tin) {  // replay: the void fraction from the taped radii, no RP
                 launch_scatter_radii(s, h->g, h->bp, bnow, tin->Rt_it[loop], h->fgb[target], h->sc_d);

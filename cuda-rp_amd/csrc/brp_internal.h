@@ -271,7 +271,7 @@ struct BubbleParams {
     int cylindrical;
     int rp_exact;
     int heavy_threshold;    // sub-steps that put a bubble at the queue front
-    int extreme_threshold;  // sub-steps that give a bubble a wavefront of its own
+    int extreme_threshold;  // sub-steps that give a bubble a wavefront of its own (at most)
     const double *rp_shared;  // device table of rp_table_values (kRpTable doubles)
 };
 
@@ -374,8 +374,9 @@ bool bubble_step_unordered(const RPLaunch &host, int cus);
 void rp_grid_query(int device, int *cus, int *per_cu);
 int bubble_step_blocks(int n_bubbles, bool lean, int cus, int per_cu);
 // The shape of the next RP launch, from the last one's longest chain and its
-// sub-steps in all.
-RPGrid bubble_step_grid(int sub_max, double sub_per_launch, int extreme_threshold, int cus);
+// sub-steps in all, and the sub-steps from which its bubbles are extreme.
+RPGrid bubble_step_grid(int sub_max, double sub_per_launch, int cus);
+int bubble_step_extreme(int sub_max, int extreme_threshold);
 // Pressure gather of a Picard iteration's bubbles into PL[plp] and its queue
 // keys (predicted or previous sub-step counts; -1: the previous iteration's
 // results stand).
