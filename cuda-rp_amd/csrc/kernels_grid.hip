@@ -557,7 +557,7 @@ __global__ __launch_bounds__(256) void k_pressure_first_small(
             const F np0 = npx + npy;
             px[o] = npx;
             py[o] = npy;
-            rmax = fabs((double)p0[o] - (double)np0);
+            rmax = fmax(0.0, fabs((double)p0[o] - (double)np0));  // passes over NaN
             bad = !isfinite((double)np0) || fabs(fg_to_d(fpred)) >= 1.0;
             p0[o] = np0;
         }
