@@ -1447,6 +1447,7 @@ __global__ __launch_bounds__(256) void k_queue_keys(GridParams g, BubbleParams b
                 k = max(k, bp.heavy_threshold);
             }
         }
+        k = max(k, 0);  // (a negative radius gives negative estimates)
     } else {
         k = PL == b.PL[plp][idx] ? -1 : b.sub[idx];
     }
