@@ -302,6 +302,26 @@ int set_err(brp_handle *h, int code, const char *fmt, ...) {
                            __FILE__, __LINE__);                                          \
     } while (0)
 
+// Makes a handle's device the calling thread's current one, and the one that
+// was current again at the end: read-backs and snapshots launch kernels, make
+// events and take memory, which belong to the device current then.
+struct DeviceScope {
+    int prev = -1;
+    hipError_t err;
+    explicit DeviceScope(int device) {
+        err = hipGetDevice(&prev);
+        if (err != hipSuccess || prev == device)
+            prev = -1;
+        else
+            err = hipSetDevice(device);
+    }
+    ~DeviceScope() {
+        if (prev >= 0) (void)hipSetDevice(prev);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 enum class Keep { kScratch, kState, kVoid };  // whether a snapshot holds the array
 int dalloc(brp_handle *h, void **p, size_t bytes, Keep keep = Keep::kScratch) {
     *p = nullptr;
@@ -1953,6 +1973,8 @@ int brp_get_field(brp_handle *h, int32_t field, double *dst, int64_t ld) {
     int nx, ny, i0, j0;
     field_extent(h, field, &nx, &ny, &i0, &j0);
     if (ld < nx) return set_err(h, BRP_ERR_INVALID, "ld %lld < %d", (long long)ld, nx);
+    const DeviceScope scope(h->device);
+    HIPCHK(h, scope.err);
     int rc = brp_prepare(h);
     if (rc) return rc;
     PackSrc p{h->prec == BRP_PREC_FP64 ? PackSrc::kDouble : PackSrc::kFloat, nx, nullptr, nullptr,
@@ -2044,6 +2066,8 @@ int brp_set_field(brp_handle *h, int32_t field, const double *src, int64_t ld) {
 
 int brp_get_bubbles(brp_handle *h, int32_t which, double *dst) {
     if (!h || !dst || which < 0 || which >= BRP_BUB_COUNT) return BRP_ERR_INVALID;
+    const DeviceScope scope(h->device);
+    HIPCHK(h, scope.err);
     int rc = brp_prepare(h);
     if (rc) return rc;
     const int n = h->nb;
@@ -2273,6 +2297,8 @@ int brp_get_bubbles_noalloc(brp_handle *h, int32_t which, double *dst) {
 
 int brp_save_state(brp_handle *h, int32_t slot) {
     if (!h || slot < 0 || slot >= 16) return BRP_ERR_INVALID;
+    const DeviceScope scope(h->device);
+    HIPCHK(h, scope.err);
     int rc = brp_prepare(h);
     if (rc) return rc;
     if ((rc = snap_save(h, h->snaps[slot]))) return rc;
@@ -2284,6 +2310,8 @@ int brp_restore_state(brp_handle *h, int32_t slot) {
     if (!h || slot < 0 || slot >= 16) return BRP_ERR_INVALID;
     Snapshot &sn = h->snaps[slot];
     if (!sn.valid) return set_err(h, BRP_ERR_STATE, "slot %d holds no state", slot);
+    const DeviceScope scope(h->device);
+    HIPCHK(h, scope.err);
     const int rc = snap_restore(h, sn);
     if (rc) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));

@@ -432,7 +432,7 @@ struct HostRing {
     void release();
 };
 // rows x src.nx values into dst (leading dimension ld); returns when they are
-// there.
+// there.  `device`, the stream's, is current.
 hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &src, int64_t rows,
                      double *dst, int64_t ld);
 

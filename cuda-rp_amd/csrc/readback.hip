@@ -116,10 +116,6 @@ hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &s
     std::atomic<int64_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     auto work = [&](int slot) {
-        if (hipError_t d = hipSetDevice(device)) {  // the current device is per thread
-            failed = (int)d;
-            return;
-        }
         double *buf = ring.host + slot * kSlotDoubles;
         for (int64_t c; failed == (int)hipSuccess && (c = next++) < pieces;) {
             const int64_t e0 = c * kSlotDoubles;
@@ -137,8 +133,14 @@ hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &s
     // two pieces or more to a thread; a thread that cannot be had is done without
     const int helpers = (int)std::min<int64_t>(kSlots, pieces / 2) - 1;
     std::vector<std::thread> pool;
+    const auto helper = [&](int slot) {
+        if (hipError_t d = hipSetDevice(device))  // the current device is per thread
+            failed = (int)d;
+        else
+            work(slot);
+    };
     try {
-        for (int w = 1; w <= helpers; w++) pool.emplace_back(work, w);
+        for (int w = 1; w <= helpers; w++) pool.emplace_back(helper, w);
     } catch (const std::system_error &) {
     } catch (const std::bad_alloc &) {
     }
