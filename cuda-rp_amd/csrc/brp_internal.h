@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "../../include/bubbles_rp.h"
 #include "rp_vfit.h"
 
@@ -421,15 +423,17 @@ struct PackSrc {
     double scale;                   // kDensity: the liquid's density
 };
 // Pinned memory of a handle's read-backs: `small` (the handle's, small_doubles
-// long) for arrays that it holds, else a ring of slots.
+// long) for arrays that it holds, else a ring of slots.  One read-back at a
+// time has them: a handle may be read by several threads.
 struct HostRing {
     static constexpr int64_t kMaxSmall = 1 << 17;
+    std::mutex mu;
     double *small = nullptr;
     int64_t small_doubles = 0;
     double *host = nullptr;
     hipEvent_t ev[8] = {};
     hipError_t reserve();
-    void release();
+    void release();  // the ring's slots and events
 };
 // rows x src.nx values into dst (leading dimension ld); returns when they are
 // there.  `device`, the stream's, is current.

@@ -56,10 +56,12 @@ constexpr int64_t kSlotDoubles = HostRing::kMaxSmall;
 constexpr int kSlots = 8;
 
 void HostRing::release() {
-    for (hipEvent_t &e : ev)
+    for (hipEvent_t &e : ev) {
         if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
     if (host) (void)hipHostFree(host);
-    *this = HostRing();
+    host = nullptr;
 }
 
 hipError_t HostRing::reserve() {
@@ -69,14 +71,7 @@ hipError_t HostRing::reserve() {
     if (e != hipSuccess) host = nullptr;
     for (int k = 0; k < kSlots && e == hipSuccess; k++)
         e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-    if (e != hipSuccess) {
-        for (hipEvent_t &v : ev) {
-            if (v) (void)hipEventDestroy(v);
-            v = nullptr;
-        }
-        if (host) (void)hipHostFree(host);
-        host = nullptr;
-    }
+    if (e != hipSuccess) release();
     return e;
 }
 
@@ -105,6 +100,7 @@ hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &s
                      double *dst, int64_t ld) {
     const int64_t nx = src.nx, total = nx * rows;
     if (total <= 0) return hipSuccess;
+    const std::lock_guard<std::mutex> lock(ring.mu);
     if (total <= ring.small_doubles) {
         hipError_t e = launch_pack(s, src, 0, (int)total, ring.small);
         if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -1,20 +1,26 @@
 // A HIP runtime of two devices in host memory, for tests of the library's host
 // code on a machine without a GPU: linked into this program, its functions
-// take the place of the runtime's.  Launches compute nothing.  Streams, events and memory belong to the device that is
+// take the place of the runtime's.  Launches compute nothing, but for k_pack
+// of FP64 fields.  Streams, events and memory belong to the device that is
 // current when they are made; a launch or a record on another device's stream
 // is counted, as is memory taken on another device than the test names.
 //
 //   fake_hip devices   one handle per device, read back, saved and restored
 //                      while the other device is current
+//   fake_hip threads   two threads read two fields of one handle
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <string>
+#include <thread>
 #include <vector>
 
+#include "brp_internal.h"
 #include "bubbles_rp.h"
 
 namespace {
@@ -22,6 +28,7 @@ thread_local int current = 0;
 std::atomic<int> foreign{0};    // launches and records on another device's stream
 std::atomic<int> expected{-1};  // device on which memory has to be taken, -1: any
 std::atomic<int> misplaced{0};
+std::atomic<bool> slow{false};  // waits take a while
 struct Handle {
     int device;
 };
@@ -32,7 +39,16 @@ struct Config {
 };
 thread_local Config config;
 
+// kernel names (the library registers its kernels before main's statics are made)
+std::map<const void *, std::string> &names() {
+    static std::map<const void *, std::string> m;
+    return m;
+}
+
 int device_of(const void *h) { return h ? ((const Handle *)h)->device : current; }
+void pause_a_little() {
+    if (slow) std::this_thread::sleep_for(std::chrono::microseconds(200));
+}
 }  // namespace
 
 extern "C" {
@@ -41,8 +57,10 @@ void **__hipRegisterFatBinary(const void *) {
     return &p;
 }
 void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *,
-                           void *, void *, int *) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *,
+                           void *, void *, void *, int *) {
+    names()[host] = name;
+}
 void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t shared, hipStream_t s) {
     config = Config{g, b, shared, s};
@@ -55,8 +73,20 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream
     *s = config.s;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s) {
     if (device_of(s) != current) foreign++;
+    if (names().at(f).find("k_pack") != std::string::npos) {
+        const auto &src = *(const brp::PackSrc *)args[0];
+        const int64_t e0 = *(const int64_t *)args[1];
+        const int n = *(const int *)args[2];
+        double *out = *(double **)args[3];
+        if (src.kind == brp::PackSrc::kDouble)
+            for (int k = 0; k < n; k++) {
+                const int64_t j = (e0 + k) / src.nx, i = (e0 + k) - j * src.nx;
+                out[k] = ((const double *)src.src)[brp::frame_off((int)i + src.i0, (int)j + src.j0,
+                                                                 src.pitch)];
+            }
+    }
     return hipSuccess;
 }
 hipError_t hipGetDeviceCount(int *n) {
@@ -128,6 +158,7 @@ hipError_t hipStreamDestroy(hipStream_t s) {
 }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) {
+    pause_a_little();
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
@@ -143,6 +174,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t) {
+    pause_a_little();
     return hipSuccess;
 }
 hipError_t hipGetLastError() { return hipSuccess; }
@@ -216,12 +248,54 @@ void devices() {
         for (brp_handle *q : h) brp_destroy(q);
     }
 }
+
+void threads() {
+    for (int n : {48, 400, 700}) {
+        brp_handle *h = make(n, false);
+        const size_t m = (size_t)(n + 3) * (n + 3);
+        const int32_t field[2] = {BRP_FIELD_P0, BRP_FIELD_PX};
+        std::vector<double> in[2];
+        for (int k = 0; k < 2; k++) {
+            in[k].resize(m);
+            for (size_t q = 0; q < m; q++) in[k][q] = (k ? -1.0 : 1.0) * (double)(q + 1);
+            if (brp_set_field(h, field[k], in[k].data(), n + 3) != BRP_OK) std::exit(2);
+        }
+        slow = true;
+        std::atomic<int> wrong{0};
+        const auto reader = [&](int k) {
+            int nx, ny, i0, j0;
+            brp_field_shape(h, field[k], &nx, &ny, &i0, &j0);
+            std::vector<double> out(m);
+            for (int r = 0; r < 20; r++) {
+                if (brp_get_field(h, field[k], out.data(), n + 3) != BRP_OK) wrong++;
+                for (int j = 0; j < ny; j++)
+                    for (int i = 0; i < nx; i++)
+                        if (out[(size_t)j * (n + 3) + i] != in[k][(size_t)j * (n + 3) + i]) {
+                            wrong++;
+                            j = ny;
+                            break;
+                        }
+            }
+        };
+        std::thread other(reader, 1);
+        reader(0);
+        other.join();
+        slow = false;
+        if (wrong) {
+            std::printf("%d^2: %d of 40 reads returned other values\n", n, wrong.load());
+            bad = 1;
+        }
+        brp_destroy(h);
+    }
+}
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "devices")
         devices();
+    else if (what == "threads")
+        threads();
     else
         return 2;
     return bad;

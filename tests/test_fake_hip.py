@@ -28,8 +28,9 @@ def fake(tmp_path_factory):
     return exe
 
 
-# devices: read-back, snapshots and restores with the other device current
-@pytest.mark.parametrize("what", ["devices"])
+# devices: read-back, snapshots and restores with the other device current; threads: two
+# threads read one handle
+@pytest.mark.parametrize("what", ["devices", "threads"])
 def test_host_code(fake, what):
     r = subprocess.run([fake, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
