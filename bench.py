@@ -122,7 +122,7 @@ def rp_roofline(sm, nb, traffic):
     one launch per Picard iteration, after k_queue_keys gathered the
     pressures): algorithmic FP64 operations of the sub-steps it integrated
     (results kept from the previous iteration count none) per launch over its
-    mean launch time by the device clock: from its start to the next kernel's."""
+    mean launch time by the device clock."""
     flops = (RP_FLOPS_PER_SUBSTEP * sm["substeps"] + BUBBLE_FLOPS_PER_CALL * nb * sm["launches"]) \
         / max(sm["launches"], 1)
     achieved = flops / (sm["rp_launch_ms"] * 1e-3) / 1e12

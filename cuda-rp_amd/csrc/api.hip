@@ -490,7 +490,9 @@ int alloc_bubbles(brp_handle *h, int n) {
         return rc;
     if ((rc = dalloc(h, (void **)&h->b.totals, sizeof(RPTotals) * 4 * (size_t)(h->cus * h->per_cu))))
         return rc;
-    if ((rc = dalloc(h, (void **)&h->b.bbox_blk, sizeof(int) * 4 * (size_t)((n + 255) / 256 + 1))))
+    const size_t nblk = (size_t)((n + 255) / 256 + 1);
+    if ((rc = dalloc(h, (void **)&h->b.bbox_blk, sizeof(int) * 4 * nblk)) ||
+        (rc = dalloc(h, (void **)&h->b.end_blk, sizeof(unsigned int) * nblk)))
         return rc;
     return BRP_OK;
 }
@@ -1047,7 +1049,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                                  h->fgb[old_n], h->fgb[old_m], h->W, ax, bx, ay, by, h->xu_d,
                                  h->rxp_d, h->sc_d);
         launch_pressure_ghosts<F>(s, g, p0, h->el_amp_d, h->el_phase_d, h->t, 0, nullptr, 0,
-                                  h->b.bbox_blk, bub && !blind ? (h->nb + 255) / 256 : 0, h->sc_d,
+                                  h->b.bbox_blk, h->b.end_blk, bub && !blind ? (h->nb + 255) / 256 : 0, h->sc_d,
                                   blind         ? nullptr
                                   : ahead_steps ? h->rep_ahead + step % kStepsAhead
                                                 : h->rep,
@@ -1152,7 +1154,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                     int rc = schedule_record_call(h);
                     if (rc) return rc;
                 }
-                if (h->cfg.tr_cylindrical) launch_cyl_fold(s, h->g, h->fgb[target]);
+                if (h->cfg.tr_cylindrical) launch_cyl_fold(s, h->g, h->fgb[target], h->sc_d);
                 if (rec && rec->want_bub) {
                     CopyPlan plan;
                     plan.add(rec->PLp_it[loop], h->b.PL[h->pl_p], sizeof(double) * h->nb);
@@ -1167,7 +1169,7 @@ int run_steps(brp_handle *h, int k, brp_step_stats *stats, StepCtl *ctl = nullpt
                 // blind: only where an iteration changes a ghost cell
                 if (!blind || !pressure_ghosts_fixed(h->g))
                     launch_pressure_ghosts<F>(s, h->g, p0, h->el_amp_d, h->el_phase_d, h->t, loop,
-                                              h->b.totals, rp_waves, nullptr, 0, h->sc_d,
+                                              h->b.totals, rp_waves, nullptr, nullptr, 0, h->sc_d,
                                               blind ? nullptr : h->rep, blind ? 0 : ++h->rep_seq,
                                               (unsigned)h->nb * (unsigned)loop);
                 // The step probably ends here, as the one before did: the next
@@ -1928,7 +1930,7 @@ int brp_prepare(brp_handle *h) {
         launch_zero_scalars(h->stream, h->sc_d, 1);
         if (h->cfg.tr_cylindrical && h->W.i0 <= 1 && h->W.i0 <= h->W.i1) h->W.i0 = 0;
         launch_scatter_initial(h->stream, h->g, h->bp, h->b, h->fgb[0], h->sc_d);
-        if (h->cfg.tr_cylindrical) launch_cyl_fold(h->stream, h->g, h->fgb[0]);
+        if (h->cfg.tr_cylindrical) launch_cyl_fold(h->stream, h->g, h->fgb[0], nullptr);
         HIPCHK(h, hipMemcpyAsync(h->fgb[1], h->fgb[0], sizeof(int64_t) * h->frame, hipMemcpyDeviceToDevice, h->stream));
         HIPCHK(h, hipMemcpyAsync(h->fgb[2], h->fgb[0], sizeof(int64_t) * h->frame, hipMemcpyDeviceToDevice, h->stream));
         int flags = 0;
@@ -2172,7 +2174,7 @@ int brp_scatter_variant(brp_handle *h, int32_t mode, double *dst, int64_t ld) {
         launch_scatter_radii(s, h->g, h->bp, h->b, h->b.R_t, spare, h->sc_d);
     else
         launch_scatter_variant(s, h->g, h->bp, h->b, mode, spare, (int64_t)h->frame);
-    if (h->cfg.tr_cylindrical && mode == BRP_VF_INT64) launch_cyl_fold(s, h->g, spare);
+    if (h->cfg.tr_cylindrical && mode == BRP_VF_INT64) launch_cyl_fold(s, h->g, spare, nullptr);
     HIPCHK(h, hipGetLastError());
     std::vector<double> fr(h->frame);
     if (mode == BRP_VF_INT64) {

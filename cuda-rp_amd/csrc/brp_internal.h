@@ -73,6 +73,7 @@ struct RPTotals {
     unsigned long long sub_sum;  // sub-steps integrated
     unsigned int done, kept;     // bubbles written back; of them, kept
     int sub_max, flags;          // StepScalars::flags bits
+    unsigned long long end;      // the device's clock when it was done
 };
 
 // The RP launch's work queue has kQueueHeads heads, each on a line of its own:
@@ -81,8 +82,11 @@ constexpr int kQueueHeads = 16, kHeadStride = 32;
 
 // Where the phases of a step begin: the velocity update, the bubble motion,
 // the first pressure evaluation; in a Picard iteration the queue, the RP
-// launch and the pressure evaluation; the temperature solve.
-enum Mark { kMarkVelocity, kMarkMotion, kMarkPressure, kMarkQueue, kMarkRP, kMarkPicard,
+// launch, the fold at the axis and the pressure evaluation; the temperature
+// solve.  A phase ends where the next begins, but for the motion and the RP
+// launch: the kernel after them may be queued only once the host has read a
+// report, so their own workgroups and wavefronts say when they end.
+enum Mark { kMarkVelocity, kMarkMotion, kMarkPressure, kMarkQueue, kMarkRP, kMarkFold, kMarkPicard,
             kMarkThermal, kMarks };
 
 // What the host reads after an evaluation: k_pressure_ghosts, the
@@ -258,6 +262,7 @@ struct BubbleArrays {
     int *sort_hist;       // partition scratch: 2048 bin counts / offsets of that sort
     int *part;            // partition scratch: per-block extreme and heavy offsets + totals
     int *bbox_blk;        // per-block stencil bounding boxes of k_motion (4 ints each)
+    unsigned int *end_blk;  // per block of k_motion: the device's clock at its end (low word)
     RPTotals *totals;     // per wavefront of the RP launch
     unsigned int *heads;  // kQueueHeads work-queue heads, kHeadStride apart, twice
                           // (the second for the extreme entries on lane pairs)
@@ -343,8 +348,9 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
                             const double *el_phase, double t, int eval, const RPTotals *tot,
-                            int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
-                            StepReport *rep, unsigned long long seq, unsigned int done_want);
+                            int n_tot, const int *bbox_blk, const unsigned int *end_blk,
+                            int n_bbox, StepScalars *sc, StepReport *rep, unsigned long long seq,
+                            unsigned int done_want);
 // Whether a Picard iteration's evaluation changes no ghost cell of p0: they
 // hold the source row, or nothing, and mirror no wall.
 inline bool pressure_ghosts_fixed(const GridParams &g) {
@@ -390,7 +396,8 @@ void launch_order_partition(hipStream_t s, const BubbleArrays &b, const int *key
                             int ext, bool sort, const StepScalars *sc, double p_inf);
 void launch_scatter_initial(hipStream_t s, const GridParams &g, const BubbleParams &bp,
                             const BubbleArrays &b, int64_t *fg_target, StepScalars *sc);
-void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg);
+// (sc may be null)
+void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg, StepScalars *sc);
 // Frozen schedule: record the accepted RP step sizes of the last RP launch
 // (same inputs, same sub-step function) and replay them in a later run.
 void launch_rp_record(hipStream_t s, const RPLaunch *dev, int n, int cur, int plm, int pln,

@@ -53,10 +53,11 @@ __device__ inline int64_t to_fixed(double v, bool *bad) {
 }
 
 // Block-wide reduction of (min, max) pairs into this block's slot of out
-// (4 ints); k_pressure_ghosts folds the slots into sc->bbox.  One plain store per
-// block instead of device-scope atomics on four shared addresses, which
+// (4 ints), and when it was done; k_pressure_ghosts folds the slots into sc->bbox.  One plain
+// store per block instead of device-scope atomics on four shared addresses, which
 // serialise across the whole grid.
-__device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *out) {
+__device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *out,
+                                  unsigned int *end) {
     for (int off = 32; off > 0; off >>= 1) {
         imin = min(imin, __shfl_xor(imin, off, 64));
         imax = max(imax, __shfl_xor(imax, off, 64));
@@ -84,6 +85,7 @@ __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *o
         out[4 * blockIdx.x + 1] = imax;
         out[4 * blockIdx.x + 2] = jmin;
         out[4 * blockIdx.x + 3] = jmax;
+        end[blockIdx.x] = (unsigned int)wall_clock64();
     }
 }
 
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(256) void k_motion(GridParams g, BubbleParams bp, B
         }
     }
     if (stop) return;
-    block_bbox(imin, imax, jmin, jmax, b.bbox_blk);
+    block_bbox(imin, imax, jmin, jmax, b.bbox_blk, b.end_blk);
 }
 
 // A bubble's volume per cell area, the quantity the scatter spreads
@@ -317,7 +319,7 @@ __device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
     const int flags = (__ballot(bad) ? 2 : 0) | (__ballot(capped) ? 4 : 0);
     if (lane == 0)
         tot[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)] =
-            RPTotals{sub_sum, done, kept, sub_max, flags};
+            RPTotals{sub_sum, done, kept, sub_max, flags, (unsigned long long)wall_clock64()};
 }
 
 // The next batch of `size` entries of a wavefront from the queue of n (whole
@@ -1089,7 +1091,8 @@ __global__ __launch_bounds__(256) void k_scatter_variant(GridParams g, BubblePar
 
 // VoidFractionCylinderKernel (bubble_CUDA_kernel.cuh:559-573) for order 2:
 // the axis fold f_g(0, j) += f_g(1, j); f_g(1, j) = f_g(0, j), exact in int64.
-__global__ void k_cyl_fold(GridParams g, int64_t *fg) {
+__global__ void k_cyl_fold(GridParams g, int64_t *fg, StepScalars *sc) {
+    if (sc) set_mark(sc, kMarkFold);
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j > g.M + 1) return;
     const int64_t o0 = frame_off(0, j, g.pitch), o1 = frame_off(1, j, g.pitch);
@@ -1537,8 +1540,8 @@ template void launch_rp_replay<float>(hipStream_t, const RPLaunch *, int, int, i
                                       const float *, int64_t *, StepScalars *, const int64_t *,
                                       const double *);
 
-void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg) {
-    hipLaunchKernelGGL(k_cyl_fold, dim3((g.M + 2 + 255) / 256), dim3(256), 0, s, g, fg);
+void launch_cyl_fold(hipStream_t s, const GridParams &g, int64_t *fg, StepScalars *sc) {
+    hipLaunchKernelGGL(k_cyl_fold, dim3((g.M + 2 + 255) / 256), dim3(256), 0, s, g, fg, sc);
 }
 
 void launch_copy_d(hipStream_t s, double *dst, const double *src, int n) {

@@ -170,7 +170,6 @@ __device__ inline void clear_scalars(StepScalars *sc) {
     sc->done = 0u;
     sc->reused = 0u;
     for (int k = 0; k < 5; k++) sc->phase[k] = 0ull;
-    sc->mark[kMarkMotion] = 0ull;
 }
 
 // Focused source value of row-0 cell i at time t (MixtureBoundaryPressureKernel
@@ -636,6 +635,7 @@ __device__ inline void totals_add(RPTotals &a, const RPTotals &b) {
     a.kept += b.kept;
     a.sub_max = max(a.sub_max, b.sub_max);
     a.flags |= b.flags;
+    a.end = max(a.end, b.end);
 }
 
 // MixtureBoundaryPressureKernel (bubble_CUDA_kernel.cuh:870-952) for order 2,
@@ -654,7 +654,8 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           const double *el_amp,
                                                           const double *el_phase, double t,
                                                           int eval, const RPTotals *tot, int n_tot,
-                                                          const int *bbox_blk, int n_bbox,
+                                                          const int *bbox_blk,
+                                                          const unsigned int *end_blk, int n_bbox,
                                                           StepScalars *sc, StepReport *rep,
                                                           unsigned long long seq,
                                                           unsigned int done_want) {
@@ -662,14 +663,16 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
     const unsigned long long began = wall_clock64();
+    unsigned long long rp_end = 0ull;  // thread 0's
+    unsigned int motion = 0u;          // how long k_motion took (thread 0's)
     if (n_tot > 0) {  // workgroup-uniform
         __shared__ RPTotals red[16];
-        RPTotals a{0ull, 0u, 0u, 0, 0};
+        RPTotals a{0ull, 0u, 0u, 0, 0, 0ull};
         for (int k = tid; k < n_tot; k += nt) totals_add(a, tot[k]);
         for (int off = 32; off > 0; off >>= 1)
             totals_add(a, RPTotals{__shfl_xor(a.sub_sum, off, 64), __shfl_xor(a.done, off, 64),
                                    __shfl_xor(a.kept, off, 64), __shfl_xor(a.sub_max, off, 64),
-                                   __shfl_xor(a.flags, off, 64)});
+                                   __shfl_xor(a.flags, off, 64), __shfl_xor(a.end, off, 64)});
         if ((tid & 63) == 0) red[tid >> 6] = a;
         __syncthreads();
         if (tid == 0) {
@@ -679,10 +682,13 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             sc->reused += a.kept;
             sc->sub_max = max(sc->sub_max, a.sub_max);
             sc->flags |= a.flags;
+            rp_end = a.end;
         }
     }
     if (n_bbox > 0) {  // workgroup-uniform
         __shared__ int box[16][4];
+        __shared__ unsigned int took[16];
+        const unsigned int start = (unsigned int)sc->mark[kMarkMotion];
         int v[4] = {0x7fffffff, -0x7fffffff, 0x7fffffff, -0x7fffffff};
         for (int k = tid; k < n_bbox; k += nt) {
             const int4 q = ((const int4 *)bbox_blk)[k];
@@ -690,19 +696,26 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             v[1] = max(v[1], q.y);
             v[2] = min(v[2], q.z);
             v[3] = max(v[3], q.w);
+            motion = max(motion, end_blk[k] - start);
         }
-        for (int off = 32; off > 0; off >>= 1)
+        for (int off = 32; off > 0; off >>= 1) {
             for (int c = 0; c < 4; c++) {
                 const int u = __shfl_xor(v[c], off, 64);
                 v[c] = (c & 1) ? max(v[c], u) : min(v[c], u);
             }
-        if ((tid & 63) == 0)
+            motion = max(motion, (unsigned int)__shfl_xor((int)motion, off, 64));
+        }
+        if ((tid & 63) == 0) {
             for (int c = 0; c < 4; c++) box[tid >> 6][c] = v[c];
+            took[tid >> 6] = motion;
+        }
         __syncthreads();
         if (tid == 0) {
-            for (int w = 1; w < nt / 64; w++)
+            for (int w = 1; w < nt / 64; w++) {
                 for (int c = 0; c < 4; c++)
                     v[c] = (c & 1) ? max(v[c], box[w][c]) : min(v[c], box[w][c]);
+                motion = max(motion, took[w]);
+            }
             if (v[0] <= v[1])
                 for (int c = 0; c < 4; c++) sc->bbox[c] = v[c];
         }
@@ -747,14 +760,14 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
         for (int k = 0; k < 5; k++) ph[k] = sc->phase[k];
         const unsigned long long now = wall_clock64();
         if (eval == 0) {
-            const unsigned long long motion = m[kMarkMotion] ? m[kMarkMotion] : m[kMarkPressure];
-            ph[0] += motion - m[kMarkVelocity];
-            ph[1] += m[kMarkPressure] - motion;
+            ph[0] += m[n_bbox > 0 ? kMarkMotion : kMarkPressure] - m[kMarkVelocity];
+            ph[1] += motion;
             ph[2] += now - m[kMarkPressure];
         } else {  // an empty window has no evaluation kernel
             const unsigned long long p = m[kMarkPicard] > m[kMarkRP] ? m[kMarkPicard] : began;
             ph[4] += m[kMarkQueue] ? m[kMarkRP] - m[kMarkQueue] : 0ull;
-            ph[3] += p - m[kMarkRP];
+            ph[3] += (n_tot > 0 ? rp_end : p) - m[kMarkRP];
+            if (n_tot > 0 && m[kMarkFold] > m[kMarkRP]) ph[3] += p - m[kMarkFold];
             ph[2] += now - p;
         }
         out.resid = __longlong_as_double((long long)sc->resid[eval]);
@@ -853,10 +866,12 @@ void launch_pressure_picard(hipStream_t s, const GridParams &g, const F *vx, con
 template <typename F>
 void launch_pressure_ghosts(hipStream_t s, const GridParams &g, F *p0, const double *el_amp,
                             const double *el_phase, double t, int eval, const RPTotals *tot,
-                            int n_tot, const int *bbox_blk, int n_bbox, StepScalars *sc,
-                            StepReport *rep, unsigned long long seq, unsigned int done_want) {
+                            int n_tot, const int *bbox_blk, const unsigned int *end_blk,
+                            int n_bbox, StepScalars *sc, StepReport *rep, unsigned long long seq,
+                            unsigned int done_want) {
     hipLaunchKernelGGL(k_pressure_ghosts<F>, dim3(1), dim3(1024), 0, s, g, p0, el_amp,
-                       el_phase, t, eval, tot, n_tot, bbox_blk, n_bbox, sc, rep, seq, done_want);
+                       el_phase, t, eval, tot, n_tot, bbox_blk, end_blk, n_bbox, sc, rep, seq,
+                       done_want);
 }
 
 void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
@@ -877,7 +892,8 @@ void launch_zero_scalars(hipStream_t s, StepScalars *sc, int nslots) {
         const F *, const F *, const double *, const double *, StepScalars *, int);           \
     template void launch_pressure_ghosts<F>(hipStream_t, const GridParams &, F *,           \
                                             const double *, const double *, double, int,     \
-                                            const RPTotals *, int, const int *, int,         \
+                                            const RPTotals *, int, const int *,              \
+                                            const unsigned int *, int,                       \
                                             StepScalars *, StepReport *, unsigned long long,  \
                                             unsigned int);
 

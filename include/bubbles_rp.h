@@ -326,7 +326,11 @@ int brp_restore_state(brp_handle *h, int32_t slot);
 int brp_set_focus(brp_handle *h, double fp_x, double fp_y, double f_dist);
 
 /* Device time of the last brp_step call split by phase (ms): [0] velocity,
- * [1] bubble motion, [2] pressure, [3] gather+RP+scatter, [4] other (ordering of the bubble work queue). */
+ * [1] bubble motion, [2] pressure, [3] RP+scatter, with the pressure gather of
+ * populations that need no work queue, [4] other (the gather and ordering of
+ * the bubble work queue, the temperature).  By the device's clock, from a
+ * phase's first kernel to its last one's end; where the next phase's kernels
+ * are queued with it, to their start.  Waits for the host are in no phase. */
 int brp_get_phase_times(const brp_handle *h, double ms[5]);
 
 /* Objective of brp_adjoint: J = mean of p0^2 over the cells
