@@ -456,8 +456,10 @@ __global__ __launch_bounds__(256) void k_adj_bubble(GridParams g, BubbleParams b
 // Adjoint of k_motion: x' = x + dt vLx(x, y; vx), y' = y + dt vLy(x, y; vy)
 // at the step's start positions (xs, ys); Lx, Ly hold dJ/dx', dJ/dy' and
 // become dJ/dx, dJ/dy.  The node adjoints Lvx, Lvy are summed through the
-// workgroup's LDS tiles, both in one pass.  Also carries the liquid-pressure
-// history's adjoints across the step boundary:
+// workgroup's LDS tiles: both in one pass where their joint patch fits, else
+// one after the other, each with the whole LDS (crowded cells far apart, 1024
+// bubbles in 16 cells: 18.1 us with global atomics, 12.9 so; 4096: 9.2 and 8.7).
+// Also carries the liquid-pressure history's adjoints across the step boundary:
 //   Picard ran:  LA <- lPLn + LB,  LB <- lPLm, and the RP adjoints of the step's
 //                end, LR, were consumed: zeros, for the step before to
 //                accumulate in (they become its start's after a swap)
@@ -468,7 +470,10 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
                                                      Rect<F> vx, Rect<F> vy, double *Lvx,
                                                      double *Lvy, double *Lx, double *Ly,
                                                      AdjHistory H) {
-    __shared__ StencilTiles<2, 2048> tiles;  // vx and vy nodes
+    __shared__ union {
+        StencilTiles<2, 2048> both;  // vx and vy nodes
+        StencilTiles<1, 4096> one;   // of either
+    } tiles;
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = idx < n;
     double x = 0.0, y = 0.0, lx = 0.0, ly = 0.0;
@@ -501,10 +506,11 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
     const bool any_y = valid && ly != 0.0 && yi0 <= yi1 && yj0 <= yj1;
     const int big = 0x7fffffff;
     const TileBox t =
-        tiles_begin(tiles, any_x || any_y, min(any_x ? xi0 : big, any_y ? yi0 : big),
+        tiles_begin(tiles.both, any_x || any_y, min(any_x ? xi0 : big, any_y ? yi0 : big),
                     max(any_x ? xi1 : -big, any_y ? yi1 : -big),
                     min(any_x ? xj0 : big, any_y ? yj0 : big),
                     max(any_x ? xj1 : -big, any_y ? yj1 : -big));
+    const bool apart = t.w > 0 && !t.binned;  // workgroup-uniform
     if (valid) {
 #pragma unroll
         for (int a = 0; a < NB; a++) {
@@ -513,14 +519,16 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
                 if (a >= nb || c >= nb) continue;
                 const int i = ibmx + bp.nbs + a, j = ibny + bp.mbs + c;
                 if (i >= xi0 && i <= xi1 && j >= xj0 && j <= xj1) {
-                    if (any_x) tiles_add(tiles, 0, t, Lvx, g.pitch, i, j, dt * lx * Xm.w[a] * Yn.w[c]);
+                    if (any_x && !apart)
+                        tiles_add(tiles.both, 0, t, Lvx, g.pitch, i, j, dt * lx * Xm.w[a] * Yn.w[c]);
                     const double v = (double)vx.at(i, j);
                     dvx_dx += v * Xm.d[a] * Yn.w[c];
                     dvx_dy += v * Xm.w[a] * Yn.d[c];
                 }
                 const int k = ibnx + bp.mbs + a, l = ibmy + bp.nbs + c;
                 if (k >= yi0 && k <= yi1 && l >= yj0 && l <= yj1) {
-                    if (any_y) tiles_add(tiles, 1, t, Lvy, g.pitch, k, l, dt * ly * Xn.w[a] * Ym.w[c]);
+                    if (any_y && !apart)
+                        tiles_add(tiles.both, 1, t, Lvy, g.pitch, k, l, dt * ly * Xn.w[a] * Ym.w[c]);
                     const double v = (double)vy.at(k, l);
                     dvy_dx += v * Xn.d[a] * Ym.w[c];
                     dvy_dy += v * Xn.w[a] * Ym.d[c];
@@ -528,8 +536,28 @@ __global__ __launch_bounds__(256) void k_adj_motion(GridParams g, BubbleParams b
             }
         }
     }
-    double *const glob[2] = {Lvx, Lvy};
-    tiles_flush(tiles, t, glob, g.pitch);
+    if (!apart) {
+        double *const glob[2] = {Lvx, Lvy};
+        tiles_flush(tiles.both, t, glob, g.pitch);
+    } else {
+        const auto nodes = [&](bool any, int first_i, int first_j, int i0, int i1, int j0, int j1,
+                               const double *wi, const double *wj, double s, double *L) {
+            const TileBox b = tiles_begin(tiles.one, any, i0, i1, j0, j1);
+            if (any)
+#pragma unroll
+                for (int a = 0; a < NB; a++)
+#pragma unroll
+                    for (int c = 0; c < NB; c++) {
+                        const int i = first_i + a, j = first_j + c;
+                        if (a < nb && c < nb && i >= i0 && i <= i1 && j >= j0 && j <= j1)
+                            tiles_add(tiles.one, 0, b, L, g.pitch, i, j, s * wi[a] * wj[c]);
+                    }
+            double *const glob[1] = {L};
+            tiles_flush(tiles.one, b, glob, g.pitch);
+        };
+        nodes(any_x, ibmx + bp.nbs, ibny + bp.mbs, xi0, xi1, xj0, xj1, Xm.w, Yn.w, dt * lx, Lvx);
+        nodes(any_y, ibnx + bp.mbs, ibmy + bp.nbs, yi0, yi1, yj0, yj1, Xn.w, Ym.w, dt * ly, Lvy);
+    }
     if (valid) {
         Lx[idx] = lx + dt * (lx * dvx_dx + ly * dvy_dx);
         Ly[idx] = ly + dt * (lx * dvx_dy + ly * dvy_dy);
