@@ -635,15 +635,17 @@ size_t snap_plan(const brp_handle *h, const Window &w, char *block, bool save, C
     return at;
 }
 
-int snap_save(brp_handle *h, Snapshot &sn) {
-    const size_t need = snap_plan(h, h->W, nullptr, true, nullptr);
+// room: the largest window that the snapshot's block is to hold, as every save
+// into it gives it (the handle's own for a snapshot saved once; the whole frame
+// for a slot, which is saved again without taking memory).
+int snap_save(brp_handle *h, Snapshot &sn, const Window &room) {
+    const size_t need = snap_plan(h, room, nullptr, true, nullptr);
     if (sn.arrays && sn.arrays != h->state.size())
         return set_err(h, BRP_ERR_STATE, "snapshot layout changed");
-    if (need > sn.capacity) {
+    if (!sn.block) {
         char *q = nullptr;
         if (hipMalloc((void **)&q, need) != hipSuccess)
             return set_err(h, BRP_ERR_DEVICE, "snapshot allocation failed (%zu bytes)", need);
-        if (sn.block) (void)hipFree(sn.block);
         sn.block = q;
         sn.capacity = need;
     }
@@ -1452,7 +1454,7 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
     wins.reserve(n);
     fctl.win_out = &wins;
     for (int sg = 0; sg < nseg; sg++) {
-        if ((rc = snap_save(h, ck[sg]))) return rc;
+        if ((rc = snap_save(h, ck[sg], h->W))) return rc;
         const int s_end = std::min(n, (sg + 1) * K);
         for (int st = sg * K + 1; st <= s_end; st++) {
             fctl.rec = use_tape ? &tape[st - 1] : nullptr;
@@ -1460,7 +1462,7 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
             if (st > n - ob.window) launch_box_sumsq<F>(s, h->g, (const F *)h->p0, box, jacc + st - 1);
         }
     }
-    if ((rc = snap_save(h, fin))) return rc;
+    if ((rc = snap_save(h, fin, h->W))) return rc;
     std::vector<double> jh(n);
     HIPCHK(h, hipMemcpy(jh.data(), jacc, sizeof(double) * n, hipMemcpyDeviceToHost));
     double J = 0.0;
@@ -2303,7 +2305,7 @@ int brp_save_state(brp_handle *h, int32_t slot) {
     HIPCHK(h, scope.err);
     int rc = brp_prepare(h);
     if (rc) return rc;
-    if ((rc = snap_save(h, h->snaps[slot]))) return rc;
+    if ((rc = snap_save(h, h->snaps[slot], Window{0, h->N + 1, 0, h->M + 1}))) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return BRP_OK;
 }

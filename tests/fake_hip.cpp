@@ -8,6 +8,7 @@
 //   fake_hip devices   one handle per device, read back, saved and restored
 //                      while the other device is current
 //   fake_hip threads   two threads read two fields of one handle
+//   fake_hip slots     a slot saved again after the window has grown
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -28,6 +29,7 @@ thread_local int current = 0;
 std::atomic<int> foreign{0};    // launches and records on another device's stream
 std::atomic<int> expected{-1};  // device on which memory has to be taken, -1: any
 std::atomic<int> misplaced{0};
+std::atomic<int> taken{0};      // allocations of device memory
 std::atomic<bool> slow{false};  // waits take a while
 struct Handle {
     int device;
@@ -112,6 +114,7 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
 }
 hipError_t hipMalloc(void **p, size_t n) {
     if (expected >= 0 && current != expected) misplaced++;
+    taken++;
     *p = std::calloc(n, 1);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -288,6 +291,20 @@ void threads() {
         brp_destroy(h);
     }
 }
+
+void slots() {
+    const int n = 200;
+    brp_handle *h = make(n, true);
+    if (brp_save_state(h, 0) != BRP_OK) std::exit(2);
+    std::vector<double> fg((size_t)(n + 2) * (n + 2), 1e-6);
+    if (brp_set_field(h, BRP_FIELD_FGN, fg.data(), n + 2) != BRP_OK) std::exit(2);
+    taken = 0;
+    if (brp_save_state(h, 0) != BRP_OK || taken) {
+        std::printf("a slot saved again took memory %d times\n", taken.load());
+        bad = 1;
+    }
+    brp_destroy(h);
+}
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -296,6 +313,8 @@ int main(int argc, char **argv) {
         devices();
     else if (what == "threads")
         threads();
+    else if (what == "slots")
+        slots();
     else
         return 2;
     return bad;
