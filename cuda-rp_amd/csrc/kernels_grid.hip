@@ -816,7 +816,7 @@ template <typename F>
 void launch_velocity(hipStream_t s, const GridParams &g, F *vx, F *vy, const F *p0,
                      const int64_t *fgn, Window w, int first_step, const F *cxa, const F *cxb,
                      const F *cya, const F *cyb, double t, StepScalars *sc, int nslots) {
-    if (velocity_small(g) && std::min(g.N, g.M) >= 4) {  // (one thread for each wall)
+    if (velocity_small(g)) {  // (brp_create refuses sides below 4: one thread for each wall)
         hipLaunchKernelGGL(k_velocity_small<F>, dim3((g.N + kBX) / kBX, (g.M + kBY) / kBY),
                            dim3(kBX, kBY), 0, s, g, vx, vy, p0, fgn, w, first_step, cxa, cxb, cya,
                            cyb, t, sc, nslots);
