@@ -1205,7 +1205,14 @@ int launch_bubble_step(hipStream_t s, const RPLaunch &host, const RPLaunch *dev,
     }
     const bool lean = shape == kRPLean;
     const dim3 grid(bubble_step_blocks(host.b.n, lean, cus, per_cu));
-    const int quota = std::max(8, std::min(64, (host.b.n + 4 * (int)grid.x - 1) / (4 * (int)grid.x)));
+    // A wavefront's share of a population too small to fill them all; but with
+    // the operation-by-operation sub-step, whose wavefronts at different places
+    // of its longer code keep a chain waiting for instructions (20 steps of a
+    // collapse, 30 bubbles 88 ms in full wavefronts, 97 spread over four; 100
+    // bubbles 154 and 162, 300 and more the same).
+    const int waves = 4 * (int)grid.x;
+    const int quota =
+        host.bp.rp_exact ? 64 : std::max(8, std::min(64, (host.b.n + waves - 1) / waves));
     // Dedicated wavefronts: up to one per workgroup on the lean grid, where
     // the longest chains bound the launch.  On the full grid, bound by the
     // work, every one costs a SIMD of throughput: 2^22 clustered bubbles with
