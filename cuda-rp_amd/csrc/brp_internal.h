@@ -73,7 +73,7 @@ struct RPTotals {
     unsigned long long sub_sum;  // sub-steps integrated
     unsigned int done, kept;     // bubbles written back; of them, kept
     int sub_max, flags;          // StepScalars::flags bits
-    unsigned long long end;      // the device's clock when it was done
+    unsigned int end;            // the device's clock when it was done (low word)
 };
 
 // The RP launch's work queue has kQueueHeads heads, each on a line of its own:

@@ -58,6 +58,7 @@ __device__ inline int64_t to_fixed(double v, bool *bad) {
 // serialise across the whole grid.
 __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *out,
                                   unsigned int *end) {
+    const unsigned int now = (unsigned int)wall_clock64();  // (its latency passes meanwhile)
     for (int off = 32; off > 0; off >>= 1) {
         imin = min(imin, __shfl_xor(imin, off, 64));
         imax = max(imax, __shfl_xor(imax, off, 64));
@@ -85,7 +86,7 @@ __device__ inline void block_bbox(int imin, int imax, int jmin, int jmax, int *o
         out[4 * blockIdx.x + 1] = imax;
         out[4 * blockIdx.x + 2] = jmin;
         out[4 * blockIdx.x + 3] = jmax;
-        end[blockIdx.x] = (unsigned int)wall_clock64();
+        end[blockIdx.x] = now;
     }
 }
 
@@ -310,6 +311,7 @@ __device__ inline unsigned long long lanemask_lt(int lane) {
 __device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
                                         unsigned long long sub_sum, unsigned int done,
                                         unsigned int kept, bool bad, bool capped) {
+    const unsigned int now = (unsigned int)wall_clock64();  // (its latency passes meanwhile)
     for (int off = 32; off > 0; off >>= 1) {
         sub_max = max(sub_max, __shfl_xor(sub_max, off, 64));
         sub_sum += __shfl_xor(sub_sum, off, 64);
@@ -319,7 +321,7 @@ __device__ inline void rp_launch_totals(RPTotals *tot, int lane, int sub_max,
     const int flags = (__ballot(bad) ? 2 : 0) | (__ballot(capped) ? 4 : 0);
     if (lane == 0)
         tot[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)] =
-            RPTotals{sub_sum, done, kept, sub_max, flags, (unsigned long long)wall_clock64()};
+            RPTotals{sub_sum, done, kept, sub_max, flags, now};
 }
 
 // The next batch of `size` entries of a wavefront from the queue of n (whole

@@ -635,7 +635,25 @@ __device__ inline void totals_add(RPTotals &a, const RPTotals &b) {
     a.kept += b.kept;
     a.sub_max = max(a.sub_max, b.sub_max);
     a.flags |= b.flags;
-    a.end = max(a.end, b.end);
+}
+
+// The largest of a wavefront's values, by lane moves within the vector unit:
+// shifts by 1 to 8 lanes within the rows of 16, then rows onto the next ones;
+// lane 63 has it.  (By shuffles through LDS the launches' lengths, which
+// k_pressure_ghosts takes twice a step, cost 1 us of 74 at 256^2 with 1024
+// bubbles at rest.)
+template <int MOVE, int ROWS>
+__device__ inline unsigned int max_from(unsigned int v) {
+    return max(v, (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, MOVE, ROWS, 0xf, false));
+}
+__device__ inline unsigned int wave_max(unsigned int v) {
+    v = max_from<0x111, 0xf>(v);  // row_shr:1
+    v = max_from<0x112, 0xf>(v);
+    v = max_from<0x114, 0xf>(v);
+    v = max_from<0x118, 0xf>(v);
+    v = max_from<0x142, 0xa>(v);  // row_bcast:15
+    v = max_from<0x143, 0xc>(v);  // row_bcast:31
+    return (unsigned int)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // MixtureBoundaryPressureKernel (bubble_CUDA_kernel.cuh:870-952) for order 2,
@@ -663,31 +681,42 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
     const int N = g.N, M = g.M, P = g.pitch;
     const int tid = threadIdx.x, nt = blockDim.x;
     const unsigned long long began = wall_clock64();
-    unsigned long long rp_end = 0ull;  // thread 0's
-    unsigned int motion = 0u;          // how long k_motion took (thread 0's)
+    unsigned int took = 0u;  // thread 0: how long the RP launch, or k_motion, took
+    __shared__ unsigned int took_w[16];
     if (n_tot > 0) {  // workgroup-uniform
         __shared__ RPTotals red[16];
-        RPTotals a{0ull, 0u, 0u, 0, 0, 0ull};
-        for (int k = tid; k < n_tot; k += nt) totals_add(a, tot[k]);
+        const unsigned int start = (unsigned int)sc->mark[kMarkRP];
+        RPTotals a{0ull, 0u, 0u, 0, 0, 0u};
+        for (int k = tid; k < n_tot; k += nt) {
+            const RPTotals q = tot[k];
+            totals_add(a, q);
+            took = max(took, q.end - start);
+        }
+        took = wave_max(took);
+        a.sub_max = (int)wave_max((unsigned int)a.sub_max);
         for (int off = 32; off > 0; off >>= 1)
             totals_add(a, RPTotals{__shfl_xor(a.sub_sum, off, 64), __shfl_xor(a.done, off, 64),
-                                   __shfl_xor(a.kept, off, 64), __shfl_xor(a.sub_max, off, 64),
-                                   __shfl_xor(a.flags, off, 64), __shfl_xor(a.end, off, 64)});
-        if ((tid & 63) == 0) red[tid >> 6] = a;
+                                   __shfl_xor(a.kept, off, 64), 0, __shfl_xor(a.flags, off, 64),
+                                   0u});
+        if ((tid & 63) == 0) {
+            red[tid >> 6] = a;
+            took_w[tid >> 6] = took;
+        }
         __syncthreads();
         if (tid == 0) {
-            for (int w = 1; w < nt / 64; w++) totals_add(a, red[w]);
+            for (int w = 1; w < nt / 64; w++) {
+                totals_add(a, red[w]);
+                took = max(took, took_w[w]);
+            }
             sc->sub_sum += a.sub_sum;
             sc->done += a.done;
             sc->reused += a.kept;
             sc->sub_max = max(sc->sub_max, a.sub_max);
             sc->flags |= a.flags;
-            rp_end = a.end;
         }
     }
     if (n_bbox > 0) {  // workgroup-uniform
         __shared__ int box[16][4];
-        __shared__ unsigned int took[16];
         const unsigned int start = (unsigned int)sc->mark[kMarkMotion];
         int v[4] = {0x7fffffff, -0x7fffffff, 0x7fffffff, -0x7fffffff};
         for (int k = tid; k < n_bbox; k += nt) {
@@ -696,25 +725,24 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
             v[1] = max(v[1], q.y);
             v[2] = min(v[2], q.z);
             v[3] = max(v[3], q.w);
-            motion = max(motion, end_blk[k] - start);
+            took = max(took, end_blk[k] - start);
         }
-        for (int off = 32; off > 0; off >>= 1) {
+        took = wave_max(took);
+        for (int off = 32; off > 0; off >>= 1)
             for (int c = 0; c < 4; c++) {
                 const int u = __shfl_xor(v[c], off, 64);
                 v[c] = (c & 1) ? max(v[c], u) : min(v[c], u);
             }
-            motion = max(motion, (unsigned int)__shfl_xor((int)motion, off, 64));
-        }
         if ((tid & 63) == 0) {
             for (int c = 0; c < 4; c++) box[tid >> 6][c] = v[c];
-            took[tid >> 6] = motion;
+            took_w[tid >> 6] = took;
         }
         __syncthreads();
         if (tid == 0) {
             for (int w = 1; w < nt / 64; w++) {
                 for (int c = 0; c < 4; c++)
                     v[c] = (c & 1) ? max(v[c], box[w][c]) : min(v[c], box[w][c]);
-                motion = max(motion, took[w]);
+                took = max(took, took_w[w]);
             }
             if (v[0] <= v[1])
                 for (int c = 0; c < 4; c++) sc->bbox[c] = v[c];
@@ -761,12 +789,12 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
         const unsigned long long now = wall_clock64();
         if (eval == 0) {
             ph[0] += m[n_bbox > 0 ? kMarkMotion : kMarkPressure] - m[kMarkVelocity];
-            ph[1] += motion;
+            ph[1] += took;
             ph[2] += now - m[kMarkPressure];
         } else {  // an empty window has no evaluation kernel
             const unsigned long long p = m[kMarkPicard] > m[kMarkRP] ? m[kMarkPicard] : began;
             ph[4] += m[kMarkQueue] ? m[kMarkRP] - m[kMarkQueue] : 0ull;
-            ph[3] += (n_tot > 0 ? rp_end : p) - m[kMarkRP];
+            ph[3] += n_tot > 0 ? took : p - m[kMarkRP];
             if (n_tot > 0 && m[kMarkFold] > m[kMarkRP]) ph[3] += p - m[kMarkFold];
             ph[2] += now - p;
         }
