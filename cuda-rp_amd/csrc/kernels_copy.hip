@@ -48,14 +48,20 @@ __global__ __launch_bounds__(256) void k_copy_many(CopyPlan c) {
     }
 }
 
-// Row blockIdx.y of rectangle blockIdx.z, from its frame to its dense buffer.
+// Rows blockIdx.y, blockIdx.y + gridDim.y, ... of rectangle blockIdx.z, from its
+// frame to its dense buffer.  (A launch may have 65 536 workgroups in y, the
+// tallest frame has 65 539 rows.)
+constexpr int kRectRows = 1 << 15;
+
 __global__ __launch_bounds__(256) void k_copy_rects(RectPlan r, Window w, int pitch) {
-    const int z = blockIdx.z, row = blockIdx.y;
+    const int z = blockIdx.z;
     const int words = (w.i1 - w.i0 + 1) * (r.elem[z] / 4);
-    const unsigned *src = (const unsigned *)((const char *)r.src[z] +
-                                             frame_off(w.i0, w.j0 + row, pitch) * r.elem[z]);
-    unsigned *dst = (unsigned *)r.dst[z] + (size_t)row * words;
-    for (int k = blockIdx.x * 256 + threadIdx.x; k < words; k += gridDim.x * 256) dst[k] = src[k];
+    for (int row = blockIdx.y; row <= w.j1 - w.j0; row += gridDim.y) {
+        const unsigned *src = (const unsigned *)((const char *)r.src[z] +
+                                                 frame_off(w.i0, w.j0 + row, pitch) * r.elem[z]);
+        unsigned *dst = (unsigned *)r.dst[z] + (size_t)row * words;
+        for (int k = blockIdx.x * 256 + threadIdx.x; k < words; k += gridDim.x * 256) dst[k] = src[k];
+    }
 }
 
 }  // namespace
@@ -77,8 +83,9 @@ void launch_copy_many(hipStream_t s, const CopyPlan &c) {
 void launch_copy_rects(hipStream_t s, const RectPlan &r, const Window &w, int pitch) {
     if (r.n <= 0 || w.i0 > w.i1 || w.j0 > w.j1) return;
     const int cols = w.i1 - w.i0 + 1;
-    hipLaunchKernelGGL(k_copy_rects, dim3(std::min(8, (2 * cols + 255) / 256), w.j1 - w.j0 + 1, r.n),
-                       dim3(256), 0, s, r, w, pitch);
+    const int rows = std::min(kRectRows, w.j1 - w.j0 + 1);
+    hipLaunchKernelGGL(k_copy_rects, dim3(std::min(8, (2 * cols + 255) / 256), rows, r.n), dim3(256),
+                       0, s, r, w, pitch);
 }
 
 }  // namespace brp

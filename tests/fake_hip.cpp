@@ -9,6 +9,7 @@
 //                      while the other device is current
 //   fake_hip threads   two threads read two fields of one handle
 //   fake_hip slots     a slot saved again after the window has grown
+//   fake_hip rows      a rectangle of more rows than a launch has workgroups in y
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -30,6 +31,7 @@ std::atomic<int> foreign{0};    // launches and records on another device's stre
 std::atomic<int> expected{-1};  // device on which memory has to be taken, -1: any
 std::atomic<int> misplaced{0};
 std::atomic<int> taken{0};      // allocations of device memory
+std::atomic<int> too_tall{0};   // launches of more than 65535 workgroups in y or z
 std::atomic<bool> slow{false};  // waits take a while
 struct Handle {
     int device;
@@ -75,7 +77,8 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream
     *s = config.s;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **args, size_t, hipStream_t s) {
+    if (g.y > 65535 || g.z > 65535) too_tall++;
     if (device_of(s) != current) foreign++;
     if (names().at(f).find("k_pack") != std::string::npos) {
         const auto &src = *(const brp::PackSrc *)args[0];
@@ -305,6 +308,18 @@ void slots() {
     }
     brp_destroy(h);
 }
+
+void rows() {
+    // the tallest grid's frame (65 536 cells and its ghosts)
+    brp::RectPlan r;
+    int64_t a[1], b[1];
+    r.add(a, b, sizeof(int64_t));
+    brp::launch_copy_rects(nullptr, r, brp::Window{-1, 9, -1, 65537}, 128);
+    if (too_tall) {
+        std::printf("%d launches of more than 65535 workgroups in y\n", too_tall.load());
+        bad = 1;
+    }
+}
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -315,6 +330,8 @@ int main(int argc, char **argv) {
         threads();
     else if (what == "slots")
         slots();
+    else if (what == "rows")
+        rows();
     else
         return 2;
     return bad;

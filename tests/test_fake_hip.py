@@ -29,8 +29,9 @@ def fake(tmp_path_factory):
 
 
 # devices: read-back, snapshots and restores with the other device current; threads: two
-# threads read one handle; slots: a snapshot slot saved again takes no memory
-@pytest.mark.parametrize("what", ["devices", "threads", "slots"])
+# threads read one handle; slots: a snapshot slot saved again takes no memory; rows: no launch
+# is larger in y than the runtime allows
+@pytest.mark.parametrize("what", ["devices", "threads", "slots", "rows"])
 def test_host_code(fake, what):
     r = subprocess.run([fake, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
