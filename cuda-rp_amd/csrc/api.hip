@@ -1,11 +1,15 @@
 // api.hip -- C ABI of libbubbles_rp (include/bubbles_rp.h): set-up, the
-// step scheduler and data movement.  Host code; kernels live in
-// kernels_grid.hip and kernels_bubble.hip.
+// step scheduler and data movement.  Host code; kernels live in kernels_*.hip.
 //
-// The step is driven from the host: each pressure evaluation ends with one
-// small device-to-host read of the residual (and, after the first
-// evaluation, the bubble bounding box), which decides the Picard sub-loop
-// exactly as the reference's host loop does (bubble_CUDA.cu:240-276).
+// The step is driven from the host.  The last kernel of each pressure
+// evaluation writes a report into pinned memory (residual, flags, counts and,
+// after the first evaluation, the bubbles' bounding box), and the host decides
+// the Picard sub-loop by it exactly as the reference's host loop does
+// (bubble_CUDA.cu:240-276).  Where the next launches are likely enough they are
+// queued before the report is there, and the device tests the same conditions:
+// a step's first RP call does nothing if the step has no iteration
+// (picard_needed), the next step's first launches if the step goes on or has
+// failed (halted), and steps of acoustics alone run up to kStepsAhead ahead.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

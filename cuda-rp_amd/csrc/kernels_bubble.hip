@@ -413,8 +413,10 @@ __device__ inline crpl *rpl(const RPLaunch *p) {
 // before the others are taken a lane each; and once the queue is empty a wavefront with at most 32 bubbles left
 // moves them onto lane pairs.  A pair does a sub-step in 0.7 of a lane's time,
 // and a chain of the 257th rank is nearly as long as the first: RP launch of
-// 2^20 bubbles 2142 -> 1476 us, 2^22 (with the full grid) 2523 -> 1907,
-// 30 011 1640 -> 1460, 65 536 1207 -> 1110.  At most 256 VGPRs, so that two wavefronts fit a SIMD; held to that by the attribute for
+// 2^20 bubbles 2142 -> 1476 us, 30 011 1640 -> 1460, 65 536 1207 -> 1110; 2^22
+// in clouds (with the full grid; the average of 20 steps) 3.00 -> 2.50 ms, 2.10
+// since the queue keys tell a step's first launch its long chains.  At most 256
+// VGPRs, so that two wavefronts fit a SIMD; held to that by the attribute for
 // two the compiler spills nine, and a launch without long chains took 12 %
 // more.
 //
@@ -1133,10 +1135,13 @@ void launch_motion(hipStream_t s, const GridParams &g, const BubbleParams &bp,
 // Workgroups of the persistent RP kernel: as many as fit (two per CU) when
 // the launch is bound by the work of all bubbles; one per CU ("lean") when a
 // few long sub-step chains bound it, so that each wavefront has a SIMD of its
-// own.  Collapsing bubbles, ms per step on the lean / full grid: 2^20 (2500
-// sub-steps in the longest chain, 0.14 of that in a lane of the lean grid on
-// average) 6.3 / 7.4; 2^22 (2700, 0.49) 13.4 / 11.2.  bubble_step_grid decides
-// from the previous launch.
+// own.  bubble_step_grid decides from the previous launch, by the sub-steps
+// that fall to a lane of the lean grid on average against the longest chain's.
+// Collapsing bubbles at 2048^2, steps on the full grid against the lean one,
+// by that ratio: 0.03 to 0.05 0.98 to 1.01, 0.09 to 0.13 1.01 to 1.04 (2^20 to 1.4e6
+// bubbles), 0.18 to 0.196 1.00 to 1.03 (2^21), 0.24 to 0.26 0.87 (2.8e6; at
+// half the amplitude 0.96), 0.27 0.83 (3e6 in clouds), 0.35 to 0.37 0.73
+// (2^22): the line at 0.2 lies where they cross.
 void rp_grid_query(int device, int *cus, int *per_cu) {
     int c = 0, p = 0;
     (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, device);
@@ -1417,7 +1422,14 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const int *sub, const int 
 //    such, and none missed is longer than half the longest; what is missed
 //    starts late and ends the launch.  By 10 (-dR/dt) (R / R0) sqrt(3 um / R0),
 //    without regard to the time left, 29 900 were found among 80 900: first RP
-//    launch of a step 3.1 -> 2.0 ms, as the later ones.
+//    launch of a step 3.68 -> 2.46 ms, the second 2.29.
+//    The two constants of the energy's logarithm are a fit to that population
+//    (water, 2 MHz, 3 MPa, steps of 33 ns); surface tension, viscosity and the
+//    length of the step do not enter.  The key orders the queue and no more,
+//    so a poor estimate costs time.  Elsewhere, first launch before and now /
+//    later ones now, ms: 2^20 bubbles, 1 MHz, 1.5 MPa 1.81, 1.54 / 1.54, with
+//    steps of 17 ns 1.46, 1.30 / 1.29, of 7 ns 1.28, 1.19 / 1.18, 0.75 MPa 1.37,
+//    1.34 / 1.35; 2^18, 3 MPa 2.01, 1.77 / 1.75.
 //  * Later iterations: the previous iteration's sub-step count, or -1 where
 //    the gathered pressure equals the previous iteration's bit for bit.
 //    That iteration integrated the same inputs (start state, pressure
