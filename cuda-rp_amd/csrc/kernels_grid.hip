@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void k_velocity(GridParams g, F *__restrict__ 
     const int i0 = (blockIdx.x * kBX + lane) * kGW;
     const int jb = blockIdx.y * kGBlockRows + threadIdx.y * kGRows;
     if (jb > g.M) return;  // wave-uniform
-    const bool live = i0 <= g.N;
+    const bool live = i0 <= g.N + 1;  // the lane after the last has p0's ghost column for it
     const F dt = (F)g.dt;
     const F rdx = (F)g.rdx;
     const F half = (F)0.5;
