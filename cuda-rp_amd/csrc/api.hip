@@ -1597,7 +1597,8 @@ int adjoint_impl(brp_handle *h, const brp_objective &ob, double *grad_amp, doubl
 
     // gradients
     if (grad_fg0) {
-        const PackSrc p{PackSrc::kSum3, h->N + 2, a.LfC, a.LfN, a.LfM, nullptr, 0, 0, h->pitch, 0.0};
+        const PackSrc p{PackSrc::kSum3, h->N + 2, a.LfC, a.LfN, a.LfM, nullptr, 0, 0, h->pitch, 0.0,
+                        nullptr};
         HIPCHK(h, read_back(s, h->device, h->ring, p, h->M + 2, grad_fg0, ld));
     }
     if ((grad_amp || grad_phase) && h->n_elem > 0) {
@@ -1813,8 +1814,8 @@ int brp_create(const brp_config *cfg, brp_handle **out) {
     // the step reports and, behind them, the small read-back slot
     const size_t rep_bytes = (sizeof(StepReport) * (1 + kStepsAhead) + 255) & ~size_t(255);
     h->ring.small_doubles = std::min<int64_t>(HostRing::kMaxSmall, (int64_t)(h->N + 3) * (h->M + 3));
-    if (hipHostMalloc((void **)&h->rep, rep_bytes + sizeof(double) * h->ring.small_doubles,
-                      hipHostMallocDefault) != hipSuccess ||
+    const size_t small_bytes = std::max(sizeof(double) * h->ring.small_doubles, HostRing::kCopyMax);
+    if (hipHostMalloc((void **)&h->rep, rep_bytes + small_bytes, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&h->rpl_h, sizeof(RPLaunch), hipHostMallocDefault) != hipSuccess)
         return fail(set_err(h, BRP_ERR_DEVICE, "hipHostMalloc failed"));
     std::memset(h->rep, 0, sizeof(StepReport) * (1 + kStepsAhead));
@@ -1986,7 +1987,7 @@ int brp_get_field(brp_handle *h, int32_t field, double *dst, int64_t ld) {
     int rc = brp_prepare(h);
     if (rc) return rc;
     PackSrc p{h->prec == BRP_PREC_FP64 ? PackSrc::kDouble : PackSrc::kFloat, nx, nullptr, nullptr,
-              nullptr, nullptr, i0, j0, h->pitch, h->rho_inf};
+              nullptr, nullptr, i0, j0, h->pitch, h->rho_inf, nullptr};
     double fill = 0.0;  // the value of a field without an array
     switch (field) {
         case BRP_FIELD_P0: p.src = h->p0; break;
@@ -2109,7 +2110,8 @@ int brp_get_bubbles(brp_handle *h, int32_t which, double *dst) {
             src = tmpd;
         }
     }
-    const PackSrc p{kind, n, src, nullptr, nullptr, h->iperm_d, 0, 0, 0, 0.0};
+    const PackSrc p{kind, n, src, nullptr, nullptr, h->iperm_d, 0, 0, 0, 0.0,
+                    tmpd ? nullptr : h->perm.data()};
     const hipError_t e = read_back(h->stream, h->device, h->ring, p, 1, dst, n);
     if (tmpd) (void)hipFree(tmpd);
     if (e != hipSuccess) return set_err(h, BRP_ERR_DEVICE, "get_bubbles: %s", hipGetErrorString(e));

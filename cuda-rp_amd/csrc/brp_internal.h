@@ -428,12 +428,15 @@ struct PackSrc {
     const int *iperm;               // caller index -> sorted bubble
     int i0, j0, pitch;
     double scale;                   // kDensity: the liquid's density
+    const int *perm;                // the inverse of iperm, on the host (null: src is just being made)
 };
-// Pinned memory of a handle's read-backs: `small` (the handle's, small_doubles
-// long) for arrays that it holds, else a ring of slots.  One read-back at a
+// Pinned memory of a handle's read-backs: `small` (the handle's) for arrays of
+// up to small_doubles values and copies of up to kCopyMax bytes, else a ring of
+// slots.  One read-back at a
 // time has them: a handle may be read by several threads.
 struct HostRing {
     static constexpr int64_t kMaxSmall = 1 << 17;
+    static constexpr size_t kCopyMax = 1 << 16;
     std::mutex mu;
     double *small = nullptr;
     int64_t small_doubles = 0;

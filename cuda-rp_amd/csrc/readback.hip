@@ -21,16 +21,14 @@
 namespace brp {
 namespace {
 
-// Element e of the logical array, row-major over nx columns.
-__device__ inline double pack_value(const PackSrc &s, int64_t e) {
-    if (s.kind == PackSrc::kPerm || s.kind == PackSrc::kPermInt) {
-        const int k = s.iperm[e];
-        return s.kind == PackSrc::kPerm ? ((const double *)s.src)[k] : (double)((const int *)s.src)[k];
-    }
-    const int64_t j = e / s.nx, i = e - j * s.nx;
-    const int64_t o = frame_off((int)i + s.i0, (int)j + s.j0, s.pitch);
+bool permuted(const PackSrc &s) { return s.kind == PackSrc::kPerm || s.kind == PackSrc::kPermInt; }
+
+// The value at element o of the source.
+__host__ __device__ inline double source_value(const PackSrc &s, int64_t o) {
     switch (s.kind) {
         case PackSrc::kFloat: return (double)((const float *)s.src)[o];
+        case PackSrc::kPermInt: return (double)((const int *)s.src)[o];
+        case PackSrc::kPerm:
         case PackSrc::kDouble: return ((const double *)s.src)[o];
         case PackSrc::kFixed: return (double)((const int64_t *)s.src)[o] * kFgInvScale;
         case PackSrc::kDensity:
@@ -39,6 +37,13 @@ __device__ inline double pack_value(const PackSrc &s, int64_t e) {
             return ((const double *)s.src)[o] + ((const double *)s.src2)[o] +
                    ((const double *)s.src3)[o];
     }
+}
+
+// Element e of the logical array, row-major over nx columns.
+__device__ inline double pack_value(const PackSrc &s, int64_t e) {
+    if (s.kind == PackSrc::kPerm || s.kind == PackSrc::kPermInt) return source_value(s, s.iperm[e]);
+    const int64_t j = e / s.nx, i = e - j * s.nx;
+    return source_value(s, frame_off((int)i + s.i0, (int)j + s.j0, s.pitch));
 }
 
 __global__ __launch_bounds__(256) void k_pack(PackSrc s, int64_t e0, int n, double *out) {
@@ -54,6 +59,14 @@ __global__ __launch_bounds__(256) void k_pack(PackSrc s, int64_t e0, int n, doub
 // `small`, which is pinned with the handle and serves one thread.
 constexpr int64_t kSlotDoubles = HostRing::kMaxSmall;
 constexpr int kSlots = 8;
+
+// Arrays of more than 16 and up to 64 KiB are copied as they are and converted
+// here: the copy engine, which takes copies beyond 16 KiB, is 4 us faster than a
+// kernel on an idle stream (into pinned memory 7.8 against 11.9 us at 17 KB, 9.6
+// against 12.4 at 64; 2100 radii 13.7 -> 10.5 us, a 30^2 field 13.4 -> 9.7), and
+// up to there the conversion takes less.  Behind a kernel it is slower (bubble
+// indices, 25 against 18 us).
+constexpr size_t kCopyMin = 1 << 14;
 
 void HostRing::release() {
     for (hipEvent_t &e : ev) {
@@ -94,6 +107,27 @@ hipError_t launch_pack(hipStream_t s, const PackSrc &src, int64_t e0, int n, dou
     hipLaunchKernelGGL(k_pack, dim3(std::min(512, (n + 255) / 256)), dim3(256), 0, s, src, e0, n, out);
     return hipGetLastError();
 }
+
+// The bytes from the source's beginning to the end of its last row, or of the
+// bubble array; 0 where the kernel has to do it.
+size_t source_span(const PackSrc &s, int64_t rows) {
+    const size_t elem = s.kind == PackSrc::kFloat || s.kind == PackSrc::kPermInt ? 4 : 8;
+    if (permuted(s)) return s.perm ? elem * s.nx : 0;
+    return s.kind == PackSrc::kSum3 ? 0 : elem * s.pitch * (rows + s.j0 + 1);
+}
+
+// The source's values from a copy of its span.
+void convert_out(PackSrc s, const void *copy, int64_t rows, double *dst, int64_t ld) {
+    s.src = copy;
+    if (permuted(s)) {
+        for (int64_t k = 0; k < s.nx; k++) dst[s.perm[k]] = source_value(s, k);
+        return;
+    }
+    for (int64_t j = 0; j < rows; j++) {
+        const int64_t o = frame_off(s.i0, (int)j + s.j0, s.pitch);
+        for (int64_t i = 0; i < s.nx; i++) dst[j * ld + i] = source_value(s, o + i);
+    }
+}
 }  // namespace
 
 hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &src, int64_t rows,
@@ -101,6 +135,13 @@ hipError_t read_back(hipStream_t s, int device, HostRing &ring, const PackSrc &s
     const int64_t nx = src.nx, total = nx * rows;
     if (total <= 0) return hipSuccess;
     const std::lock_guard<std::mutex> lock(ring.mu);
+    const size_t span = source_span(src, rows);
+    if (span > kCopyMin && span <= HostRing::kCopyMax) {
+        hipError_t e = hipMemcpyAsync(ring.small, src.src, span, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e == hipSuccess) convert_out(src, ring.small, rows, dst, ld);
+        return e;
+    }
     if (total <= ring.small_doubles) {
         hipError_t e = launch_pack(s, src, 0, (int)total, ring.small);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
