@@ -679,7 +679,8 @@ __global__ __launch_bounds__(1024) void k_pressure_ghosts(GridParams g, F *p0,
                                                           unsigned int done_want) {
     if (halted(g, sc)) return;
     const int N = g.N, M = g.M, P = g.pitch;
-    const int tid = threadIdx.x, nt = blockDim.x;
+    const int tid = threadIdx.x;
+    constexpr int nt = 1024;  // blockDim.x, known to the folds over the wavefronts
     const unsigned long long began = wall_clock64();
     unsigned int took = 0u;  // thread 0: how long the RP launch, or k_motion, took
     __shared__ unsigned int took_w[16];
